@@ -162,12 +162,10 @@ static Bases bases_for(dmhm_hmat_s* A, dmhm_hmat_s* B, dmhm_hmat_s* C, void* X, 
 // Tile-engine candidates per execution slot (FP64, FP32, FP32 with BF16
 // operands allowed); FP32 engines stay candidates in the BF16 slot, since a
 // more precise engine that is also faster is the better choice there.
-// (The prefetching MFMA form is not a candidate in FP64: it produced wrong
-// products there on gfx950 while the same source is exact in FP32.)
-static const int kTuneCands[3][5] = {{TILE_LDS, TILE_MFMA, -1, -1, -1},
-                                     {TILE_LDS, TILE_MFMA, TILE_MFMA_PF, -1, -1},
-                                     {TILE_LDS, TILE_MFMA, TILE_MFMA_PF, TILE_MFMA_BF16, TILE_MFMA_BF16_PF}};
-static const int kTuneCount[3] = {2, 3, 5};
+static const int kTuneCands[3][3] = {{TILE_LDS, TILE_MFMA, -1},
+                                     {TILE_LDS, TILE_MFMA, -1},
+                                     {TILE_LDS, TILE_MFMA, TILE_MFMA_BF16}};
+static const int kTuneCount[3] = {2, 2, 3};
 
 // Launches a TILE phase with its engine. Autotuning (no engine forced): the
 // first run of a phase in a slot is a warm-up with the first candidate (its
@@ -2383,7 +2381,7 @@ void Plan::upload()
             // Segment table of a merged tile phase: the members' source
             // arrays must already be on the device.
             std::vector<TileSeg> segs;
-            int b1 = 0, b4 = 0;
+            int b1 = 0, b2 = 0, b4 = 0;
             for (const auto& s : ph.segSrc) {
                 const int n = (int)s.src->tiles.size();
                 if (n > 0 && (!s.src->dTiles || !s.src->dContribs))
@@ -2394,12 +2392,15 @@ void Plan::upload()
                 for (int k = 0; k < NUM_SLOTS; ++k) { t.val[k] = s.val[k]; t.rank[k] = s.rank[k]; }
                 t.count = n;
                 t.first1 = b1;
+                t.first2 = b2;
                 t.first4 = b4;
                 b1 += n;
+                b2 += (n + 1) / 2;
                 b4 += (n + 3) / 4;
                 segs.push_back(t);
             }
             ph.segBlocks1 = b1;
+            ph.segBlocks2 = b2;
             ph.segBlocks4 = b4;
             HIPCHECK(hipMalloc(&ph.dSegs, segs.size() * sizeof(TileSeg)));
             HIPCHECK(copy_sync(ph.dSegs, segs.data(), segs.size() * sizeof(TileSeg), hipMemcpyHostToDevice));

@@ -198,8 +198,13 @@ __device__ __forceinline__ void tile_body(const BV& b, const Tile& tl, const Con
 
 // Segmented launches (merged plans of independent members): the member
 // segment holding workgroup g, found by bisection over the segments' first
-// workgroups (one or four tiles per workgroup), and the member's bases, the
+// workgroups (one, two or four tiles per workgroup), and the member's bases, the
 // launch's bases shifted by the member's offsets.
+template <int TPB>
+__device__ __forceinline__ int seg_first(const TileSeg& s)
+{
+    return TPB == 1 ? s.first1 : TPB == 2 ? s.first2 : s.first4;
+}
 template <int TPB>
 __device__ __forceinline__ int seg_of(const TileSeg* __restrict__ segs, int nseg, int g)
 {
@@ -207,13 +212,13 @@ __device__ __forceinline__ int seg_of(const TileSeg* __restrict__ segs, int nseg
         // One load per lane and a ballot: the segment is the last one whose
         // first workgroup is at or before g.
         const int l = threadIdx.x & 63;
-        const int f = l < nseg ? (TPB == 1 ? segs[l].first1 : segs[l].first4) : INT_MAX;
+        const int f = l < nseg ? seg_first<TPB>(segs[l]) : INT_MAX;
         return (int)__popcll(__ballot(f <= g)) - 1;
     }
     int lo = 0, hi = nseg - 1;
     while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
-        const int f = TPB == 1 ? segs[mid].first1 : segs[mid].first4;
+        const int f = seg_first<TPB>(segs[mid]);
         if (f <= g) lo = mid;
         else hi = mid - 1;
     }
@@ -238,25 +243,44 @@ __global__ void __launch_bounds__(256) tile_seg_kernel(Bases b, const TileSeg* _
 }
 
 // ---------------------------------------------------------------------------
-// MFMA engine: one wave per 16-row block of an output tile. A phase of 64-row
-// tiles runs one workgroup of four waves per tile (wave w owns rows
-// 16w..16w+15), a phase of tiles of at most 16 rows packs four tiles per
-// workgroup; no LDS and no barriers, so every wave streams its contributions
-// independently. A wave computes its block transposed, D^T = R^T L^T, in
-// 16 x 16 MFMA blocks: the first operand is a 16-column block of R^T, the
-// second the wave's 16-row block of L^T, and lane l holds
-// D(row0 + l%16, cb*16 + c(l, r)) in accumulator register r, so each group of
-// 16 lanes stores 16 consecutive rows of a column. The FP32 and BF16
-// instructions place output row 4*(l/16) + r of the 16 x 16 block in register
-// r of lane l, the FP64 one row l/16 + 4*r (measured on gfx950), hence
-// c(l, r) = 4*(l/16) + r for FP32 accumulators and l/16 + 4*r for FP64. The
-// inner dimension advances in chunks of 16; lane l supplies inner indices
-// p0 + 4*(l/16) + e, e < 4, to both operands: four K = 4 steps of
-// v_mfma_f64_16x16x4f64 / v_mfma_f32_16x16x4f32 (MODE 0, arithmetic in T), or
-// one K = 16 step of v_mfma_f32_16x16x16_bf16 on operands rounded from FP32 to
-// BF16 with FP32 accumulation (MODE 1). Out-of-range entries load as zero.
-// PF = 1 issues the loads of the next chunk (possibly of the next
-// contribution) before the MFMAs of the current one.
+// MFMA engine. A wave computes one unit of an output tile, RB x CB blocks of
+// 16 x 16 entries, straight from global memory: no LDS, no barriers. It
+// computes the unit transposed, D^T = R^T L^T: the first MFMA operand is a
+// 16-column block of R^T, the second a 16-row block of L^T, and lane
+// l = (li, lk) = (l % 16, l / 16) holds D(row li, column c) in accumulator
+// register r, c = 4*lk + r for FP32 and BF16, lk + 4*r for FP64 (measured on
+// gfx950), so each group of 16 lanes stores 16 rows of a column.
+//
+// Inner chunks of 16: lane lk supplies the four inner indices mf_k(s, lk),
+// s < 4, to both operands, one per K = 4 instruction (v_mfma_f64_16x16x4f64,
+// v_mfma_f32_16x16x4f32) or all four to one v_mfma_f32_16x16x16_bf16 (MODE 1:
+// FP32 operands rounded to BF16, FP32 accumulation). The map makes 16 bytes
+// along the inner dimension belong to one lane, so an operand stored with the
+// inner dimension contiguous is read with 16-byte loads; an operand stored
+// with rows (columns) contiguous is read two neighbouring rows at a time:
+// row block b of a pair takes the rows of parity b. Rows and columns outside
+// the tile are clamped to its last one (their results are never stored);
+// inner indices outside the contribution are read at its last one and zeroed.
+// Loads of the next chunk (possibly of the next contribution) are issued
+// before the MFMAs of the current one, into the other of two register sets.
+//
+// Contribution records and run-time ranks are read 64 at a time, one per
+// lane, and handed out by lane reads: two memory latencies per 64
+// contributions, not two per contribution.
+//
+// S = 4: the four waves of a workgroup share one unit and split its
+// contributions (every fourth one, or every fourth chunk where a tile has
+// fewer than four contributions) and add their sums through LDS in wave order.
+//
+// What bounds it: operand bytes through L2 and the 256 MB cache, and the FP64
+// MFMA (64 cycles each) where tiles are 64 x 64. Units of 32 x 32 read every
+// operand twice per 64 x 64 tile through L1 and leave room for three waves per
+// SIMD with two chunks of operands in flight each. Measured against the LDS
+// engine (FP64, 256^2, rank 16, one product): projections of 16 x 20 tiles
+// (20 GB of operands) 5.9 -> 3.0 ms, dense accumulation of 64 x 64 tiles 5.7
+// -> 4.1 ms (41 TFLOP/s), all tile phases 82 -> 55 ms; FP32 3D update 19.5
+// -> 12.3 ms. Bounding the registers for four waves per SIMD spills the 32 x 32
+// unit (6.9 -> 7.6 ms in its largest phase).
 // ---------------------------------------------------------------------------
 typedef double mf_d4 __attribute__((ext_vector_type(4)));
 typedef float mf_f4 __attribute__((ext_vector_type(4)));
@@ -282,187 +306,437 @@ __device__ __forceinline__ mf_f4 mf_step_bf16(const float (&a)[4], const float (
     return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(x, y, c, 0, 0, 0);
 }
 
-// Operands of one contribution as the wave reads them.
-template <typename T>
-struct MfSrc {
-    const T* L;
-    const T* R;
-    int64_t ldl, ldr;
-    int q;
-    T a;
-    bool tL, tR;
+// Global-memory pointers (plain global loads, not flat ones) and vectors that
+// need only the element's alignment.
+template <typename T> using GPtr = const __attribute__((address_space(1))) T*;
+template <typename T> struct MfVec;
+template <> struct MfVec<double> {
+    static constexpr int VP = 2;                // elements in 16 bytes
+    typedef double v2 __attribute__((ext_vector_type(2), aligned(8)));
+    typedef v2 vp;
+};
+template <> struct MfVec<float> {
+    static constexpr int VP = 4;
+    typedef float v2 __attribute__((ext_vector_type(2), aligned(4)));
+    typedef float vp __attribute__((ext_vector_type(4), aligned(4)));
 };
 
-template <typename T, typename BV>
-__device__ __forceinline__ MfSrc<T> mf_src(const BV& b, const Contrib& C, int q, T alpha, T beta)
+// Inner index (within a chunk) that lane group lk supplies to step s.
+template <typename T>
+__device__ __forceinline__ int mf_k(int s, int lk)
 {
-    MfSrc<T> s;
-    s.L = b.template val<const T>(C.lslot) + C.loff;
-    s.R = b.template val<const T>(C.rslot) + C.roff;
-    s.ldl = C.ldl; s.ldr = C.ldr; s.q = q;
-    s.a = (C.flags & CF_RUNTIME_ALPHA) ? alpha * T(C.alpha)
-        : (C.flags & CF_RUNTIME_BETA) ? beta * T(C.alpha) : T(C.alpha);
-    s.tL = C.flags & CF_TRANS_L; s.tR = C.flags & CF_TRANS_R;
-    return s;
+    constexpr int VP = MfVec<T>::VP;
+    return (s / VP) * (4 * VP) + lk * VP + s % VP;
 }
 
-// Fragments of chunk p0: lf[e] = L(row, p), rf[cb][e] = a R(p, cb*16 + l%16),
-// p = p0 + 4*(l/16) + e.
-template <typename T, int NBMAX>
-__device__ __forceinline__ void mf_load(const MfSrc<T>& s, int p0, int row, int m, int k, int NB, int li, int lk,
-                                        T (&lf)[4], T (&rf)[NBMAX][4])
+// Row (column) that entry j of block b covers, relative to the unit's first.
+template <int NB>
+__device__ __forceinline__ int mf_row(int b, int j)
 {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const int p = p0 + 4 * lk + e;
-        const bool pin = p < s.q;
-        lf[e] = (pin && row < m) ? (s.tL ? s.L[p + row * s.ldl] : s.L[row + p * s.ldl]) : T(0);
-#pragma unroll
-        for (int cb = 0; cb < NBMAX; ++cb) {
-            const int col = cb * 16 + li;
-            rf[cb][e] = (cb < NB && pin && col < k) ? s.a * (s.tR ? s.R[col + p * s.ldr] : s.R[p + col * s.ldr])
-                                                    : T(0);
-        }
-    }
+    return NB == 1 ? j : 32 * (b >> 1) + 2 * j + (b & 1);
 }
 
-template <typename T, int MODE, int NBMAX, typename Acc>
-__device__ __forceinline__ void mf_mma(const T (&lf)[4], const T (&rf)[NBMAX][4], int NB, Acc (&acc)[NBMAX])
+// Fragments of one operand for one chunk: f[b][s] = X(n, p + mf_k(s, lk)), n
+// the row (column) n0 + mf_row(b, li) clamped below nmax, zero where the inner
+// index reaches q. pc: the inner dimension is contiguous, X(n, p) = X[p + n ld],
+// else X[n + p ld].
+template <typename T, int NB>
+__device__ __forceinline__ void mf_load(GPtr<T> X, int64_t ld, bool pc, int n0, int nmax, int p, int q, int li,
+                                        int lk, T (&f)[NB][4])
 {
+    constexpr int VP = MfVec<T>::VP;
+    typedef typename MfVec<T>::v2 v2;
+    typedef typename MfVec<T>::vp vp;
+    const int qc = q - p;                       // uniform
+    const bool tail = qc < 16;
+    if (pc) {
+        if (!tail) {
 #pragma unroll
-    for (int cb = 0; cb < NBMAX; ++cb) {
-        if (cb >= NB) continue;
-        if constexpr (MODE == 1) {
-            acc[cb] = mf_step_bf16(rf[cb], lf, acc[cb]);
+            for (int b = 0; b < NB; ++b) {
+                const int n = min(n0 + mf_row<NB>(b, li), nmax - 1);
+                GPtr<T> x = X + p + ((int64_t)n * ld + lk * VP);
+#pragma unroll
+                for (int h = 0; h < 4 / VP; ++h) {
+                    const vp v = *(const __attribute__((address_space(1))) vp*)(x + h * 4 * VP);
+#pragma unroll
+                    for (int e = 0; e < VP; ++e) f[b][h * VP + e] = v[e];
+                }
+            }
         } else {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc[cb] = mf_step(rf[cb][e], lf[e], acc[cb]);
+            for (int b = 0; b < NB; ++b) {
+                const int n = min(n0 + mf_row<NB>(b, li), nmax - 1);
+                GPtr<T> x = X + p + (int64_t)n * ld;
+#pragma unroll
+                for (int s = 0; s < 4; ++s) f[b][s] = x[min(mf_k<T>(s, lk), qc - 1)];
+            }
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+                if (mf_k<T>(s, lk) >= qc) {
+#pragma unroll
+                    for (int b = 0; b < NB; ++b) f[b][s] = T(0);
+                }
+        }
+        return;
+    }
+    if (NB > 1 && nmax > 1) {
+        // Pairs of neighbouring rows; a pair that would cross the last row
+        // starts one row earlier and takes its second entry.
+        const bool edge = n0 + 16 * NB > nmax;  // uniform
+#pragma unroll
+        for (int g = 0; g < NB / 2; ++g) {
+            const int want = n0 + 32 * g + 2 * li, at = min(want, nmax - 2);
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                const int k = tail ? min(mf_k<T>(s, lk), qc - 1) : mf_k<T>(s, lk);
+                const v2 v = *(const __attribute__((address_space(1))) v2*)(X + p * ld + (k * ld + at));
+                f[2 * g][s] = v[0];
+                f[2 * g + 1][s] = v[1];
+            }
+            if (edge) {
+#pragma unroll
+                for (int s = 0; s < 4; ++s) f[2 * g][s] = want > at ? f[2 * g + 1][s] : f[2 * g][s];
+            }
+        }
+    } else {
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const int n = min(n0 + mf_row<NB>(b, li), nmax - 1);
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                const int k = tail ? min(mf_k<T>(s, lk), qc - 1) : mf_k<T>(s, lk);
+                f[b][s] = X[p * ld + (k * ld + n)];
+            }
+        }
+    }
+    if (tail) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+            if (mf_k<T>(s, lk) >= qc) {
+#pragma unroll
+                for (int b = 0; b < NB; ++b) f[b][s] = T(0);
+            }
+    }
+}
+
+// The chunks of a tile's contributions as one wave walks them (all members
+// wave-uniform but the per-lane records of the current 64 contributions).
+template <typename T, int S, typename BV>
+struct MfWalk {
+    const BV& b;
+    const Contrib* __restrict__ cs;
+    T alpha, beta;
+    int c0, ce, w, lane;
+    bool byChunk;               // S waves split chunks, not contributions
+    int chunks;                 // chunks before the current contribution (byChunk)
+    uint64_t left;              // contributions of the batch still to visit
+    // lane records
+    int64_t dl, dr;
+    int dldl, dldr, dq;
+    uint32_t dmeta;
+    float dalpha;
+    // current chunk
+    GPtr<T> L, R;
+    int64_t ldl, ldr;
+    int q, p;
+    T a;
+    bool tL, tR;
+
+    __device__ __forceinline__ void batch()
+    {
+        const int c = c0 + lane;
+        const bool in = c < ce;
+        const Contrib& C = cs[in ? c : ce - 1];
+        dl = C.loff; dr = C.roff; dldl = C.ldl; dldr = C.ldr; dalpha = C.alpha;
+        dmeta = (uint32_t)C.lslot | (uint32_t)C.rslot << 8 | (uint32_t)C.flags << 16;
+        dq = contrib_q(b, C);
+        const bool mine = S == 1 || byChunk || (lane & (S - 1)) == w;
+        left = __ballot(in && mine && dq > 0);
+    }
+    __device__ __forceinline__ MfWalk(const BV& b_, const Tile& tl, const Contrib* __restrict__ cs_, int w_, T al,
+                                      T be)
+        : b(b_), cs(cs_), alpha(al), beta(be), c0(tl.cb), ce(tl.ce), w(w_), lane(threadIdx.x & 63),
+          byChunk(S > 1 && tl.ce - tl.cb < S), chunks(0), left(0), q(0), p(0)
+    {
+        if (c0 < ce) batch();
+    }
+    // Moves to the wave's next chunk; false at the end.
+    __device__ __forceinline__ bool next()
+    {
+        p += S > 1 && byChunk ? 16 * S : 16;
+        while (p >= q) {
+            while (left == 0) {
+                c0 += 64;
+                if (c0 >= ce) return false;
+                batch();
+            }
+            const int i = __builtin_ctzll(left);
+            left &= left - 1;
+            if (S > 1 && byChunk) chunks += (q + 15) >> 4;
+            q = __builtin_amdgcn_readlane(dq, i);
+            const uint32_t m = __builtin_amdgcn_readlane(dmeta, i);
+            const int fl = (m >> 16) & 255;
+            const float ca = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(dalpha), i));
+            a = (fl & CF_RUNTIME_ALPHA) ? alpha * T(ca) : (fl & CF_RUNTIME_BETA) ? beta * T(ca) : T(ca);
+            tL = fl & CF_TRANS_L;
+            tR = fl & CF_TRANS_R;
+            ldl = __builtin_amdgcn_readlane(dldl, i);
+            ldr = __builtin_amdgcn_readlane(dldr, i);
+            L = (GPtr<T>)(b.template val<const T>(m & 255) + lane_i64(dl, i));
+            R = (GPtr<T>)(b.template val<const T>((m >> 8) & 255) + lane_i64(dr, i));
+            p = S > 1 && byChunk ? 16 * ((w - chunks) & (S - 1)) : 0;
+        }
+        return true;
+    }
+    static __device__ __forceinline__ int64_t lane_i64(int64_t v, int i)
+    {
+        const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)v, i);
+        const uint32_t hi = __builtin_amdgcn_readlane((int)(v >> 32), i);
+        return (int64_t)((uint64_t)hi << 32 | lo);
+    }
+};
+
+template <typename T, int RB, int CB>
+struct MfFrag {
+    T l[RB][4], r[CB][4];
+    T a;
+    int qc;
+};
+
+template <typename T, int RB, int CB, typename W>
+__device__ __forceinline__ void mf_fetch(const W& k, int row0, int col0, int m, int n, int li, int lk,
+                                         MfFrag<T, RB, CB>& f)
+{
+    mf_load<T, RB>(k.L, k.ldl, k.tL, row0, m, k.p, k.q, li, lk, f.l);
+    mf_load<T, CB>(k.R, k.ldr, !k.tR, col0, n, k.p, k.q, li, lk, f.r);
+    f.a = k.a;
+    f.qc = k.q - k.p;
+}
+
+template <typename T, int MODE, int RB, int CB, typename Acc>
+__device__ __forceinline__ void mf_mma(MfFrag<T, RB, CB>& f, Acc (&acc)[RB][CB])
+{
+    if (f.a != T(1)) {
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) f.l[rb][s] *= f.a;
+    }
+    if constexpr (MODE == 1) {
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb) acc[rb][cb] = mf_step_bf16(f.r[cb], f.l[rb], acc[rb][cb]);
+    } else {
+        // FP64 chunks of at most 8 inner indices fill the first two steps only.
+        constexpr int HALF = sizeof(T) == 8 ? 2 : 4;
+#pragma unroll
+        for (int s = 0; s < HALF; ++s)
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+                for (int cb = 0; cb < CB; ++cb) acc[rb][cb] = mf_step(f.r[cb][s], f.l[rb][s], acc[rb][cb]);
+        if (HALF < 4 && f.qc > 8) {
+#pragma unroll
+            for (int s = HALF; s < 4; ++s)
+#pragma unroll
+                for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+                    for (int cb = 0; cb < CB; ++cb) acc[rb][cb] = mf_step(f.r[cb][s], f.l[rb][s], acc[rb][cb]);
         }
     }
 }
 
-// First contribution at or after c with a non-empty inner dimension.
-template <typename BV>
-__device__ __forceinline__ int mf_next(const BV& b, const Contrib* __restrict__ cs, int c, int ce, int& q)
-{
-    for (; c < ce; ++c) {
-        q = contrib_q(b, cs[c]);
-        if (q > 0) break;
-    }
-    return c;
-}
-
-template <typename T, int MODE, int MBMAX, int NBMAX, int PF, typename BV>
-__device__ __forceinline__ void mfma_body(const BV& b, const Tile& tl, const Contrib* __restrict__ cs, int rb,
-                                          T alpha, T beta)
+// One unit (row group ur, column group uc) of tile tl; w: the wave's share of
+// the contributions (S > 1).
+template <typename T, int MODE, int RB, int CB, int S, typename BV>
+__device__ __forceinline__ void mfma_body(const BV& b, const Tile& tl, const Contrib* __restrict__ cs, int ur,
+                                          int uc, int w, T alpha, T beta)
 {
     static_assert(MODE == 0 || sizeof(T) == 4, "the BF16 mode reads FP32 operands");
-    static_assert(MBMAX == 1 || MBMAX == 4, "tiles of at most 16 or 64 rows");
+    static_assert(S == 1 || S == 4, "one wave or the four waves of a workgroup per unit");
     typedef typename MfAcc<T>::type Acc;
-    int m = tl.m, k = tl.k;
+    int m = tl.m, n = tl.k;
     if (tl.mrank >= 0) m = min(m, max(0, b.rank(tl.mslot)[tl.mrank] - tl.moff));
-    if (tl.krank >= 0) k = min(k, max(0, b.rank(tl.kslot)[tl.krank] - tl.koff));
-    if (m <= rb * 16 || k <= 0) return;
-    const int NB = (k + 15) >> 4;
+    if (tl.krank >= 0) n = min(n, max(0, b.rank(tl.kslot)[tl.krank] - tl.koff));
+    const int row0 = ur * 16 * RB, col0 = uc * 16 * CB;
+    if (m <= row0 || n <= col0) return;         // uniform over the waves that share the unit
     const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
-    const int row = rb * 16 + li;
-    Acc acc[NBMAX];
+    Acc acc[RB][CB];
 #pragma unroll
-    for (int cb = 0; cb < NBMAX; ++cb)
+    for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) acc[cb][r] = T(0);
+        for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[rb][cb][r] = T(0);
 
-    int q = 0;
-    int c = mf_next(b, cs, tl.cb, tl.ce, q);
-    if (c < tl.ce) {
-        MfSrc<T> src = mf_src<T>(b, cs[c], q, alpha, beta);
-        int p0 = 0;
-        T lf[4], rf[NBMAX][4];
-        mf_load<T, NBMAX>(src, p0, row, m, k, NB, li, lk, lf, rf);
+    MfWalk<T, S, BV> k(b, tl, cs, w, alpha, beta);
+    MfFrag<T, RB, CB> f0, f1;
+    if (k.next()) {
+        mf_fetch(k, row0, col0, m, n, li, lk, f0);
         while (true) {
-            // The next chunk: p0 + 16 of this contribution, or the next one.
-            int p1 = p0 + 16, c1 = c, q1 = src.q;
-            if (p1 >= src.q) { p1 = 0; c1 = mf_next(b, cs, c + 1, tl.ce, q1); }
-            const bool more = c1 < tl.ce;
-            MfSrc<T> src1 = src;
-            if (more && c1 != c) src1 = mf_src<T>(b, cs[c1], q1, alpha, beta);
-            if constexpr (PF == 1) {
-                T lf1[4], rf1[NBMAX][4];
-                if (more) mf_load<T, NBMAX>(src1, p1, row, m, k, NB, li, lk, lf1, rf1);
-                mf_mma<T, MODE, NBMAX>(lf, rf, NB, acc);
-                if (!more) break;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    lf[e] = lf1[e];
-#pragma unroll
-                    for (int cb = 0; cb < NBMAX; ++cb) rf[cb][e] = rf1[cb][e];
-                }
-            } else {
-                mf_mma<T, MODE, NBMAX>(lf, rf, NB, acc);
-                if (!more) break;
-                mf_load<T, NBMAX>(src1, p1, row, m, k, NB, li, lk, lf, rf);
-            }
-            c = c1; p0 = p1; src = src1;
+            const bool more1 = k.next();
+            if (more1) mf_fetch(k, row0, col0, m, n, li, lk, f1);
+            mf_mma<T, MODE>(f0, acc);
+            if (!more1) break;
+            const bool more0 = k.next();
+            if (more0) mf_fetch(k, row0, col0, m, n, li, lk, f0);
+            mf_mma<T, MODE>(f1, acc);
+            if (!more0) break;
         }
     }
-    if (row >= m) return;
+
     T* out = b.template val<T>(tl.slot) + tl.off;
     const bool useBeta = (tl.flags & TF_RUNTIME_BETA) && beta != T(0);
     const bool accum = (tl.flags & TF_ACCUMULATE);
     const int64_t ld = tl.ld;
+    auto put = [&](int row, int col, T v) {
+        if (row >= m || col >= n) return;
+        T* o = out + row + col * ld;
+        if (useBeta) *o = beta * *o + v;
+        else if (accum) *o += v;
+        else *o = v;
+    };
+    auto cidx = [&](int r) { return sizeof(T) == 8 ? lk + 4 * r : 4 * lk + r; };
+    if constexpr (S == 1) {
 #pragma unroll
-    for (int cb = 0; cb < NBMAX; ++cb) {
-        if (cb >= NB) continue;
+        for (int cb = 0; cb < CB; ++cb)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int col = cb * 16 + (sizeof(T) == 8 ? lk + 4 * r : 4 * lk + r);
-            if (col < k) {
-                T* o = out + row + col * ld;
-                const T v = acc[cb][r];
-                if (useBeta) *o = beta * *o + v;
-                else if (accum) *o += v;
-                else *o = v;
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int rb = 0; rb < RB; ++rb)
+                    put(row0 + mf_row<RB>(rb, li), col0 + mf_row<CB>(cb, cidx(r)), acc[rb][cb][r]);
+    } else {
+        // Wave w adds up register w of every wave's blocks, in wave order.
+        __shared__ T part[S][RB * CB][4][64];
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) part[w][rb * CB + cb][r][lane] = acc[rb][cb][r];
+        __syncthreads();
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb) {
+                T v = part[0][rb * CB + cb][w][lane];
+#pragma unroll
+                for (int x = 1; x < S; ++x) v += part[x][rb * CB + cb][w][lane];
+                put(row0 + mf_row<RB>(rb, li), col0 + mf_row<CB>(cb, cidx(w)), v);
             }
-        }
     }
 }
 
-template <typename T, int MODE, int MBMAX, int NBMAX, int PF>
-__global__ void __launch_bounds__(256) tile_mfma_kernel(Bases b, const Tile* __restrict__ tiles,
-                                                        const Contrib* __restrict__ cs, int ntiles, T alpha,
-                                                        T beta)
+// Units of a phase's tiles: ur x uc per tile (the phase's largest tile over
+// the unit's size), numbered tile-major. S = 1: four units per workgroup,
+// S = 4: one.
+struct MfGrid { int ur, uc; };
+
+// Workgroups are dealt to the eight XCDs in turn; kXcdRun consecutive ones of
+// the tile order go to one XCD, so that neighbouring tiles, which share
+// operands, meet in one L2 (FP32 3D update 13.7 ms with the plain order, 13.1
+// with runs of 16, 13.0 with 64; the 256^2 FP64 product 62.9, 62.1 and 62.8).
+constexpr int kXcdRun = 16;
+__device__ __forceinline__ int xcd_order(int g, int n)
 {
-    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int id = MBMAX == 4 ? (int)blockIdx.x : (int)blockIdx.x * 4 + w;
-    if (id >= ntiles) return;
-    mfma_body<T, MODE, MBMAX, NBMAX, PF>(ArgBases{b}, tiles[id], cs, MBMAX == 4 ? w : 0, alpha, beta);
+    const int full = n / (8 * kXcdRun) * (8 * kXcdRun);
+    if (g >= full) return g;
+    const int j = g >> 3;
+    return (j / kXcdRun) * (8 * kXcdRun) + (g & 7) * kXcdRun + j % kXcdRun;
 }
 
-template <typename T, int MODE, int MBMAX, int NBMAX, int PF>
-__global__ void __launch_bounds__(256) tile_mfma_seg_kernel(Bases b, const TileSeg* __restrict__ segs, int nseg,
-                                                            T alpha, T beta)
+template <typename T, int MODE, int RB, int CB, int S>
+__global__ void __launch_bounds__(256) tile_mfma_kernel(Bases b, const Tile* __restrict__ tiles,
+                                                        const Contrib* __restrict__ cs, int ntiles, MfGrid gr,
+                                                        T alpha, T beta)
 {
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const TileSeg* sg = segs + seg_of<MBMAX == 4 ? 1 : 4>(segs, nseg, (int)blockIdx.x);
-    const int local = MBMAX == 4 ? (int)blockIdx.x - sg->first1 : ((int)blockIdx.x - sg->first4) * 4 + w;
-    if (local >= sg->count) return;
-    mfma_body<T, MODE, MBMAX, NBMAX, PF>(SegBases{b, sg}, sg->tiles[local], sg->cs, MBMAX == 4 ? w : 0, alpha, beta);
+    const int g = xcd_order((int)blockIdx.x, (int)gridDim.x);
+    const int u = S == 1 ? g * 4 + w : g;
+    const int per = gr.ur * gr.uc, id = u / per, sub = u - id * per;
+    if (id >= ntiles) return;
+    mfma_body<T, MODE, RB, CB, S>(ArgBases{b}, tiles[id], cs, sub / gr.uc, sub % gr.uc, w, alpha, beta);
+}
+
+template <typename T, int MODE, int RB, int CB, int S>
+__global__ void __launch_bounds__(256) tile_mfma_seg_kernel(Bases b, const TileSeg* __restrict__ segs, int nseg,
+                                                            MfGrid gr, T alpha, T beta)
+{
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int per = gr.ur * gr.uc;
+    // Workgroups per tile (S = 4: one per unit), else four units each, a
+    // segment's last workgroup partly idle.
+    const int g = (int)blockIdx.x;
+    int u;
+    const TileSeg* sg;
+    if (S == 4) {
+        sg = segs + seg_of<1>(segs, nseg, g / per);
+        u = g - sg->first1 * per;
+    } else if (per == 4) {
+        sg = segs + seg_of<1>(segs, nseg, g);
+        u = (g - sg->first1) * 4 + w;
+    } else if (per == 2) {
+        sg = segs + seg_of<2>(segs, nseg, g);
+        u = (g - sg->first2) * 4 + w;
+    } else {
+        sg = segs + seg_of<4>(segs, nseg, g);
+        u = (g - sg->first4) * 4 + w;
+    }
+    const int id = u / per, sub = u - id * per;
+    if (id >= sg->count) return;
+    mfma_body<T, MODE, RB, CB, S>(SegBases{b, sg}, sg->tiles[id], sg->cs, sub / gr.uc, sub % gr.uc, w, alpha, beta);
+}
+
+// Units of the launch: 32 x 32 entries per wave where the phase has tiles
+// enough to give each of the 1,024 SIMDs two such waves, else 16 x 16 split
+// over the four waves of a workgroup: such a phase is one tile's latency, and
+// the split cuts it (direct inversion of 64^2 at rank 8, 940 launches of at
+// most a few hundred tiles: 15.4 -> 10.6 ms; of 256^2 at rank 16 with its
+// refinement: 648 -> 500 ms).
+constexpr int64_t kMfmaWaves = 2048;
+struct MfShape { int rb, cb, s; };
+static MfShape mf_shape(int64_t ntiles, int mmax, int kmax)
+{
+    const int rb = mmax <= 16 ? 1 : 2, cb = kmax <= 16 ? 1 : 2;
+    const int64_t units = ntiles * ((mmax + 16 * rb - 1) / (16 * rb)) * ((kmax + 16 * cb - 1) / (16 * cb));
+    if (units >= kMfmaWaves) return {rb, cb, 1};
+    return {1, 1, 4};
+}
+
+template <typename T, int MODE, int RB, int CB, int S>
+static void launch_mfma_u(const Phase& ph, const Bases& b, T alpha, T beta, hipStream_t s)
+{
+    const MfGrid gr{(ph.maxMTile + 16 * RB - 1) / (16 * RB), (ph.maxKTile + 16 * CB - 1) / (16 * CB)};
+    const int per = gr.ur * gr.uc;
+    if (!ph.segSrc.empty()) {
+        const int64_t grid = S == 4 ? (int64_t)ph.segBlocks1 * per
+                           : per == 4 ? ph.segBlocks1 : per == 2 ? ph.segBlocks2 : ph.segBlocks4;
+        if (S == 1 && per != 1 && per != 2 && per != 4) throw std::runtime_error("segmented tile units");
+        if (grid == 0) return;
+        tile_mfma_seg_kernel<T, MODE, RB, CB, S><<<(unsigned)grid, 256, 0, s>>>(
+            b, static_cast<const TileSeg*>(ph.dSegs), (int)ph.segSrc.size(), gr, alpha, beta);
+        return;
+    }
+    const int64_t units = (int64_t)ph.tiles.size() * per, grid = S == 4 ? units : (units + 3) / 4;
+    tile_mfma_kernel<T, MODE, RB, CB, S><<<(unsigned)grid, 256, 0, s>>>(
+        b, static_cast<const Tile*>(ph.dTiles), static_cast<const Contrib*>(ph.dContribs), (int)ph.tiles.size(), gr,
+        alpha, beta);
+}
+
+template <typename T, int MODE>
+static void launch_mfma(const Phase& ph, const Bases& b, T alpha, T beta, hipStream_t s)
+{
+    const int64_t n = ph.segSrc.empty() ? (int64_t)ph.tiles.size() : ph.segBlocks1;
+    const MfShape u = mf_shape(n, ph.maxMTile, ph.maxKTile);
+    if (u.s == 4) launch_mfma_u<T, MODE, 1, 1, 4>(ph, b, alpha, beta, s);
+    else if (u.rb == 1 && u.cb == 1) launch_mfma_u<T, MODE, 1, 1, 1>(ph, b, alpha, beta, s);
+    else if (u.rb == 1) launch_mfma_u<T, MODE, 1, 2, 1>(ph, b, alpha, beta, s);
+    else if (u.cb == 1) launch_mfma_u<T, MODE, 2, 1, 1>(ph, b, alpha, beta, s);
+    else launch_mfma_u<T, MODE, 2, 2, 1>(ph, b, alpha, beta, s);
 }
 
 // Segmented launches of a merged phase (its members' segment table).
-template <typename T, int MODE, int MBMAX, int PF>
-static void launch_mfma_seg_mb(const Phase& ph, const Bases& b, T alpha, T beta, hipStream_t s)
-{
-    const int grid = MBMAX == 4 ? ph.segBlocks1 : ph.segBlocks4;
-    const int nseg = (int)ph.segSrc.size();
-    const TileSeg* sg = static_cast<const TileSeg*>(ph.dSegs);
-    const int kmax = ph.maxKTile;
-    if (grid == 0) return;
-    if (kmax <= 16) tile_mfma_seg_kernel<T, MODE, MBMAX, 1, PF><<<grid, 256, 0, s>>>(b, sg, nseg, alpha, beta);
-    else if (kmax <= 32) tile_mfma_seg_kernel<T, MODE, MBMAX, 2, PF><<<grid, 256, 0, s>>>(b, sg, nseg, alpha, beta);
-    else tile_mfma_seg_kernel<T, MODE, MBMAX, 4, PF><<<grid, 256, 0, s>>>(b, sg, nseg, alpha, beta);
-}
-
 template <typename T, int MR>
 static void launch_tile_seg_mr(const Phase& ph, const Bases& b, T alpha, T beta, hipStream_t s)
 {
@@ -477,33 +751,6 @@ static void launch_tile_seg_mr(const Phase& ph, const Bases& b, T alpha, T beta,
     else tile_seg_kernel<T, MR, 64, TM, 4><<<grid, 256, 0, s>>>(b, sg, nseg, alpha, beta);
 }
 
-template <typename T, int MODE, int PF>
-static void launch_mfma_seg(const Phase& ph, const Bases& b, T alpha, T beta, hipStream_t s)
-{
-    if (ph.maxMTile <= 16) launch_mfma_seg_mb<T, MODE, 1, PF>(ph, b, alpha, beta, s);
-    else launch_mfma_seg_mb<T, MODE, 4, PF>(ph, b, alpha, beta, s);
-}
-
-template <typename T, int MODE, int MBMAX, int PF>
-static void launch_mfma_mb(int n, int kmax, const Bases& b, const Tile* t, const Contrib* c, T alpha, T beta,
-                           hipStream_t s)
-{
-    const int grid = MBMAX == 4 ? n : (n + 3) / 4;
-    if (kmax <= 16) tile_mfma_kernel<T, MODE, MBMAX, 1, PF><<<grid, 256, 0, s>>>(b, t, c, n, alpha, beta);
-    else if (kmax <= 32) tile_mfma_kernel<T, MODE, MBMAX, 2, PF><<<grid, 256, 0, s>>>(b, t, c, n, alpha, beta);
-    else tile_mfma_kernel<T, MODE, MBMAX, 4, PF><<<grid, 256, 0, s>>>(b, t, c, n, alpha, beta);
-}
-
-template <typename T, int MODE, int PF>
-static void launch_mfma(const Phase& ph, const Bases& b, T alpha, T beta, hipStream_t s)
-{
-    const int n = (int)ph.tiles.size();
-    const Tile* t = static_cast<const Tile*>(ph.dTiles);
-    const Contrib* c = static_cast<const Contrib*>(ph.dContribs);
-    if (ph.maxMTile <= 16) launch_mfma_mb<T, MODE, 1, PF>(n, ph.maxKTile, b, t, c, alpha, beta, s);
-    else launch_mfma_mb<T, MODE, 4, PF>(n, ph.maxKTile, b, t, c, alpha, beta, s);
-}
-
 template <typename T, int ROLE, int MR>
 static void launch_tile_mr(int n, int kmax, const Bases& b, const Tile* t, const Contrib* c, T alpha, T beta,
                            hipStream_t s)
@@ -512,6 +759,18 @@ static void launch_tile_mr(int n, int kmax, const Bases& b, const Tile* t, const
     if (kmax <= 16) tile_kernel<T, MR, 16, TM, 1, ROLE><<<n, 256, 0, s>>>(b, t, c, alpha, beta);
     else if (kmax <= 32) tile_kernel<T, MR, 32, TM, 2, ROLE><<<n, 256, 0, s>>>(b, t, c, alpha, beta);
     else tile_kernel<T, MR, 64, TM, 4, ROLE><<<n, 256, 0, s>>>(b, t, c, alpha, beta);
+}
+
+template <typename T>
+static void launch_mfma_engine(const Phase& ph, const Bases& b, T alpha, T beta, hipStream_t s, int engine)
+{
+    if constexpr (sizeof(T) == 4) {
+        if (engine == TILE_MFMA_BF16 || engine == TILE_MFMA_BF16_PF) {
+            launch_mfma<float, 1>(ph, b, alpha, beta, s);
+            return;
+        }
+    }
+    launch_mfma<T, 0>(ph, b, alpha, beta, s);
 }
 
 // Member segments of at least this many tiles launch one by one.
@@ -541,17 +800,7 @@ void launch_tile_phase(const Phase& ph, const Bases& b, T alpha, T beta, hipStre
             return;
         }
         if (engine != TILE_LDS) {
-            const bool bf16 = (engine == TILE_MFMA_BF16 || engine == TILE_MFMA_BF16_PF) && sizeof(T) == 4;
-            const bool pf = (engine == TILE_MFMA_PF || engine == TILE_MFMA_BF16_PF) && sizeof(T) == 4;
-            if (bf16) {
-                if constexpr (sizeof(T) == 4) {
-                    if (pf) launch_mfma_seg<float, 1, 1>(ph, b, alpha, beta, s);
-                    else launch_mfma_seg<float, 1, 0>(ph, b, alpha, beta, s);
-                }
-            } else {
-                if (pf) launch_mfma_seg<T, 0, 1>(ph, b, alpha, beta, s);
-                else launch_mfma_seg<T, 0, 0>(ph, b, alpha, beta, s);
-            }
+            launch_mfma_engine<T>(ph, b, alpha, beta, s, engine);
         } else if (ph.maxMTile <= 16) {
             launch_tile_seg_mr<T, 16>(ph, b, alpha, beta, s);
         } else {
@@ -567,19 +816,7 @@ void launch_tile_phase(const Phase& ph, const Bases& b, T alpha, T beta, hipStre
     const int kmax = ph.maxKTile;
     if (kmax > 64 || ph.maxMTile > 64) throw std::runtime_error("tile larger than 64 x 64");
     if (engine != TILE_LDS) {
-        const bool bf16 = (engine == TILE_MFMA_BF16 || engine == TILE_MFMA_BF16_PF) && sizeof(T) == 4;
-        // The prefetching form runs in FP32 only: in FP64 it produced wrong
-        // products on gfx950 (the non-prefetching form is exact).
-        const bool pf = (engine == TILE_MFMA_PF || engine == TILE_MFMA_BF16_PF) && sizeof(T) == 4;
-        if (bf16) {
-            if constexpr (sizeof(T) == 4) {
-                if (pf) launch_mfma<float, 1, 1>(ph, b, alpha, beta, s);
-                else launch_mfma<float, 1, 0>(ph, b, alpha, beta, s);
-            }
-        } else {
-            if (pf) launch_mfma<T, 0, 1>(ph, b, alpha, beta, s);
-            else launch_mfma<T, 0, 0>(ph, b, alpha, beta, s);
-        }
+        launch_mfma_engine<T>(ph, b, alpha, beta, s, engine);
         HIP_LAUNCH_CHECK();
         return;
     }

@@ -18,10 +18,10 @@ struct TruncPolicy {
 };
 
 // Tile engines: TILE_LDS, the workgroup-per-tile kernel staging operands
-// through LDS (vector FMA); TILE_MFMA, the wave-per-row-block MFMA kernel in
-// the storage precision; TILE_MFMA_BF16, the same with FP32 operands rounded
-// to BF16 and FP32 accumulation (FP64 storage falls back to TILE_MFMA); the
-// _PF forms prefetch the next chunk before the current one's MFMAs.
+// through LDS (vector FMA); TILE_MFMA, the wave-per-unit MFMA kernel in the
+// storage precision; TILE_MFMA_BF16, the same with FP32 operands rounded to
+// BF16 and FP32 accumulation (FP64 storage falls back to TILE_MFMA). The MFMA
+// kernel always prefetches; the _PF values name the same engines.
 enum TileEngine { TILE_LDS = 0, TILE_MFMA = 1, TILE_MFMA_PF = 2, TILE_MFMA_BF16 = 3, TILE_MFMA_BF16_PF = 4,
                   TILE_ENGINES = 5 };
 template <typename T>

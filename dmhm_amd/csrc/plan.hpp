@@ -114,14 +114,14 @@ enum PhaseKind { PH_TILE, PH_QR, PH_SVD, PH_RNG, PH_SCALE_C, PH_MV_ZERO, PH_MV_P
 // One member's share of a merged tile phase that is not copied: the member
 // plan's tile and contribution arrays (device) and the shifts of its slots
 // (elements, rank indices; the workspace slot is shifted to the member's
-// workspace region). first1 / first4: the member's first workgroup when a
-// workgroup takes one / four tiles.
+// workspace region). first1 / first2 / first4: the member's first workgroup
+// when a workgroup takes one / two / four tiles.
 struct TileSeg {
     const Tile* tiles;
     const Contrib* cs;
     int64_t val[NUM_SLOTS];
     int64_t rank[NUM_SLOTS];
-    int count, first1, first4, pad;
+    int count, first1, first2, first4;
 };
 
 struct Phase {
@@ -142,7 +142,7 @@ struct Phase {
     struct SegSrc { const Phase* src; int64_t val[NUM_SLOTS]; int64_t rank[NUM_SLOTS]; };
     std::vector<SegSrc> segSrc;
     void* dSegs = nullptr;
-    int segBlocks1 = 0, segBlocks4 = 0;   // workgroups of a segmented launch (1 / 4 tiles each)
+    int segBlocks1 = 0, segBlocks2 = 0, segBlocks4 = 0;   // workgroups of a segmented launch (1 / 2 / 4 tiles each)
     int mvK = 0, ldx = 0, ldy = 0;
     void* dAux = nullptr;
     int qrK = 0;            // panel width of the QR phase
