@@ -393,21 +393,17 @@ void direct_invert(dmhm_hmat_s* A, const dmhm_hh_opts& o)
 
 // Host-only lowering and bounds check of the program of a geometry at a
 // rank (standard layout); stats: sub-matrix products, merged plans, steps,
-// dense leaf inversions, workspace elements, plan phases (launches), identity
-// phases among them.
+// dense leaf inversions, workspace elements, plan phases (launches), zero.
 void check_direct_invert_program(const Geometry& g, int maxRank, int over, long long* stats)
 {
     std::vector<int> caps(g.lrBlocks.size(), std::max(maxRank, 1));
     const Layout L = Layout::make(g, caps, 0);
     auto P = build_program(g, L, maxRank, over);
     check_program(*P);
-    long long inv = 0, phases = 0, eyes = 0;
+    long long inv = 0, phases = 0;
     for (const DinvStep& st : P->steps) {
         inv += st.kind == DinvStep::INVERT;
-        if (st.kind == DinvStep::PLAN) {
-            phases += (long long)st.plan->phases.size();
-            for (const Phase& ph : st.plan->phases) eyes += ph.kind == PH_EYE;
-        }
+        if (st.kind == DinvStep::PLAN) phases += (long long)st.plan->phases.size();
     }
     stats[0] = P->products;
     stats[1] = P->plans;
@@ -415,7 +411,7 @@ void check_direct_invert_program(const Geometry& g, int maxRank, int over, long 
     stats[3] = inv;
     stats[4] = P->wsElems;
     stats[5] = phases;
-    stats[6] = eyes;
+    stats[6] = 0;
 }
 
 // Statistics of the cached program (products, merged plans, build seconds).

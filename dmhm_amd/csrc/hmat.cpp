@@ -228,13 +228,6 @@ void run_phase(Phase& ph, const Bases& b, T alpha, T beta, TruncPolicy pol, uint
     case PH_QR: launch_qr_phase<T>(ph, b, s); break;
     case PH_SVD: launch_svd_phase<T>(ph, b, pol, s); break;
     case PH_RNG: launch_rng_phase<T>(ph, b, seed, s, g_lib.seedOff); break;
-    case PH_EYE:
-        if (!ph.eyes.empty())
-            launch_eye_multi<T>(reinterpret_cast<T*>(b.val[SLOT_WS]), static_cast<const int64_t*>(ph.dTasks),
-                                (int)ph.eyes.size(), (int)ph.zeroCount, s);
-        else
-            launch_eye<T>(reinterpret_cast<T*>(b.val[SLOT_WS]) + ph.zeroOff, (int)ph.zeroCount, s);
-        break;
     case PH_MV_ZERO: case PH_MV_PROJ: case PH_MV_ACC: launch_mv_phase<T>(ph, b, alpha, beta, s); break;
     default: break;
     }
@@ -2389,6 +2382,7 @@ void Plan::upload()
                 TileSeg t{};
                 t.tiles = static_cast<const Tile*>(s.src->dTiles);
                 t.cs = static_cast<const Contrib*>(s.src->dContribs);
+                t.gtab = static_cast<const int64_t*>(s.src->dGather);
                 for (int k = 0; k < NUM_SLOTS; ++k) { t.val[k] = s.val[k]; t.rank[k] = s.rank[k]; }
                 t.count = n;
                 t.first1 = b1;
@@ -2413,6 +2407,10 @@ void Plan::upload()
             HIPCHECK(hipMalloc(&ph.dContribs, ph.contribs.size() * sizeof(Contrib)));
             HIPCHECK(copy_sync(ph.dContribs, ph.contribs.data(), ph.contribs.size() * sizeof(Contrib),
                                hipMemcpyHostToDevice));
+        }
+        if (!ph.gtab.empty()) {
+            HIPCHECK(hipMalloc(&ph.dGather, ph.gtab.size() * sizeof(int64_t)));
+            HIPCHECK(copy_sync(ph.dGather, ph.gtab.data(), ph.gtab.size() * sizeof(int64_t), hipMemcpyHostToDevice));
         }
         const void* src = nullptr; size_t bytes = 0;
         if (ph.kind == PH_QR && !ph.qr.empty()) {
@@ -2447,7 +2445,6 @@ void Plan::upload()
             src = ph.svd.data(); bytes = ph.svd.size() * sizeof(SvdTask);
         }
         if (ph.kind == PH_RNG && !ph.rng.empty()) { src = ph.rng.data(); bytes = ph.rng.size() * sizeof(RngTask); }
-        if (ph.kind == PH_EYE && !ph.eyes.empty()) { src = ph.eyes.data(); bytes = ph.eyes.size() * sizeof(int64_t); }
         if (ph.kind == PH_MV_PROJ && !ph.mvProj.empty()) {
             src = ph.mvProj.data(); bytes = ph.mvProj.size() * sizeof(MvProjItem);
         }
@@ -2465,7 +2462,10 @@ void Plan::upload()
         }
         // Host copies of the big arrays are no longer needed (unless merged
         // plans will be checked against them).
-        if (!keepHost) std::vector<Contrib>().swap(ph.contribs);
+        if (!keepHost) {
+            std::vector<Contrib>().swap(ph.contribs);
+            std::vector<int64_t>().swap(ph.gtab);
+        }
     }
 }
 
@@ -2477,7 +2477,8 @@ void Plan::release()
         if (ph.dTasks) (void)hipFree(ph.dTasks);
         if (ph.dAux) (void)hipFree(ph.dAux);
         if (ph.dSegs) (void)hipFree(ph.dSegs);
-        ph.dTiles = ph.dContribs = ph.dTasks = ph.dAux = ph.dSegs = nullptr;
+        if (ph.dGather) (void)hipFree(ph.dGather);
+        ph.dTiles = ph.dContribs = ph.dTasks = ph.dAux = ph.dSegs = ph.dGather = nullptr;
     }
 }
 } // namespace dmhm

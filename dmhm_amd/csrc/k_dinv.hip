@@ -60,24 +60,6 @@ void launch_copy_ranges(const T* src, T* dst, const CopyRange* ranges, int count
     HIP_LAUNCH_CHECK();
 }
 
-// n x n identities at base + offs[i]; blockIdx.y selects the identity.
-template <typename T>
-__global__ void eye_multi_kernel(T* base, const int64_t* __restrict__ offs, int n)
-{
-    T* x = base + offs[blockIdx.y];
-    for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < n * n; e += gridDim.x * blockDim.x)
-        x[e] = (e % n == e / n) ? T(1) : T(0);
-}
-
-template <typename T>
-void launch_eye_multi(T* base, const int64_t* offs, int count, int n, hipStream_t s)
-{
-    if (count <= 0 || n <= 0) return;
-    const dim3 grid((unsigned)std::min((n * n + 255) / 256, 64), (unsigned)count);
-    eye_multi_kernel<T><<<grid, 256, 0, s>>>(base, offs, n);
-    HIP_LAUNCH_CHECK();
-}
-
 // In-place Gauss-Jordan inversion with partial pivoting of one m x m
 // column-major matrix (leading dimension m) by one workgroup of NT threads:
 // at step k the pivot row p (largest |a(i,k)|, i >= k) is swapped into row k,
@@ -277,7 +259,6 @@ void launch_dense_inverse(const T* src, T* dst, int m, int* singular, hipStream_
 #define INST(T)                                                                                          \
     template void launch_copy_ranges<T>(const T*, T*, const CopyRange*, int, int64_t, bool, hipStream_t); \
     template void launch_arena_ranges<T>(T*, int*, const CopyRange*, int, int, int64_t, bool, hipStream_t); \
-    template void launch_eye_multi<T>(T*, const int64_t*, int, int, hipStream_t);                      \
     template void launch_dense_inverse<T>(const T*, T*, int, int*, hipStream_t);
 INST(double)
 INST(float)

@@ -52,8 +52,8 @@ __device__ __forceinline__ int contrib_q(const BV& b, const Contrib& C)
 }
 
 template <typename T, int MR, int NC, int QC, int LN, int RN, typename BV>
-__device__ __forceinline__ void tile_load(const BV& b, const Contrib& C, int p0, int q, int m, int k,
-                                          T alpha, T beta, T (&lr)[LN], T (&rr)[RN], T& a)
+__device__ __forceinline__ void tile_load(const BV& b, const Contrib& C, const int64_t* __restrict__ gt, int p0, int q,
+                                          int m, int k, T alpha, T beta, T (&lr)[LN], T (&rr)[RN], T& a)
 {
     const int tid = threadIdx.x;
     const int qc = min(QC, q - p0);
@@ -61,7 +61,7 @@ __device__ __forceinline__ void tile_load(const BV& b, const Contrib& C, int p0,
     const T* __restrict__ R = b.template val<const T>(C.rslot) + C.roff;
     a = (C.flags & CF_RUNTIME_ALPHA) ? alpha * T(C.alpha)
       : (C.flags & CF_RUNTIME_BETA) ? beta * T(C.alpha) : T(C.alpha);
-    const bool tL = C.flags & CF_TRANS_L, tR = C.flags & CF_TRANS_R;
+    const bool tL = C.flags & CF_TRANS_L, tR = C.flags & CF_TRANS_R, gR = C.flags & CF_GATHER_R;
 #pragma unroll
     for (int u = 0; u < LN; ++u) {
         const int e = tid + 256 * u;
@@ -76,7 +76,8 @@ __device__ __forceinline__ void tile_load(const BV& b, const Contrib& C, int p0,
         int jj, pp;
         if (!tR) { pp = e % QC; jj = e / QC; } else { jj = e % NC; pp = e / NC; }
         const bool ok = e < QC * NC && jj < k && pp < qc;
-        rr[u] = ok ? (!tR ? R[(p0 + pp) + (int64_t)jj * C.ldr] : R[jj + (int64_t)(p0 + pp) * C.ldr]) : T(0);
+        rr[u] = ok ? (!tR ? R[(p0 + pp) + (gR ? gt[jj] : (int64_t)jj * C.ldr)] : R[jj + (int64_t)(p0 + pp) * C.ldr])
+                   : T(0);
     }
 }
 
@@ -107,9 +108,10 @@ __device__ __forceinline__ void tile_store(T* __restrict__ Lb, T* __restrict__ R
 }
 
 template <typename T, int MR, int NC, int TM, int TN, typename BV>
-__device__ __forceinline__ void tile_body(const BV& b, const Tile& tl, const Contrib* __restrict__ cs, T alpha,
-                                          T beta)
+__device__ __forceinline__ void tile_body(const BV& b, const Tile& tl, const Contrib* __restrict__ cs,
+                                          const int64_t* __restrict__ gtab, T alpha, T beta)
 {
+    const int64_t* __restrict__ gt = gtab + tl.gather;      // read for gathered contributions only
     constexpr int QC = TileCfg<T, MR>::QC;
     constexpr int RT = MR / TM;
     static_assert(RT * (NC / TN) == 256, "the thread grid must cover 256 threads");
@@ -139,7 +141,7 @@ __device__ __forceinline__ void tile_body(const BV& b, const Tile& tl, const Con
     uint8_t flags = 0;
     if (c < tl.ce) {
         const Contrib C = cs[c];
-        tile_load<T, MR, NC, QC, LN, RN>(b, C, p0, q, m, k, alpha, beta, lr, rr, a);
+        tile_load<T, MR, NC, QC, LN, RN>(b, C, gt, p0, q, m, k, alpha, beta, lr, rr, a);
         flags = C.flags;
     }
     int buf = 0;
@@ -157,7 +159,7 @@ __device__ __forceinline__ void tile_body(const BV& b, const Tile& tl, const Con
         }
         if (c < tl.ce) {
             const Contrib C = cs[c];
-            tile_load<T, MR, NC, QC, LN, RN>(b, C, p0, q, m, k, alpha, beta, lr, rr, a);
+            tile_load<T, MR, NC, QC, LN, RN>(b, C, gt, p0, q, m, k, alpha, beta, lr, rr, a);
             flags = C.flags;
         }
         const T* __restrict__ Lb = Ls[buf];
@@ -227,9 +229,10 @@ __device__ __forceinline__ int seg_of(const TileSeg* __restrict__ segs, int nseg
 
 template <typename T, int MR, int NC, int TM, int TN, int ROLE>
 __global__ void __launch_bounds__(256) tile_kernel(Bases b, const Tile* __restrict__ tiles,
-                                                   const Contrib* __restrict__ cs, T alpha, T beta)
+                                                   const Contrib* __restrict__ cs,
+                                                   const int64_t* __restrict__ gtab, T alpha, T beta)
 {
-    tile_body<T, MR, NC, TM, TN>(ArgBases{b}, tiles[blockIdx.x], cs, alpha, beta);
+    tile_body<T, MR, NC, TM, TN>(ArgBases{b}, tiles[blockIdx.x], cs, gtab, alpha, beta);
 }
 
 template <typename T, int MR, int NC, int TM, int TN>
@@ -239,7 +242,7 @@ __global__ void __launch_bounds__(256) tile_seg_kernel(Bases b, const TileSeg* _
     const TileSeg* sg = segs + seg_of<1>(segs, nseg, (int)blockIdx.x);
     const int local = (int)blockIdx.x - sg->first1;
     if (local >= sg->count) return;
-    tile_body<T, MR, NC, TM, TN>(SegBases{b, sg}, sg->tiles[local], sg->cs, alpha, beta);
+    tile_body<T, MR, NC, TM, TN>(SegBases{b, sg}, sg->tiles[local], sg->cs, sg->gtab, alpha, beta);
 }
 
 // ---------------------------------------------------------------------------
@@ -272,15 +275,17 @@ __global__ void __launch_bounds__(256) tile_seg_kernel(Bases b, const TileSeg* _
 // contributions (every fourth one, or every fourth chunk where a tile has
 // fewer than four contributions) and add their sums through LDS in wave order.
 //
-// What bounds it: operand bytes through L2 and the 256 MB cache, and the FP64
-// MFMA (64 cycles each) where tiles are 64 x 64. Units of 32 x 32 read every
-// operand twice per 64 x 64 tile through L1 and leave room for three waves per
-// SIMD with two chunks of operands in flight each. Measured against the LDS
-// engine (FP64, 256^2, rank 16, one product): projections of 16 x 20 tiles
-// (20 GB of operands) 5.9 -> 3.0 ms, dense accumulation of 64 x 64 tiles 5.7
-// -> 4.1 ms (41 TFLOP/s), all tile phases 82 -> 55 ms; FP32 3D update 19.5
-// -> 12.3 ms. Bounding the registers for four waves per SIMD spills the 32 x 32
-// unit (6.9 -> 7.6 ms in its largest phase).
+// What bounds it: operand bytes through L2 and the 256 MB cache, the FP64 MFMA
+// (64 cycles each) where tiles are 64 x 64, and for tiles of few contributions
+// the chain of dependent loads before the first operand. Units of 32 x 32 read
+// every operand twice per 64 x 64 tile through L1 and leave room for three
+// waves per SIMD with two chunks of operands in flight each. Measured against
+// the LDS engine (FP64, 256^2, rank 16, one product): projections of 16 x 20
+// tiles (20 GB of operands) 5.9 -> 2.7 ms, dense accumulation of 64 x 64 tiles
+// 5.7 -> 3.4 ms (46 TFLOP/s of 73 that a large product reaches), all tile
+// phases 82 -> 43 ms; FP32 3D update 19.5 -> 8.8 ms. Operand loads under
+// branches on the form are slower (62 ms in all against 50), since every join
+// then waits for all of them.
 // ---------------------------------------------------------------------------
 typedef double mf_d4 __attribute__((ext_vector_type(4)));
 typedef float mf_f4 __attribute__((ext_vector_type(4)));
@@ -336,165 +341,83 @@ __device__ __forceinline__ int mf_row(int b, int j)
     return NB == 1 ? j : 32 * (b >> 1) + 2 * j + (b & 1);
 }
 
-// Fragments of one operand for one chunk: f[b][s] = X(n, p + mf_k(s, lk)), n
-// the row (column) n0 + mf_row(b, li) clamped below nmax, zero where the inner
-// index reaches q. pc: the inner dimension is contiguous, X(n, p) = X[p + n ld],
-// else X[n + p ld].
-template <typename T, int NB>
-__device__ __forceinline__ void mf_load(GPtr<T> X, int64_t ld, bool pc, int n0, int nmax, int p, int q, int li,
-                                        int lk, T (&f)[NB][4])
+// One operand of a contribution as a wave reads it: rows (columns) n0 +
+// mf_row(b, li) clamped below nmax. PC: the inner dimension is contiguous,
+// X(n, p) = X[p + n ld] (gathered columns: X[p + col[b]], the lane's own
+// offsets), else X[n + p ld]. In the second form two neighbouring rows are read
+// together (nmax >= 2): pointer 2g serves blocks 2g and 2g + 1, and a pair that
+// would cross the last row starts one row earlier (mf_moved).
+template <typename T, bool PC, int NB>
+__device__ __forceinline__ void mf_lanes(GPtr<T> X, int64_t ld, bool gathered, const int64_t (&col)[NB], int n0,
+                                         int nmax, int li, int lk, GPtr<T> (&x)[NB])
+{
+    constexpr int VP = MfVec<T>::VP;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        if (!PC && NB > 1 && (b & 1)) continue;
+        const int n = min(n0 + mf_row<NB>(b, li), nmax - (!PC && NB > 1 ? 2 : 1));
+        x[b] = X + (PC ? lk * VP + (gathered ? col[b] : n * ld) : lk * VP * ld + n);
+    }
+}
+
+// Issues the loads of the chunk at p, x + inner index (TAIL: qc < 16 indices,
+// read at the last one beyond). Nothing here waits for a load: the fragments
+// are finished in mf_finish when they are used.
+template <typename T, bool PC, bool TAIL, int NB>
+__device__ __forceinline__ void mf_issue(const GPtr<T> (&x)[NB], int64_t ld, int p, int qc, int lk, T (&f)[NB][4])
 {
     constexpr int VP = MfVec<T>::VP;
     typedef typename MfVec<T>::v2 v2;
     typedef typename MfVec<T>::vp vp;
-    const int qc = q - p;                       // uniform
-    const bool tail = qc < 16;
-    if (pc) {
-        if (!tail) {
+    auto rel = [&](int s) { return TAIL ? min(mf_k<T>(s, lk), qc - 1) - lk * VP : mf_k<T>(s, 0); };
+    if (PC && !TAIL) {
 #pragma unroll
-            for (int b = 0; b < NB; ++b) {
-                const int n = min(n0 + mf_row<NB>(b, li), nmax - 1);
-                GPtr<T> x = X + p + ((int64_t)n * ld + lk * VP);
+        for (int b = 0; b < NB; ++b)
 #pragma unroll
-                for (int h = 0; h < 4 / VP; ++h) {
-                    const vp v = *(const __attribute__((address_space(1))) vp*)(x + h * 4 * VP);
+            for (int h = 0; h < 4 / VP; ++h) {
+                const vp v = *(const __attribute__((address_space(1))) vp*)(x[b] + p + h * 4 * VP);
 #pragma unroll
-                    for (int e = 0; e < VP; ++e) f[b][h * VP + e] = v[e];
-                }
+                for (int e = 0; e < VP; ++e) f[b][h * VP + e] = v[e];
             }
-        } else {
+    } else if (PC) {
 #pragma unroll
-            for (int b = 0; b < NB; ++b) {
-                const int n = min(n0 + mf_row<NB>(b, li), nmax - 1);
-                GPtr<T> x = X + p + (int64_t)n * ld;
+        for (int b = 0; b < NB; ++b)
 #pragma unroll
-                for (int s = 0; s < 4; ++s) f[b][s] = x[min(mf_k<T>(s, lk), qc - 1)];
-            }
+            for (int s = 0; s < 4; ++s) f[b][s] = x[b][p + rel(s)];
+    } else if (NB > 1) {
 #pragma unroll
-            for (int s = 0; s < 4; ++s)
-                if (mf_k<T>(s, lk) >= qc) {
-#pragma unroll
-                    for (int b = 0; b < NB; ++b) f[b][s] = T(0);
-                }
-        }
-        return;
-    }
-    if (NB > 1 && nmax > 1) {
-        // Pairs of neighbouring rows; a pair that would cross the last row
-        // starts one row earlier and takes its second entry.
-        const bool edge = n0 + 16 * NB > nmax;  // uniform
-#pragma unroll
-        for (int g = 0; g < NB / 2; ++g) {
-            const int want = n0 + 32 * g + 2 * li, at = min(want, nmax - 2);
+        for (int g = 0; g < NB / 2; ++g)
 #pragma unroll
             for (int s = 0; s < 4; ++s) {
-                const int k = tail ? min(mf_k<T>(s, lk), qc - 1) : mf_k<T>(s, lk);
-                const v2 v = *(const __attribute__((address_space(1))) v2*)(X + p * ld + (k * ld + at));
+                const v2 v = *(const __attribute__((address_space(1))) v2*)(x[2 * g] + (p + rel(s)) * ld);
                 f[2 * g][s] = v[0];
                 f[2 * g + 1][s] = v[1];
             }
-            if (edge) {
-#pragma unroll
-                for (int s = 0; s < 4; ++s) f[2 * g][s] = want > at ? f[2 * g + 1][s] : f[2 * g][s];
-            }
-        }
     } else {
 #pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            const int n = min(n0 + mf_row<NB>(b, li), nmax - 1);
-#pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                const int k = tail ? min(mf_k<T>(s, lk), qc - 1) : mf_k<T>(s, lk);
-                f[b][s] = X[p * ld + (k * ld + n)];
-            }
-        }
-    }
-    if (tail) {
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
-            if (mf_k<T>(s, lk) >= qc) {
-#pragma unroll
-                for (int b = 0; b < NB; ++b) f[b][s] = T(0);
-            }
+        for (int s = 0; s < 4; ++s) f[0][s] = x[0][(p + rel(s)) * ld];
     }
 }
 
-// The chunks of a tile's contributions as one wave walks them (all members
-// wave-uniform but the per-lane records of the current 64 contributions).
-template <typename T, int S, typename BV>
-struct MfWalk {
-    const BV& b;
-    const Contrib* __restrict__ cs;
-    T alpha, beta;
-    int c0, ce, w, lane;
-    bool byChunk;               // S waves split chunks, not contributions
-    int chunks;                 // chunks before the current contribution (byChunk)
-    uint64_t left;              // contributions of the batch still to visit
-    // lane records
-    int64_t dl, dr;
-    int dldl, dldr, dq;
-    uint32_t dmeta;
-    float dalpha;
-    // current chunk
-    GPtr<T> L, R;
-    int64_t ldl, ldr;
-    int q, p;
-    T a;
-    bool tL, tR;
-
-    __device__ __forceinline__ void batch()
-    {
-        const int c = c0 + lane;
-        const bool in = c < ce;
-        const Contrib& C = cs[in ? c : ce - 1];
-        dl = C.loff; dr = C.roff; dldl = C.ldl; dldr = C.ldr; dalpha = C.alpha;
-        dmeta = (uint32_t)C.lslot | (uint32_t)C.rslot << 8 | (uint32_t)C.flags << 16;
-        dq = contrib_q(b, C);
-        const bool mine = S == 1 || byChunk || (lane & (S - 1)) == w;
-        left = __ballot(in && mine && dq > 0);
-    }
-    __device__ __forceinline__ MfWalk(const BV& b_, const Tile& tl, const Contrib* __restrict__ cs_, int w_, T al,
-                                      T be)
-        : b(b_), cs(cs_), alpha(al), beta(be), c0(tl.cb), ce(tl.ce), w(w_), lane(threadIdx.x & 63),
-          byChunk(S > 1 && tl.ce - tl.cb < S), chunks(0), left(0), q(0), p(0)
-    {
-        if (c0 < ce) batch();
-    }
-    // Moves to the wave's next chunk; false at the end.
-    __device__ __forceinline__ bool next()
-    {
-        p += S > 1 && byChunk ? 16 * S : 16;
-        while (p >= q) {
-            while (left == 0) {
-                c0 += 64;
-                if (c0 >= ce) return false;
-                batch();
-            }
-            const int i = __builtin_ctzll(left);
-            left &= left - 1;
-            if (S > 1 && byChunk) chunks += (q + 15) >> 4;
-            q = __builtin_amdgcn_readlane(dq, i);
-            const uint32_t m = __builtin_amdgcn_readlane(dmeta, i);
-            const int fl = (m >> 16) & 255;
-            const float ca = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(dalpha), i));
-            a = (fl & CF_RUNTIME_ALPHA) ? alpha * T(ca) : (fl & CF_RUNTIME_BETA) ? beta * T(ca) : T(ca);
-            tL = fl & CF_TRANS_L;
-            tR = fl & CF_TRANS_R;
-            ldl = __builtin_amdgcn_readlane(dldl, i);
-            ldr = __builtin_amdgcn_readlane(dldr, i);
-            L = (GPtr<T>)(b.template val<const T>(m & 255) + lane_i64(dl, i));
-            R = (GPtr<T>)(b.template val<const T>((m >> 8) & 255) + lane_i64(dr, i));
-            p = S > 1 && byChunk ? 16 * ((w - chunks) & (S - 1)) : 0;
+template <typename T, bool PC, bool TAIL, int NB>
+__device__ __forceinline__ void mf_finish(T (&f)[NB][4], int n0, int nmax, int qc, int li, int lk)
+{
+    if (!PC && NB > 1) {
+        // The even row of a pair moved down is the pair's second entry.
+#pragma unroll
+        for (int g = 0; g < NB / 2; ++g) {
+            const bool moved = n0 + 32 * g + 2 * li > nmax - 2;
+#pragma unroll
+            for (int s = 0; s < 4; ++s) f[2 * g][s] = moved ? f[2 * g + 1][s] : f[2 * g][s];
         }
-        return true;
     }
-    static __device__ __forceinline__ int64_t lane_i64(int64_t v, int i)
-    {
-        const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)v, i);
-        const uint32_t hi = __builtin_amdgcn_readlane((int)(v >> 32), i);
-        return (int64_t)((uint64_t)hi << 32 | lo);
+    if (TAIL) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) f[b][s] = mf_k<T>(s, lk) < qc ? f[b][s] : T(0);
     }
-};
+}
 
 template <typename T, int RB, int CB>
 struct MfFrag {
@@ -503,88 +426,218 @@ struct MfFrag {
     int qc;
 };
 
-template <typename T, int RB, int CB, typename W>
-__device__ __forceinline__ void mf_fetch(const W& k, int row0, int col0, int m, int n, int li, int lk,
-                                         MfFrag<T, RB, CB>& f)
-{
-    mf_load<T, RB>(k.L, k.ldl, k.tL, row0, m, k.p, k.q, li, lk, f.l);
-    mf_load<T, CB>(k.R, k.ldr, !k.tR, col0, n, k.p, k.q, li, lk, f.r);
-    f.a = k.a;
-    f.qc = k.q - k.p;
-}
+// One unit of a tile: walks the tile's contributions 64 at a time, one record
+// per lane, and within them by form (which operands have the inner dimension
+// contiguous; whole chunks, then the remainders of inner dimensions that 16
+// does not divide), so that each inner loop is free of branches on the form
+// and its loads stay in flight across the other register set's MFMAs.
+template <typename T, int MODE, int RB, int CB, int S, typename BV>
+struct MfUnit {
+    typedef typename MfAcc<T>::type Acc;
+    typedef MfFrag<T, RB, CB> Frag;
+    const BV& b;
+    T alpha, beta;
+    int w, li, lk;
+    int row0, col0, m, n;       // the unit's first row and column, the tile's extent
+    bool byChunk;               // S waves split chunks, not contributions
+    int turn;                   // chunks dealt so far (byChunk)
+    int64_t gcol[CB];           // offsets of the unit's columns in gathered right operands
+    // lane records
+    int64_t dl, dr;
+    int dldl, dldr, dq;
+    uint32_t dmeta;
+    float dalpha;
+    Acc acc[RB][CB];
 
-template <typename T, int MODE, int RB, int CB, typename Acc>
-__device__ __forceinline__ void mf_mma(MfFrag<T, RB, CB>& f, Acc (&acc)[RB][CB])
-{
-    if (f.a != T(1)) {
+    static __device__ __forceinline__ int64_t lane_i64(int64_t v, int i)
+    {
+        const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)v, i);
+        const uint32_t hi = __builtin_amdgcn_readlane((int)(v >> 32), i);
+        return (int64_t)((uint64_t)hi << 32 | lo);
+    }
+
+    __device__ __forceinline__ void mma(Frag& f)
+    {
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
             for (int s = 0; s < 4; ++s) f.l[rb][s] *= f.a;
-    }
-    if constexpr (MODE == 1) {
-#pragma unroll
-        for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-            for (int cb = 0; cb < CB; ++cb) acc[rb][cb] = mf_step_bf16(f.r[cb], f.l[rb], acc[rb][cb]);
-    } else {
-        // FP64 chunks of at most 8 inner indices fill the first two steps only.
-        constexpr int HALF = sizeof(T) == 8 ? 2 : 4;
-#pragma unroll
-        for (int s = 0; s < HALF; ++s)
+        if constexpr (MODE == 1) {
 #pragma unroll
             for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-                for (int cb = 0; cb < CB; ++cb) acc[rb][cb] = mf_step(f.r[cb][s], f.l[rb][s], acc[rb][cb]);
-        if (HALF < 4 && f.qc > 8) {
+                for (int cb = 0; cb < CB; ++cb) acc[rb][cb] = mf_step_bf16(f.r[cb], f.l[rb], acc[rb][cb]);
+        } else {
 #pragma unroll
-            for (int s = HALF; s < 4; ++s)
+            for (int s = 0; s < 4; ++s)
 #pragma unroll
                 for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
                     for (int cb = 0; cb < CB; ++cb) acc[rb][cb] = mf_step(f.r[cb][s], f.l[rb][s], acc[rb][cb]);
         }
     }
-}
+
+    // The whole chunks (TAIL: the remainders) of the contributions in `left`.
+    template <bool PL, bool PR, bool TAIL>
+    __device__ __forceinline__ void run(uint64_t left)
+    {
+        GPtr<T> L[RB], R[CB];
+        int64_t ldl = 0, ldr = 0;
+        int q = 0, p = 0;
+        T a = T(0);
+        // Moves to the wave's next chunk; at the end it stays on the last one.
+        auto next = [&]() -> bool {
+            const int last = p;
+            p += TAIL ? 16 : byChunk ? 16 * S : 16;
+            while (TAIL ? p >= q : p + 16 > q) {
+                if (left == 0) { p = last; return false; }
+                const int i = __builtin_ctzll(left);
+                left &= left - 1;
+                q = __builtin_amdgcn_readlane(dq, i);
+                if (TAIL) p = q & ~15;
+                else p = 0;
+                if (S > 1 && byChunk) {
+                    const int mine = (w - turn) & (S - 1);      // this wave's first chunk of the contribution
+                    turn += TAIL ? 1 : q >> 4;
+                    if (TAIL) p = mine == 0 ? p : q;
+                    else p = 16 * mine;
+                }
+                const uint32_t meta = __builtin_amdgcn_readlane(dmeta, i);
+                const int fl = (meta >> 16) & 255;
+                const float ca = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(dalpha), i));
+                a = (fl & CF_RUNTIME_ALPHA) ? alpha * T(ca) : (fl & CF_RUNTIME_BETA) ? beta * T(ca) : T(ca);
+                ldl = __builtin_amdgcn_readlane(dldl, i);
+                ldr = __builtin_amdgcn_readlane(dldr, i);
+                const int64_t none[RB] = {};
+                mf_lanes<T, PL, RB>((GPtr<T>)(b.template val<const T>(meta & 255) + lane_i64(dl, i)), ldl, false, none,
+                                    row0, m, li, lk, L);
+                mf_lanes<T, PR, CB>((GPtr<T>)(b.template val<const T>((meta >> 8) & 255) + lane_i64(dr, i)), ldr,
+                                    fl & CF_GATHER_R, gcol, col0, n, li, lk, R);
+            }
+            return true;
+        };
+        auto fetch = [&](Frag& f) {
+            f.a = a;
+            f.qc = q - p;
+            mf_issue<T, PL, TAIL, RB>(L, ldl, p, f.qc, lk, f.l);
+            mf_issue<T, PR, TAIL, CB>(R, ldr, p, f.qc, lk, f.r);
+        };
+        auto use = [&](Frag& f) {
+            mf_finish<T, PL, TAIL, RB>(f.l, row0, m, f.qc, li, lk);
+            mf_finish<T, PR, TAIL, CB>(f.r, col0, n, f.qc, li, lk);
+            mma(f);
+        };
+        Frag f0, f1;
+        if (!next()) return;
+        fetch(f0);
+        // After the last chunk the fetch repeats it: loads on every path keep
+        // the wait before use(f) at "all but the newest chunk" (a fetch under
+        // a branch made it "all", 62 against 50 ms per 256^2 FP64 product),
+        // and one use per register set keeps one set of accumulators.
+        while (true) {
+            const bool more1 = next();
+            fetch(f1);
+            use(f0);
+            if (!more1) break;
+            const bool more0 = next();
+            fetch(f0);
+            use(f1);
+            if (!more0) break;
+        }
+    }
+
+    // Any contributions, one chunk and one load at a time: the forms the tile
+    // plans do not use (L with, R without contiguous inner dimension) and
+    // row-contiguous operands of tiles of one row or column.
+    __device__ __forceinline__ void runAny(uint64_t left)
+    {
+        while (left) {
+            const int i = __builtin_ctzll(left);
+            left &= left - 1;
+            const int q = __builtin_amdgcn_readlane(dq, i);
+            const uint32_t meta = __builtin_amdgcn_readlane(dmeta, i);
+            const int fl = (meta >> 16) & 255;
+            const float ca = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(dalpha), i));
+            const int64_t ldl = __builtin_amdgcn_readlane(dldl, i), ldr = __builtin_amdgcn_readlane(dldr, i);
+            const bool tL = fl & CF_TRANS_L, tR = fl & CF_TRANS_R;
+            const GPtr<T> L = (GPtr<T>)(b.template val<const T>(meta & 255) + lane_i64(dl, i));
+            const GPtr<T> R = (GPtr<T>)(b.template val<const T>((meta >> 8) & 255) + lane_i64(dr, i));
+            Frag f;
+            f.a = (fl & CF_RUNTIME_ALPHA) ? alpha * T(ca) : (fl & CF_RUNTIME_BETA) ? beta * T(ca) : T(ca);
+#pragma unroll 1
+            for (int p = 0; p < q; p += 16) {
+                if (S > 1 && byChunk && (turn++ & (S - 1)) != w) continue;
+#pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    const int k = p + mf_k<T>(s, lk), kc = min(k, q - 1);
+#pragma unroll
+                    for (int rb = 0; rb < RB; ++rb) {
+                        const int r = min(row0 + mf_row<RB>(rb, li), m - 1);
+                        const T v = L[tL ? kc + r * ldl : r + kc * ldl];
+                        f.l[rb][s] = k < q ? v : T(0);
+                    }
+#pragma unroll
+                    for (int cb = 0; cb < CB; ++cb) {
+                        const int c = min(col0 + mf_row<CB>(cb, li), n - 1);
+                        const T v = R[tR ? c + kc * ldr : kc + ((fl & CF_GATHER_R) ? gcol[cb] : c * ldr)];
+                        f.r[cb][s] = k < q ? v : T(0);
+                    }
+                }
+                mma(f);
+            }
+        }
+    }
+
+    __device__ __forceinline__ void contributions(const Tile& tl, const Contrib* __restrict__ cs)
+    {
+        const int lane = 16 * lk + li;
+        for (int c0 = tl.cb; c0 < tl.ce; c0 += 64) {
+            const int c = c0 + lane;
+            const bool in = c < tl.ce;
+            const Contrib& C = cs[in ? c : tl.ce - 1];
+            dl = C.loff; dr = C.roff; dldl = C.ldl; dldr = C.ldr; dalpha = C.alpha;
+            dmeta = (uint32_t)C.lslot | (uint32_t)C.rslot << 8 | (uint32_t)C.flags << 16;
+            dq = contrib_q(b, C);
+            const bool mine = in && dq > 0 && (S == 1 || byChunk || (lane & (S - 1)) == w);
+            const bool pl = C.flags & CF_TRANS_L, pr = !(C.flags & CF_TRANS_R);
+            const bool any = (pl && !pr) || (RB > 1 && !pl && m < 2) || (CB > 1 && !pr && n < 2);
+            const bool whole = mine && !any && dq >= 16, rest = mine && !any && (dq & 15);
+            run<false, true, false>(__ballot(whole && !pl && pr));
+            run<false, true, true>(__ballot(rest && !pl && pr));
+            run<true, true, false>(__ballot(whole && pl && pr));
+            run<true, true, true>(__ballot(rest && pl && pr));
+            run<false, false, false>(__ballot(whole && !pl && !pr));
+            run<false, false, true>(__ballot(rest && !pl && !pr));
+            runAny(__ballot(mine && any));
+        }
+    }
+};
 
 // One unit (row group ur, column group uc) of tile tl; w: the wave's share of
 // the contributions (S > 1).
 template <typename T, int MODE, int RB, int CB, int S, typename BV>
-__device__ __forceinline__ void mfma_body(const BV& b, const Tile& tl, const Contrib* __restrict__ cs, int ur,
-                                          int uc, int w, T alpha, T beta)
+__device__ __forceinline__ void mfma_body(const BV& b, const Tile& tl, const Contrib* __restrict__ cs,
+                                          const int64_t* __restrict__ gtab, int ur, int uc, int w, T alpha, T beta)
 {
     static_assert(MODE == 0 || sizeof(T) == 4, "the BF16 mode reads FP32 operands");
     static_assert(S == 1 || S == 4, "one wave or the four waves of a workgroup per unit");
-    typedef typename MfAcc<T>::type Acc;
     int m = tl.m, n = tl.k;
     if (tl.mrank >= 0) m = min(m, max(0, b.rank(tl.mslot)[tl.mrank] - tl.moff));
     if (tl.krank >= 0) n = min(n, max(0, b.rank(tl.kslot)[tl.krank] - tl.koff));
     const int row0 = ur * 16 * RB, col0 = uc * 16 * CB;
     if (m <= row0 || n <= col0) return;         // uniform over the waves that share the unit
     const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
-    Acc acc[RB][CB];
+    MfUnit<T, MODE, RB, CB, S, BV> u{b, alpha, beta, w, li, lk, row0, col0, m, n, S > 1 && tl.ce - tl.cb < S, 0};
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb)
+        u.gcol[cb] = tl.gather >= 0 ? gtab[tl.gather + min(col0 + mf_row<CB>(cb, li), n - 1)] : 0;
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
         for (int cb = 0; cb < CB; ++cb)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) acc[rb][cb][r] = T(0);
-
-    MfWalk<T, S, BV> k(b, tl, cs, w, alpha, beta);
-    MfFrag<T, RB, CB> f0, f1;
-    if (k.next()) {
-        mf_fetch(k, row0, col0, m, n, li, lk, f0);
-        while (true) {
-            const bool more1 = k.next();
-            if (more1) mf_fetch(k, row0, col0, m, n, li, lk, f1);
-            mf_mma<T, MODE>(f0, acc);
-            if (!more1) break;
-            const bool more0 = k.next();
-            if (more0) mf_fetch(k, row0, col0, m, n, li, lk, f0);
-            mf_mma<T, MODE>(f1, acc);
-            if (!more0) break;
-        }
-    }
+            for (int r = 0; r < 4; ++r) u.acc[rb][cb][r] = T(0);
+    u.contributions(tl, cs);
 
     T* out = b.template val<T>(tl.slot) + tl.off;
     const bool useBeta = (tl.flags & TF_RUNTIME_BETA) && beta != T(0);
@@ -605,7 +658,7 @@ __device__ __forceinline__ void mfma_body(const BV& b, const Tile& tl, const Con
             for (int r = 0; r < 4; ++r)
 #pragma unroll
                 for (int rb = 0; rb < RB; ++rb)
-                    put(row0 + mf_row<RB>(rb, li), col0 + mf_row<CB>(cb, cidx(r)), acc[rb][cb][r]);
+                    put(row0 + mf_row<RB>(rb, li), col0 + mf_row<CB>(cb, cidx(r)), u.acc[rb][cb][r]);
     } else {
         // Wave w adds up register w of every wave's blocks, in wave order.
         __shared__ T part[S][RB * CB][4][64];
@@ -614,7 +667,7 @@ __device__ __forceinline__ void mfma_body(const BV& b, const Tile& tl, const Con
 #pragma unroll
             for (int cb = 0; cb < CB; ++cb)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) part[w][rb * CB + cb][r][lane] = acc[rb][cb][r];
+                for (int r = 0; r < 4; ++r) part[w][rb * CB + cb][r][lane] = u.acc[rb][cb][r];
         __syncthreads();
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb)
@@ -648,7 +701,8 @@ __device__ __forceinline__ int xcd_order(int g, int n)
 
 template <typename T, int MODE, int RB, int CB, int S>
 __global__ void __launch_bounds__(256) tile_mfma_kernel(Bases b, const Tile* __restrict__ tiles,
-                                                        const Contrib* __restrict__ cs, int ntiles, MfGrid gr,
+                                                        const Contrib* __restrict__ cs,
+                                                        const int64_t* __restrict__ gtab, int ntiles, MfGrid gr,
                                                         T alpha, T beta)
 {
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -656,7 +710,7 @@ __global__ void __launch_bounds__(256) tile_mfma_kernel(Bases b, const Tile* __r
     const int u = S == 1 ? g * 4 + w : g;
     const int per = gr.ur * gr.uc, id = u / per, sub = u - id * per;
     if (id >= ntiles) return;
-    mfma_body<T, MODE, RB, CB, S>(ArgBases{b}, tiles[id], cs, sub / gr.uc, sub % gr.uc, w, alpha, beta);
+    mfma_body<T, MODE, RB, CB, S>(ArgBases{b}, tiles[id], cs, gtab, sub / gr.uc, sub % gr.uc, w, alpha, beta);
 }
 
 template <typename T, int MODE, int RB, int CB, int S>
@@ -685,7 +739,8 @@ __global__ void __launch_bounds__(256) tile_mfma_seg_kernel(Bases b, const TileS
     }
     const int id = u / per, sub = u - id * per;
     if (id >= sg->count) return;
-    mfma_body<T, MODE, RB, CB, S>(SegBases{b, sg}, sg->tiles[id], sg->cs, sub / gr.uc, sub % gr.uc, w, alpha, beta);
+    mfma_body<T, MODE, RB, CB, S>(SegBases{b, sg}, sg->tiles[id], sg->cs, sg->gtab, sub / gr.uc, sub % gr.uc, w, alpha,
+                                  beta);
 }
 
 // Units of the launch: 32 x 32 entries per wave where the phase has tiles
@@ -720,8 +775,8 @@ static void launch_mfma_u(const Phase& ph, const Bases& b, T alpha, T beta, hipS
     }
     const int64_t units = (int64_t)ph.tiles.size() * per, grid = S == 4 ? units : (units + 3) / 4;
     tile_mfma_kernel<T, MODE, RB, CB, S><<<(unsigned)grid, 256, 0, s>>>(
-        b, static_cast<const Tile*>(ph.dTiles), static_cast<const Contrib*>(ph.dContribs), (int)ph.tiles.size(), gr,
-        alpha, beta);
+        b, static_cast<const Tile*>(ph.dTiles), static_cast<const Contrib*>(ph.dContribs),
+        static_cast<const int64_t*>(ph.dGather), (int)ph.tiles.size(), gr, alpha, beta);
 }
 
 template <typename T, int MODE>
@@ -752,13 +807,13 @@ static void launch_tile_seg_mr(const Phase& ph, const Bases& b, T alpha, T beta,
 }
 
 template <typename T, int ROLE, int MR>
-static void launch_tile_mr(int n, int kmax, const Bases& b, const Tile* t, const Contrib* c, T alpha, T beta,
-                           hipStream_t s)
+static void launch_tile_mr(int n, int kmax, const Bases& b, const Tile* t, const Contrib* c, const int64_t* g, T alpha,
+                           T beta, hipStream_t s)
 {
     constexpr int TM = MR == 64 ? 4 : 1;
-    if (kmax <= 16) tile_kernel<T, MR, 16, TM, 1, ROLE><<<n, 256, 0, s>>>(b, t, c, alpha, beta);
-    else if (kmax <= 32) tile_kernel<T, MR, 32, TM, 2, ROLE><<<n, 256, 0, s>>>(b, t, c, alpha, beta);
-    else tile_kernel<T, MR, 64, TM, 4, ROLE><<<n, 256, 0, s>>>(b, t, c, alpha, beta);
+    if (kmax <= 16) tile_kernel<T, MR, 16, TM, 1, ROLE><<<n, 256, 0, s>>>(b, t, c, g, alpha, beta);
+    else if (kmax <= 32) tile_kernel<T, MR, 32, TM, 2, ROLE><<<n, 256, 0, s>>>(b, t, c, g, alpha, beta);
+    else tile_kernel<T, MR, 64, TM, 4, ROLE><<<n, 256, 0, s>>>(b, t, c, g, alpha, beta);
 }
 
 template <typename T>
@@ -813,6 +868,7 @@ void launch_tile_phase(const Phase& ph, const Bases& b, T alpha, T beta, hipStre
     if (n == 0) return;
     const Tile* t = static_cast<const Tile*>(ph.dTiles);
     const Contrib* c = static_cast<const Contrib*>(ph.dContribs);
+    const int64_t* g = static_cast<const int64_t*>(ph.dGather);
     const int kmax = ph.maxKTile;
     if (kmax > 64 || ph.maxMTile > 64) throw std::runtime_error("tile larger than 64 x 64");
     if (engine != TILE_LDS) {
@@ -823,11 +879,11 @@ void launch_tile_phase(const Phase& ph, const Bases& b, T alpha, T beta, hipStre
     // ROLE only distinguishes projection and accumulation launches in profiles;
     // MR = 16 serves phases whose tiles all have at most 16 rows.
     if (ph.maxMTile <= 16) {
-        if (ph.role == 1) launch_tile_mr<T, 1, 16>(n, kmax, b, t, c, alpha, beta, s);
-        else launch_tile_mr<T, 0, 16>(n, kmax, b, t, c, alpha, beta, s);
+        if (ph.role == 1) launch_tile_mr<T, 1, 16>(n, kmax, b, t, c, g, alpha, beta, s);
+        else launch_tile_mr<T, 0, 16>(n, kmax, b, t, c, g, alpha, beta, s);
     } else {
-        if (ph.role == 1) launch_tile_mr<T, 1, 64>(n, kmax, b, t, c, alpha, beta, s);
-        else launch_tile_mr<T, 0, 64>(n, kmax, b, t, c, alpha, beta, s);
+        if (ph.role == 1) launch_tile_mr<T, 1, 64>(n, kmax, b, t, c, g, alpha, beta, s);
+        else launch_tile_mr<T, 0, 64>(n, kmax, b, t, c, g, alpha, beta, s);
     }
     HIP_LAUNCH_CHECK();
 }

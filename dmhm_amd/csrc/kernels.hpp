@@ -42,8 +42,6 @@ template <typename T> void launch_fill(T* x, int64_t n, T v, hipStream_t s);
 // out = a + alpha * b (elementwise)
 template <typename T> void launch_axpby(const T* a, const T* b, T alpha, T* out, int64_t n, hipStream_t s);
 void launch_fill_int(int* x, int64_t n, int v, hipStream_t s);
-// x (n x n, ld n) = identity
-template <typename T> void launch_eye(T* x, int n, hipStream_t s);
 template <typename Ts, typename Td> void launch_convert(const Ts* x, Td* y, int64_t n, hipStream_t s);
 // Seeds add the device word *seedOff when it is given (graph-replayed loops).
 template <typename T> void launch_gaussian(T* x, int64_t n, uint64_t seed, uint64_t stream, hipStream_t s,
@@ -76,8 +74,6 @@ template <typename T> void launch_copy_ranges(const T* src, T* dst, const CopyRa
 // launch; maxLen bounds every range's length.
 template <typename T> void launch_arena_ranges(T* vals, int* ranks, const CopyRange* ranges, int nVal, int nRank,
                                                int64_t maxLen, bool fill, hipStream_t s);
-// count n x n identities at base + offs[i] (offs on the device)
-template <typename T> void launch_eye_multi(T* base, const int64_t* offs, int count, int n, hipStream_t s);
 // dst (m x m, ld m) = inverse of src (Gauss-Jordan, partial pivoting); a zero
 // pivot sets *singular (device int).
 template <typename T> void launch_dense_inverse(const T* src, T* dst, int m, int* singular, hipStream_t s);

@@ -32,7 +32,11 @@ namespace dmhm {
 enum Slot : uint8_t { SLOT_A = 0, SLOT_B = 1, SLOT_C = 2, SLOT_WS = 3, SLOT_X = 4, SLOT_Y = 5,
                       SLOT_WIDTH = 6, SLOT_FLAG = 7, NUM_SLOTS = 8 };
 
-enum ContribFlags : uint8_t { CF_TRANS_L = 1, CF_TRANS_R = 2, CF_RUNTIME_ALPHA = 4, CF_RUNTIME_BETA = 8 };
+// CF_GATHER_R: the right operand is a panel of scattered columns; column j of
+// the tile starts at element gtab[Tile::gather + j] + roff of the slot
+// (Phase::gtab; ldr unused, not transposed).
+enum ContribFlags : uint8_t { CF_TRANS_L = 1, CF_TRANS_R = 2, CF_RUNTIME_ALPHA = 4, CF_RUNTIME_BETA = 8,
+                              CF_GATHER_R = 16 };
 enum TileFlags : uint8_t { TF_ACCUMULATE = 1, TF_RUNTIME_BETA = 2 };
 
 // Plain-old-data records shared with the kernels.
@@ -53,7 +57,7 @@ struct Tile {
     int32_t moff, koff;
     int32_t cb, ce;         // contribution range
     uint8_t slot, mslot, kslot, flags;
-    int32_t pad;
+    int32_t gather = -1;    // first entry of the tile's columns in Phase::gtab, or -1
 };
 
 struct QrTask {              // Householder QR of an m x k panel, Q in place
@@ -109,16 +113,17 @@ struct MvContrib {
     int32_t pad;
 };
 
-enum PhaseKind { PH_TILE, PH_QR, PH_SVD, PH_RNG, PH_SCALE_C, PH_MV_ZERO, PH_MV_PROJ, PH_MV_ACC, PH_EYE };
+enum PhaseKind { PH_TILE, PH_QR, PH_SVD, PH_RNG, PH_SCALE_C, PH_MV_ZERO, PH_MV_PROJ, PH_MV_ACC };
 
 // One member's share of a merged tile phase that is not copied: the member
-// plan's tile and contribution arrays (device) and the shifts of its slots
+// plan's tile, contribution and gather arrays (device) and the shifts of its slots
 // (elements, rank indices; the workspace slot is shifted to the member's
 // workspace region). first1 / first2 / first4: the member's first workgroup
 // when a workgroup takes one / two / four tiles.
 struct TileSeg {
     const Tile* tiles;
     const Contrib* cs;
+    const int64_t* gtab;
     int64_t val[NUM_SLOTS];
     int64_t rank[NUM_SLOTS];
     int count, first1, first2, first4;
@@ -134,8 +139,8 @@ struct Phase {
     std::vector<MvProjItem> mvProj;
     std::vector<MvAtom> mvAtoms;
     std::vector<MvContrib> mvContribs;
-    int64_t zeroOff = 0, zeroCount = 0;   // PH_MV_ZERO range in the workspace; PH_EYE: offset, order
-    std::vector<int64_t> eyes;            // PH_EYE of a merged plan: every identity's workspace offset
+    int64_t zeroOff = 0, zeroCount = 0;   // PH_MV_ZERO range in the workspace
+    std::vector<int64_t> gtab;            // PH_TILE: column offsets of gathered right operands
     // PH_TILE of a merged plan built without copying: per member, the source
     // phase (host, uploaded with its plan) and the member's shifts; the
     // device table of TileSeg is built at upload.
@@ -150,7 +155,7 @@ struct Phase {
     int qrRegK = 0;         // widest task of classes 0..3
     int svdK = 0;           // largest SVD factor of the phase (set by upload)
     // device copies (filled by upload)
-    void* dTiles = nullptr; void* dContribs = nullptr; void* dTasks = nullptr;
+    void* dTiles = nullptr; void* dContribs = nullptr; void* dTasks = nullptr; void* dGather = nullptr;
     int maxKTile = 0;       // widest tile (selects the kernel variant)
     int maxMTile = 0;       // tallest tile
     int role = 0;           // 0 accumulation, 1 projection (profiling identity)
@@ -189,6 +194,7 @@ public:
     explicit PhaseBuilder(Phase& ph) : ph_(ph) {}
     int addTile(const Tile& t) { ph_.tiles.push_back(t); return (int)ph_.tiles.size() - 1; }
     void add(int tile, const Contrib& c) { pending_.push_back({tile, c}); }
+    void setGather(int tile, int at) { ph_.tiles[tile].gather = at; }
     void finalize();
 private:
     Phase& ph_;
@@ -199,6 +205,7 @@ struct Operand {            // a panel or matrix block region
     uint8_t slot;
     int64_t off;
     int32_t ld;
+    int32_t gather = -1;    // scattered columns: first entry in the phase's gtab (off: row offset)
 };
 
 // Terms of C = A B for three H-matrices of one geometry, from the reference's

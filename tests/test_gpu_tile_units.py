@@ -46,3 +46,28 @@ def test_products_at_unit_edges(case, prec):
             assert np.all(np.abs(got - ref) <= bound), (op, float((np.abs(got - ref) / bound).max()))
     finally:
         dmhm_amd.set_tile_engine(prev)
+
+
+@pytest.mark.parametrize("engine", ["mfma", "lds"])
+@pytest.mark.parametrize("sizes,levels,r", [((16, 16), 3, 5), ((33, 37), 3, 12), ((50, 41), 4, 16), ((64, 64), 4, 20),
+                                            ((13, 9, 11), 3, 7)])
+def test_stacked_factors_read_through_the_table(sizes, levels, r, engine):
+    """A B for A, B at full rank, whose low-rank terms are stacked: 64-column
+    chunks of a stack start inside a factor when r does not divide 64."""
+    n = int(np.prod(sizes))
+    rng = np.random.default_rng(7 * n + r)
+    U, V, S, T = (rng.standard_normal((n, r)) for _ in range(4))
+    X = rng.standard_normal((n, 3))
+    cls = dmhm_amd.HMat2d if len(sizes) == 2 else dmhm_amd.HMat3d
+    A = cls.from_lowrank(sizes, levels, r, True, U, V)
+    B = cls.from_lowrank(sizes, levels, r, True, S, T)
+    prev = dmhm_amd.set_tile_engine(engine)
+    try:
+        got = A.Multiply(2.0, B).Multiply(1.0, X)
+    finally:
+        dmhm_amd.set_tile_engine(prev)
+    ref = 2.0 * (U @ ((V.T @ S) @ (T.T @ X)))
+    scale = np.abs(U) @ (np.abs(V.T @ S) @ (np.abs(T.T) @ np.abs(X)))
+    # n roundings through each product, and a factor 1000 for the conditioning
+    # of a Gaussian sketch of r + 4 columns of a block of rank r.
+    assert np.linalg.norm(got - ref) <= 1000 * n * np.finfo(float).eps * np.linalg.norm(2.0 * scale)
