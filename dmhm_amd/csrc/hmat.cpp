@@ -2374,7 +2374,7 @@ void Plan::upload()
             // Segment table of a merged tile phase: the members' source
             // arrays must already be on the device.
             std::vector<TileSeg> segs;
-            int b1 = 0, b2 = 0, b4 = 0;
+            ph.segTiles = ph.segBlocks[0] = ph.segBlocks[1] = ph.segBlocks[2] = 0;
             for (const auto& s : ph.segSrc) {
                 const int n = (int)s.src->tiles.size();
                 if (n > 0 && (!s.src->dTiles || !s.src->dContribs))
@@ -2385,21 +2385,20 @@ void Plan::upload()
                 t.gtab = static_cast<const int64_t*>(s.src->dGather);
                 for (int k = 0; k < NUM_SLOTS; ++k) { t.val[k] = s.val[k]; t.rank[k] = s.rank[k]; }
                 t.count = n;
-                t.first1 = b1;
-                t.first2 = b2;
-                t.first4 = b4;
-                b1 += n;
-                b2 += (n + 1) / 2;
-                b4 += (n + 3) / 4;
+                t.nLong = s.src->nLong;
+                t.first = ph.segTiles;
+                ph.segTiles += n;
+                for (int i = 0; i < 3; ++i) {
+                    t.firstUnit[i] = ph.segBlocks[i];
+                    ph.segBlocks[i] += (t.nLong << i) + (((n - t.nLong) << i) + 3) / 4;
+                }
                 segs.push_back(t);
             }
-            ph.segBlocks1 = b1;
-            ph.segBlocks2 = b2;
-            ph.segBlocks4 = b4;
             HIPCHECK(hipMalloc(&ph.dSegs, segs.size() * sizeof(TileSeg)));
             HIPCHECK(copy_sync(ph.dSegs, segs.data(), segs.size() * sizeof(TileSeg), hipMemcpyHostToDevice));
         }
         if (!ph.tiles.empty()) {
+            order_tiles(ph);
             HIPCHECK(hipMalloc(&ph.dTiles, ph.tiles.size() * sizeof(Tile)));
             HIPCHECK(copy_sync(ph.dTiles, ph.tiles.data(), ph.tiles.size() * sizeof(Tile), hipMemcpyHostToDevice));
         }

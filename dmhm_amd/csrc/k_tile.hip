@@ -199,32 +199,24 @@ __device__ __forceinline__ void tile_body(const BV& b, const Tile& tl, const Con
 }
 
 // Segmented launches (merged plans of independent members): the member
-// segment holding workgroup g, found by bisection over the segments' first
-// workgroups (one, two or four tiles per workgroup), and the member's bases, the
-// launch's bases shifted by the member's offsets.
-template <int TPB>
-__device__ __forceinline__ int seg_first(const TileSeg& s)
-{
-    return TPB == 1 ? s.first1 : TPB == 2 ? s.first2 : s.first4;
-}
-template <int TPB>
-__device__ __forceinline__ int seg_of(const TileSeg* __restrict__ segs, int nseg, int g)
+// segment holding workgroup g, the last one whose first workgroup (first(sg))
+// is at or before g.
+template <typename F>
+__device__ __forceinline__ const TileSeg* seg_of(const TileSeg* __restrict__ segs, int nseg, int g, F first)
 {
     if (nseg <= 64) {
-        // One load per lane and a ballot: the segment is the last one whose
-        // first workgroup is at or before g.
+        // One load per lane and a ballot.
         const int l = threadIdx.x & 63;
-        const int f = l < nseg ? seg_first<TPB>(segs[l]) : INT_MAX;
-        return (int)__popcll(__ballot(f <= g)) - 1;
+        const int f = l < nseg ? first(segs[l]) : INT_MAX;
+        return segs + (int)__popcll(__ballot(f <= g)) - 1;
     }
     int lo = 0, hi = nseg - 1;
     while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
-        const int f = seg_first<TPB>(segs[mid]);
-        if (f <= g) lo = mid;
+        if (first(segs[mid]) <= g) lo = mid;
         else hi = mid - 1;
     }
-    return lo;
+    return segs + lo;
 }
 
 template <typename T, int MR, int NC, int TM, int TN, int ROLE>
@@ -239,8 +231,8 @@ template <typename T, int MR, int NC, int TM, int TN>
 __global__ void __launch_bounds__(256) tile_seg_kernel(Bases b, const TileSeg* __restrict__ segs, int nseg, T alpha,
                                                        T beta)
 {
-    const TileSeg* sg = segs + seg_of<1>(segs, nseg, (int)blockIdx.x);
-    const int local = (int)blockIdx.x - sg->first1;
+    const TileSeg* sg = seg_of(segs, nseg, (int)blockIdx.x, [](const TileSeg& s) { return s.first; });
+    const int local = (int)blockIdx.x - sg->first;
     if (local >= sg->count) return;
     tile_body<T, MR, NC, TM, TN>(SegBases{b, sg}, sg->tiles[local], sg->cs, sg->gtab, alpha, beta);
 }
@@ -682,8 +674,7 @@ __device__ __forceinline__ void mfma_body(const BV& b, const Tile& tl, const Con
 }
 
 // Units of a phase's tiles: ur x uc per tile (the phase's largest tile over
-// the unit's size), numbered tile-major. S = 1: four units per workgroup,
-// S = 4: one.
+// the unit's size), numbered tile-major.
 struct MfGrid { int ur, uc; };
 
 // Workgroups are dealt to the eight XCDs in turn; kXcdRun consecutive ones of
@@ -691,104 +682,99 @@ struct MfGrid { int ur, uc; };
 // operands, meet in one L2 (FP32 3D update 13.7 ms with the plain order, 13.1
 // with runs of 16, 13.0 with 64; the 256^2 FP64 product 62.9, 62.1 and 62.8).
 constexpr int kXcdRun = 16;
+template <int RUN>
 __device__ __forceinline__ int xcd_order(int g, int n)
 {
-    const int full = n / (8 * kXcdRun) * (8 * kXcdRun);
+    const int full = n / (8 * RUN) * (8 * RUN);
     if (g >= full) return g;
     const int j = g >> 3;
-    return (j / kXcdRun) * (8 * kXcdRun) + (g & 7) * kXcdRun + j % kXcdRun;
+    return (j / RUN) * (8 * RUN) + (g & 7) * RUN + j % RUN;
 }
 
-template <typename T, int MODE, int RB, int CB, int S>
+// Unit of workgroup g and wave w of a tile list: every unit a workgroup's (ALL),
+// or the units of the first nLong tiles a workgroup's and the others a wave's.
+template <typename T, int MODE, int RB, int CB, bool ALL, typename BV>
+__device__ __forceinline__ void mfma_unit(const BV& b, const Tile* __restrict__ tiles,
+                                          const Contrib* __restrict__ cs, const int64_t* __restrict__ gtab, int ntiles,
+                                          int nLong, MfGrid gr, int g, int w, T alpha, T beta)
+{
+    const int per = gr.ur * gr.uc;
+    if (ALL || g < nLong * per) {
+        const int id = g / per, sub = g - id * per;
+        if (id >= ntiles) return;
+        mfma_body<T, MODE, RB, CB, 4>(b, tiles[id], cs, gtab, sub / gr.uc, sub % gr.uc, w, alpha, beta);
+    } else {
+        const int u = (g - nLong * per) * 4 + w, at = u / per, id = nLong + at, sub = u - at * per;
+        if (id >= ntiles) return;
+        mfma_body<T, MODE, RB, CB, 1>(b, tiles[id], cs, gtab, sub / gr.uc, sub % gr.uc, w, alpha, beta);
+    }
+}
+
+template <typename T, int MODE, int RB, int CB, bool ALL>
 __global__ void __launch_bounds__(256) tile_mfma_kernel(Bases b, const Tile* __restrict__ tiles,
                                                         const Contrib* __restrict__ cs,
-                                                        const int64_t* __restrict__ gtab, int ntiles, MfGrid gr,
-                                                        T alpha, T beta)
+                                                        const int64_t* __restrict__ gtab, int ntiles, int nLong,
+                                                        MfGrid gr, T alpha, T beta)
 {
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int g = xcd_order((int)blockIdx.x, (int)gridDim.x);
-    const int u = S == 1 ? g * 4 + w : g;
-    const int per = gr.ur * gr.uc, id = u / per, sub = u - id * per;
-    if (id >= ntiles) return;
-    mfma_body<T, MODE, RB, CB, S>(ArgBases{b}, tiles[id], cs, gtab, sub / gr.uc, sub % gr.uc, w, alpha, beta);
+    const int lng = ALL ? 0 : nLong * gr.ur * gr.uc, g0 = (int)blockIdx.x;
+    const int g = g0 < lng ? xcd_order<4>(g0, lng) : lng + xcd_order<kXcdRun>(g0 - lng, (int)gridDim.x - lng);
+    mfma_unit<T, MODE, RB, CB, ALL>(ArgBases{b}, tiles, cs, gtab, ntiles, nLong, gr, g, w, alpha, beta);
 }
 
-template <typename T, int MODE, int RB, int CB, int S>
+template <typename T, int MODE, int RB, int CB, bool ALL>
 __global__ void __launch_bounds__(256) tile_mfma_seg_kernel(Bases b, const TileSeg* __restrict__ segs, int nseg,
-                                                            MfGrid gr, T alpha, T beta)
+                                                            MfGrid gr, int unitLog, T alpha, T beta)
 {
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int per = gr.ur * gr.uc;
-    // Workgroups per tile (S = 4: one per unit), else four units each, a
-    // segment's last workgroup partly idle.
-    const int g = (int)blockIdx.x;
-    int u;
-    const TileSeg* sg;
-    if (S == 4) {
-        sg = segs + seg_of<1>(segs, nseg, g / per);
-        u = g - sg->first1 * per;
-    } else if (per == 4) {
-        sg = segs + seg_of<1>(segs, nseg, g);
-        u = (g - sg->first1) * 4 + w;
-    } else if (per == 2) {
-        sg = segs + seg_of<2>(segs, nseg, g);
-        u = (g - sg->first2) * 4 + w;
-    } else {
-        sg = segs + seg_of<4>(segs, nseg, g);
-        u = (g - sg->first4) * 4 + w;
-    }
-    const int id = u / per, sub = u - id * per;
-    if (id >= sg->count) return;
-    mfma_body<T, MODE, RB, CB, S>(SegBases{b, sg}, sg->tiles[id], sg->cs, sg->gtab, sub / gr.uc, sub % gr.uc, w, alpha,
-                                  beta);
+    auto first = [=](const TileSeg& s) { return ALL ? s.first * per : s.firstUnit[unitLog]; };
+    const TileSeg* sg = seg_of(segs, nseg, (int)blockIdx.x, first);
+    mfma_unit<T, MODE, RB, CB, ALL>(SegBases{b, sg}, sg->tiles, sg->cs, sg->gtab, sg->count, sg->nLong, gr,
+                                    (int)blockIdx.x - first(*sg), w, alpha, beta);
 }
 
-// Units of the launch: 32 x 32 entries per wave where the phase has tiles
-// enough to give each of the 1,024 SIMDs two such waves, else 16 x 16 split
-// over the four waves of a workgroup: such a phase is one tile's latency, and
-// the split cuts it (direct inversion of 64^2 at rank 8, 940 launches of at
-// most a few hundred tiles: 15.4 -> 10.6 ms; of 256^2 at rank 16 with its
-// refinement: 648 -> 500 ms).
-constexpr int64_t kMfmaWaves = 2048;
-struct MfShape { int rb, cb, s; };
-static MfShape mf_shape(int64_t ntiles, int mmax, int kmax)
-{
-    const int rb = mmax <= 16 ? 1 : 2, cb = kmax <= 16 ? 1 : 2;
-    const int64_t units = ntiles * ((mmax + 16 * rb - 1) / (16 * rb)) * ((kmax + 16 * cb - 1) / (16 * cb));
-    if (units >= kMfmaWaves) return {rb, cb, 1};
-    return {1, 1, 4};
-}
-
-template <typename T, int MODE, int RB, int CB, int S>
+template <typename T, int MODE, int RB, int CB, bool ALL>
 static void launch_mfma_u(const Phase& ph, const Bases& b, T alpha, T beta, hipStream_t s)
 {
     const MfGrid gr{(ph.maxMTile + 16 * RB - 1) / (16 * RB), (ph.maxKTile + 16 * CB - 1) / (16 * CB)};
     const int per = gr.ur * gr.uc;
     if (!ph.segSrc.empty()) {
-        const int64_t grid = S == 4 ? (int64_t)ph.segBlocks1 * per
-                           : per == 4 ? ph.segBlocks1 : per == 2 ? ph.segBlocks2 : ph.segBlocks4;
-        if (S == 1 && per != 1 && per != 2 && per != 4) throw std::runtime_error("segmented tile units");
+        const int lg = per == 1 ? 0 : per == 2 ? 1 : 2;
+        if (!ALL && per != 1 << lg) throw std::runtime_error("segmented tile units");
+        const int64_t grid = ALL ? (int64_t)ph.segTiles * per : ph.segBlocks[lg];
         if (grid == 0) return;
-        tile_mfma_seg_kernel<T, MODE, RB, CB, S><<<(unsigned)grid, 256, 0, s>>>(
-            b, static_cast<const TileSeg*>(ph.dSegs), (int)ph.segSrc.size(), gr, alpha, beta);
+        tile_mfma_seg_kernel<T, MODE, RB, CB, ALL><<<(unsigned)grid, 256, 0, s>>>(
+            b, static_cast<const TileSeg*>(ph.dSegs), (int)ph.segSrc.size(), gr, lg, alpha, beta);
         return;
     }
-    const int64_t units = (int64_t)ph.tiles.size() * per, grid = S == 4 ? units : (units + 3) / 4;
-    tile_mfma_kernel<T, MODE, RB, CB, S><<<(unsigned)grid, 256, 0, s>>>(
+    const int64_t n = (int64_t)ph.tiles.size(), lng = ALL ? n : ph.nLong;
+    const int64_t grid = lng * per + ((n - lng) * per + 3) / 4;
+    tile_mfma_kernel<T, MODE, RB, CB, ALL><<<(unsigned)grid, 256, 0, s>>>(
         b, static_cast<const Tile*>(ph.dTiles), static_cast<const Contrib*>(ph.dContribs),
-        static_cast<const int64_t*>(ph.dGather), (int)ph.tiles.size(), gr, alpha, beta);
+        static_cast<const int64_t*>(ph.dGather), (int)n, ph.nLong, gr, alpha, beta);
 }
+
+// Units of the launch: 32 x 32 entries (a row or column block less where the
+// tiles are narrower), one per wave but for the long tiles, where the phase
+// has tiles enough to give each of the 1,024 SIMDs two such waves, else 16 x
+// 16 split over the four waves of a workgroup: such a phase is one tile's
+// latency, and the split cuts it (direct inversion of 64^2 at rank 8, 940
+// launches of at most a few hundred tiles: 15.4 -> 10.6 ms; of 256^2 at rank
+// 16 with its refinement: 648 -> 500 ms).
+constexpr int64_t kMfmaWaves = 2048;
 
 template <typename T, int MODE>
 static void launch_mfma(const Phase& ph, const Bases& b, T alpha, T beta, hipStream_t s)
 {
-    const int64_t n = ph.segSrc.empty() ? (int64_t)ph.tiles.size() : ph.segBlocks1;
-    const MfShape u = mf_shape(n, ph.maxMTile, ph.maxKTile);
-    if (u.s == 4) launch_mfma_u<T, MODE, 1, 1, 4>(ph, b, alpha, beta, s);
-    else if (u.rb == 1 && u.cb == 1) launch_mfma_u<T, MODE, 1, 1, 1>(ph, b, alpha, beta, s);
-    else if (u.rb == 1) launch_mfma_u<T, MODE, 1, 2, 1>(ph, b, alpha, beta, s);
-    else if (u.cb == 1) launch_mfma_u<T, MODE, 2, 1, 1>(ph, b, alpha, beta, s);
-    else launch_mfma_u<T, MODE, 2, 2, 1>(ph, b, alpha, beta, s);
+    const int64_t n = ph.segSrc.empty() ? (int64_t)ph.tiles.size() : ph.segTiles;
+    const int rb = ph.maxMTile <= 16 ? 1 : 2, cb = ph.maxKTile <= 16 ? 1 : 2;
+    const int64_t units = n * ((ph.maxMTile + 16 * rb - 1) / (16 * rb)) * ((ph.maxKTile + 16 * cb - 1) / (16 * cb));
+    if (units < kMfmaWaves) launch_mfma_u<T, MODE, 1, 1, true>(ph, b, alpha, beta, s);
+    else if (rb == 1 && cb == 1) launch_mfma_u<T, MODE, 1, 1, false>(ph, b, alpha, beta, s);
+    else if (rb == 1) launch_mfma_u<T, MODE, 1, 2, false>(ph, b, alpha, beta, s);
+    else if (cb == 1) launch_mfma_u<T, MODE, 2, 1, false>(ph, b, alpha, beta, s);
+    else launch_mfma_u<T, MODE, 2, 2, false>(ph, b, alpha, beta, s);
 }
 
 // Segmented launches of a merged phase (its members' segment table).
@@ -796,7 +782,7 @@ template <typename T, int MR>
 static void launch_tile_seg_mr(const Phase& ph, const Bases& b, T alpha, T beta, hipStream_t s)
 {
     constexpr int TM = MR == 64 ? 4 : 1;
-    const int grid = ph.segBlocks1;
+    const int grid = ph.segTiles;
     const int nseg = (int)ph.segSrc.size();
     const TileSeg* sg = static_cast<const TileSeg*>(ph.dSegs);
     const int kmax = ph.maxKTile;

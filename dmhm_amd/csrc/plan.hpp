@@ -118,15 +118,17 @@ enum PhaseKind { PH_TILE, PH_QR, PH_SVD, PH_RNG, PH_SCALE_C, PH_MV_ZERO, PH_MV_P
 // One member's share of a merged tile phase that is not copied: the member
 // plan's tile, contribution and gather arrays (device) and the shifts of its slots
 // (elements, rank indices; the workspace slot is shifted to the member's
-// workspace region). first1 / first2 / first4: the member's first workgroup
-// when a workgroup takes one / two / four tiles.
+// workspace region). first: the member's first tile among all members';
+// firstUnit[i]: its first workgroup in an MFMA launch with 1 << i units per
+// tile, the first nLong tiles taking a workgroup per unit, the others a
+// quarter.
 struct TileSeg {
     const Tile* tiles;
     const Contrib* cs;
     const int64_t* gtab;
     int64_t val[NUM_SLOTS];
     int64_t rank[NUM_SLOTS];
-    int count, first1, first2, first4;
+    int count, nLong, first, firstUnit[3];
 };
 
 struct Phase {
@@ -147,7 +149,8 @@ struct Phase {
     struct SegSrc { const Phase* src; int64_t val[NUM_SLOTS]; int64_t rank[NUM_SLOTS]; };
     std::vector<SegSrc> segSrc;
     void* dSegs = nullptr;
-    int segBlocks1 = 0, segBlocks2 = 0, segBlocks4 = 0;   // workgroups of a segmented launch (1 / 2 / 4 tiles each)
+    int segTiles = 0, segBlocks[3] = {0, 0, 0};   // tiles of a segmented phase, workgroups of its MFMA launch
+    int nLong = 0;          // leading tiles whose units are split over a workgroup (order_tiles)
     int mvK = 0, ldx = 0, ldy = 0;
     void* dAux = nullptr;
     int qrK = 0;            // panel width of the QR phase
@@ -186,6 +189,13 @@ struct Plan {
     void release();
     ~Plan() { release(); }
 };
+
+// Orders a tile phase for launching: first the long tiles (Phase::nLong of
+// them), those with more inner chunks than half of what each wave would do if
+// the phase were spread evenly over the chip, whose units are split over a
+// workgroup; then the others by classes of descending chunk count (powers of
+// four), each in the order they were built.
+void order_tiles(Phase& ph);
 
 // Builds the phases. Contributions are collected per tile and sorted at
 // finalize so that each tile owns a contiguous contribution range.
