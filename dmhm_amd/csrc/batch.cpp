@@ -254,7 +254,7 @@ static Plan* merged_matvec(const Arena& H, const std::vector<int64_t>& vecBase, 
     }
     build_parallel(cls.size(), [&](size_t k) {
         const int n = cls[k].h->geo().n;
-        cls[k].plan.reset(Planner(cls[k].h->geo()).matvecStream(*cls[k].h->lay, 1, n, n));
+        cls[k].plan.reset(Planner(cls[k].h->geo()).matvecStream(*cls[k].h->lay, false, 1, n, n));
     });
     std::vector<PlanPart> parts(M);
     for (size_t m = 0; m < M; ++m) {

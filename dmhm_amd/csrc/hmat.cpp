@@ -228,7 +228,7 @@ void run_phase(Phase& ph, const Bases& b, T alpha, T beta, TruncPolicy pol, uint
     case PH_QR: launch_qr_phase<T>(ph, b, s); break;
     case PH_SVD: launch_svd_phase<T>(ph, b, pol, s); break;
     case PH_RNG: launch_rng_phase<T>(ph, b, seed, s, g_lib.seedOff); break;
-    case PH_MV_ZERO: case PH_MV_PROJ: case PH_MV_ACC: launch_mv_phase<T>(ph, b, alpha, beta, s); break;
+    case PH_MV_PROJ: case PH_MV_ACC: launch_mv_phase<T>(ph, b, alpha, beta, s); break;
     default: break;
     }
 }
@@ -280,13 +280,13 @@ static void multiply_dense(dmhm_hmat_s* h, bool trans, double alpha, const void*
                            double beta, void* Y, int ldy)
 {
     GeoCtx& gc = *h->gc;
-    const bool stream = !trans && k <= 8;
+    const bool stream = k <= 8;
     const std::string key = std::string(stream ? "mvs:" : "mv:") + std::to_string(h->lay->id) + ":" +
                             std::to_string(trans) + ":" + std::to_string(k) + ":" + std::to_string(ldx) + ":" +
                             std::to_string(ldy);
     Plan& p = get_plan(gc, key, [&] {
         Planner pl(gc.geo);
-        return stream ? pl.matvecStream(*h->lay, k, ldx, ldy) : pl.matvec(*h->lay, trans, k, ldx, ldy);
+        return stream ? pl.matvecStream(*h->lay, trans, k, ldx, ldy) : pl.matvec(*h->lay, trans, k, ldx, ldy);
     });
     ensure_ws(p, h->esize());
     Bases b = bases_for(h, nullptr, nullptr, const_cast<void*>(X), Y);
@@ -1381,7 +1381,7 @@ static void profile_matvec(dmhm_hmat_s* h, int k, int reps, double* ms, double* 
                             std::to_string(k) + ":" + std::to_string(n) + ":" + std::to_string(n);
     Plan& p = get_plan(gc, key, [&] {
         Planner pl(gc.geo);
-        return stream ? pl.matvecStream(L, k, n, n) : pl.matvec(L, false, k, n, n);
+        return stream ? pl.matvecStream(L, false, k, n, n) : pl.matvec(L, false, k, n, n);
     });
     const size_t last = p.phases.size() - 1;
     ensure_ws(p, h->esize());
@@ -2445,6 +2445,11 @@ void Plan::upload()
         }
         if (ph.kind == PH_RNG && !ph.rng.empty()) { src = ph.rng.data(); bytes = ph.rng.size() * sizeof(RngTask); }
         if (ph.kind == PH_MV_PROJ && !ph.mvProj.empty()) {
+            // Tallest first: a workgroup's each, then a wave's each.
+            std::stable_sort(ph.mvProj.begin(), ph.mvProj.end(),
+                             [](const MvProjItem& x, const MvProjItem& y) { return x.rows > y.rows; });
+            ph.mvBig = 0;
+            for (const MvProjItem& it : ph.mvProj) ph.mvBig += it.rows > kMvBigRows;
             src = ph.mvProj.data(); bytes = ph.mvProj.size() * sizeof(MvProjItem);
         }
         if (ph.kind == PH_MV_ACC && !ph.mvAtoms.empty()) {

@@ -200,76 +200,77 @@ Plan* Planner::matvec(const Layout& L, bool trans, int k, int ldx, int ldy)
     return plan;
 }
 
-Plan* Planner::matvecStream(const Layout& L, int k, int ldx, int ldy)
+Plan* Planner::matvecStream(const Layout& L, bool trans, int k, int ldx, int ldy)
 {
     const Geometry& g = g_;
     Plan* plan = new Plan();
-    plan->phases.resize(3);
-    Phase& z = plan->phases[0];
-    Phase& pr = plan->phases[1];
-    Phase& ac = plan->phases[2];
-    z.kind = PH_MV_ZERO; pr.kind = PH_MV_PROJ; ac.kind = PH_MV_ACC;
-    for (Phase* ph : {&z, &pr, &ac}) { ph->mvK = k; ph->ldx = ldx; ph->ldy = ldy; }
-    // P per low-rank block: cap x k.
+    plan->phases.resize(2);
+    Phase& pr = plan->phases[0];
+    Phase& ac = plan->phases[1];
+    pr.kind = PH_MV_PROJ; ac.kind = PH_MV_ACC;
+    for (Phase* ph : {&pr, &ac}) { ph->mvK = k; ph->ldx = ldx; ph->ldy = ldy; ph->mvTrans = trans; }
+    // P per low-rank block: cap x k, from V and the source rows (H^T: U and
+    // the target rows).
     std::vector<int64_t> P(g.lrBlocks.size());
-    int64_t pTotal = 0;
-    for (size_t i = 0; i < g.lrBlocks.size(); ++i) {
-        P[i] = wsAlloc((int64_t)L.cap[i] * k);
-        pTotal = wsUsed();
-    }
-    z.zeroOff = 0; z.zeroCount = pTotal;
-    const int chunkAtoms = 8;
     for (size_t i = 0; i < g.lrBlocks.size(); ++i) {
         const int b = g.lrBlocks[i];
-        const Box& sb = g.sbox(b);
-        const int natoms = sb.atomEnd - sb.atomBegin;
-        const bool atomic = natoms > chunkAtoms;
-        for (int a0 = sb.atomBegin; a0 < sb.atomEnd; a0 += chunkAtoms) {
-            const int a1 = std::min(sb.atomEnd, a0 + chunkAtoms);
-            const int r0 = g.atomStart[a0] - sb.off;
-            const int rows = g.atomStart[a1 - 1] + g.atomSize[a1 - 1] - g.atomStart[a0];
-            MvProjItem it{};
-            it.voff = L.vOff[i] + r0; it.ldv = sb.size; it.rows = rows;
-            it.xrow = sb.off + r0; it.poff = P[i]; it.rankIdx = (int)i; it.cap = L.cap[i];
-            it.atomic = atomic ? 1 : 0;
-            pr.mvProj.push_back(it);
-        }
-        plan->flops += 2.0 * sb.size * L.cap[i] * k;
+        const Box& in = trans ? g.tbox(b) : g.sbox(b);
+        P[i] = wsAlloc((int64_t)L.cap[i] * k);
+        MvProjItem it{};
+        it.voff = trans ? L.uOff[i] : L.vOff[i]; it.ldv = in.size; it.rows = in.size;
+        it.xrow = in.off; it.poff = P[i]; it.rankIdx = (int)i; it.cap = L.cap[i];
+        pr.mvProj.push_back(it);
+        plan->flops += 2.0 * in.size * L.cap[i] * k;
     }
-    // Longest chunks first: the grid's tail is then made of short items.
-    std::stable_sort(pr.mvProj.begin(), pr.mvProj.end(),
-                     [](const MvProjItem& a, const MvProjItem& b) { return a.rows > b.rows; });
-    // Contributions per output atom.
-    std::vector<std::vector<MvContrib>> per(g.atomStart.size());
+    // Records per output atom.
+    std::vector<std::vector<MvContrib>> per(g.atomStart.size()), dense(g.atomStart.size());
     for (int b : g.leaves) {
         const Block& B = g.blocks[b];
-        const Box& tb = g.tbox(b);
-        const Box& sb = g.sbox(b);
-        for (int a = tb.atomBegin; a < tb.atomEnd; ++a) {
-            const int ra = g.atomStart[a] - tb.off;
+        const Box& out = trans ? g.sbox(b) : g.tbox(b);
+        const Box& in = trans ? g.tbox(b) : g.sbox(b);
+        for (int a = out.atomBegin; a < out.atomEnd; ++a) {
+            const int ra = g.atomStart[a] - out.off;
             MvContrib c{};
             if (B.type == BT_DENSE) {
-                c.kind = 0; c.loff = L.denseOff[B.denseIndex] + ra; c.ld = tb.size;
-                c.q = sb.size; c.rankIdx = -1; c.roff = sb.off; c.ldr = ldx;
-                plan->flops += 2.0 * g.atomSize[a] * sb.size * k;
+                c.kind = 0; c.rankIdx = -1; c.ldr = ldx;
+                plan->flops += 2.0 * g.atomSize[a] * in.size * k;
+                if (trans) {
+                    c.loff = L.denseOff[B.denseIndex] + (int64_t)ra * in.size; c.ld = in.size;
+                    c.q = g.atomSize[a]; c.roff = in.off;
+                    dense[a].push_back(c);
+                    continue;
+                }
+                for (int p = 0; p < in.size; p += 16) {
+                    c.loff = L.denseOff[B.denseIndex] + ra + (int64_t)p * out.size; c.ld = out.size;
+                    c.q = std::min(16, in.size - p); c.roff = in.off + p;
+                    per[a].push_back(c);
+                }
             } else {
-                c.kind = 1; c.loff = L.uOff[B.lrIndex] + ra; c.ld = tb.size;
-                c.q = L.cap[B.lrIndex]; c.rankIdx = B.lrIndex; c.roff = P[B.lrIndex]; c.ldr = L.cap[B.lrIndex];
-                plan->flops += 2.0 * g.atomSize[a] * L.cap[B.lrIndex] * k;
+                const int li = B.lrIndex;
+                c.kind = 1; c.rankIdx = li; c.ldr = L.cap[li]; c.ld = out.size;
+                for (int p = 0; p < L.cap[li]; p += 16) {
+                    c.loff = (trans ? L.vOff[li] : L.uOff[li]) + ra + (int64_t)p * out.size;
+                    c.q = std::min(16, L.cap[li] - p); c.p0 = p; c.roff = P[li] + p;
+                    per[a].push_back(c);
+                }
+                plan->flops += 2.0 * g.atomSize[a] * L.cap[li] * k;
             }
-            per[a].push_back(c);
         }
     }
-    // Atoms with the most contributions first (same tail argument).
+    // Atoms with the most work first: the grid's tail is then made of short ones.
     std::vector<int> order(per.size());
     for (size_t a = 0; a < per.size(); ++a) order[a] = (int)a;
-    std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return per[x].size() > per[y].size(); });
+    std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
+        return per[x].size() + 4 * dense[x].size() > per[y].size() + 4 * dense[y].size();
+    });
     for (int a : order) {
         MvAtom at{};
         at.yrow = g.atomStart[a]; at.m = g.atomSize[a];
         at.cb = (int)ac.mvContribs.size();
         ac.mvContribs.insert(ac.mvContribs.end(), per[a].begin(), per[a].end());
-        at.ce = (int)ac.mvContribs.size();
+        at.ce = at.db = (int)ac.mvContribs.size();
+        ac.mvContribs.insert(ac.mvContribs.end(), dense[a].begin(), dense[a].end());
+        at.de = (int)ac.mvContribs.size();
         ac.mvAtoms.push_back(at);
     }
     plan->wsElems = wsUsed();
@@ -1036,7 +1037,7 @@ Plan* merge_plans(const std::vector<PlanPart>& parts, bool segmentTiles)
         out->phases.emplace_back();
         Phase& m = out->phases.back();
         m.kind = lp.kind;
-        m.mvK = lp.mvK; m.ldx = lp.ldx; m.ldy = lp.ldy;
+        m.mvK = lp.mvK; m.ldx = lp.ldx; m.ldy = lp.ldy; m.mvTrans = lp.mvTrans;
         m.role = lp.role;
         bool first = true;
         for (size_t i = 0; i < np; ++i) {
@@ -1099,16 +1100,8 @@ Plan* merge_plans(const std::vector<PlanPart>& parts, bool segmentTiles)
                     m.rng.push_back(t);
                 }
                 break;
-            case PH_MV_ZERO:
-                // A streaming product zeroes the front of its workspace (its
-                // projections); the merged phase zeroes the whole workspace.
-                if (ph.zeroOff != 0 || ph.zeroCount > parts[i].plan->wsElems)
-                    throw std::logic_error("merged zero range is not inside the part's workspace");
-                m.zeroOff = 0;
-                m.zeroCount = -1;
-                break;
             case PH_MV_PROJ:
-                if (!first && (ph.mvK != m.mvK || (ph.mvK > 1 && (ph.ldx != m.ldx || ph.ldy != m.ldy))))
+                if (!first && (ph.mvK != m.mvK || ph.mvTrans != m.mvTrans || (ph.mvK > 1 && (ph.ldx != m.ldx || ph.ldy != m.ldy))))
                     throw std::logic_error("merged streaming products of different shapes");
                 for (MvProjItem it : ph.mvProj) {
                     it.voff += vsh(i, SLOT_A);
@@ -1119,12 +1112,12 @@ Plan* merge_plans(const std::vector<PlanPart>& parts, bool segmentTiles)
                 }
                 break;
             case PH_MV_ACC: {
-                if (!first && (ph.mvK != m.mvK || (ph.mvK > 1 && (ph.ldx != m.ldx || ph.ldy != m.ldy))))
+                if (!first && (ph.mvK != m.mvK || ph.mvTrans != m.mvTrans || (ph.mvK > 1 && (ph.ldx != m.ldx || ph.ldy != m.ldy))))
                     throw std::logic_error("merged streaming products of different shapes");
                 const int cbase = (int)m.mvContribs.size();
                 for (MvAtom a : ph.mvAtoms) {
                     a.yrow += vsh(i, SLOT_Y);
-                    a.cb += cbase; a.ce += cbase;
+                    a.cb += cbase; a.ce += cbase; a.db += cbase; a.de += cbase;
                     m.mvAtoms.push_back(a);
                 }
                 for (MvContrib c : ph.mvContribs) {
@@ -1142,7 +1135,6 @@ Plan* merge_plans(const std::vector<PlanPart>& parts, bool segmentTiles)
         }
     }
     for (auto& ph : out->phases) {
-        if (ph.kind == PH_MV_ZERO) ph.zeroCount = out->wsElems;
         out->tileCount += ph.tiles.size();
         out->contribCount += ph.contribs.size();
         for (const auto& sg : ph.segSrc) {

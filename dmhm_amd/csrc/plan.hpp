@@ -86,34 +86,35 @@ struct RngTask {
     uint64_t stream;        // stream id mixed into the counter
 };
 
-// Streaming H*X for few right-hand sides (HBM-bound): projections
-// P = V^T X per (low-rank block, row chunk) by one wave each, then one
-// workgroup per output row atom summing dense-leaf and U*P contributions.
+// Streaming H*X and H^T*X for few right-hand sides (HBM-bound): projections
+// P = V^T X per low-rank block (U^T X for H^T), then one workgroup per output
+// row atom summing its records of at most 16 columns of dense leaves and of U
+// (V). For H^T the dense leaves are separate records [db, de), one per leaf.
 struct MvProjItem {
-    int64_t voff;           // slot A offset of V(row0, 0) (ld = ldv)
-    int64_t xrow;           // first X row of the chunk
+    int64_t voff;           // slot A offset of the factor (ld = ldv)
+    int64_t xrow;           // first X row
     int64_t poff;           // workspace offset of P (cap x k, ld cap)
-    int32_t ldv, rows;      // V leading dimension, rows in this chunk
+    int32_t ldv, rows;
     int32_t rankIdx, cap;
-    int32_t atomic;         // several chunks share P: accumulate atomically
-    int32_t pad;
 };
+// Rows from which a projection takes a workgroup instead of a wave.
+constexpr int kMvBigRows = 512;
 struct MvAtom {
     int64_t yrow;
-    int32_t m, cb, ce, pad;
+    int32_t m, cb, ce, db, de, pad;
 };
 struct MvContrib {
-    int64_t loff;           // slot A offset of the first row of L (dense leaf or U)
+    int64_t loff;           // slot A offset of L's first row and column (H^T dense leaf: first column)
     int64_t roff;           // X row offset (kind 0) or workspace offset of P (kind 1)
-    int32_t ld;             // leading dimension of L
-    int32_t q;              // inner dimension (static) ...
-    int32_t rankIdx;        // ... or the block's rank (kind 1)
-    int32_t kind;           // 0: dense leaf times X rows, 1: U rows times P
+    int32_t ld;             // leading dimension of L (H^T dense leaf: also its rows)
+    int32_t q;              // columns (at most 16), for kind 1 those below the block's rank:
+    int32_t rankIdx;        // min(q, rank - p0)
+    int32_t kind;           // 0: dense leaf times X rows, 1: factor rows times P
     int32_t ldr;            // P leading dimension (cap) for kind 1
-    int32_t pad;
+    int32_t p0;             // first column within the factor (kind 1)
 };
 
-enum PhaseKind { PH_TILE, PH_QR, PH_SVD, PH_RNG, PH_SCALE_C, PH_MV_ZERO, PH_MV_PROJ, PH_MV_ACC };
+enum PhaseKind { PH_TILE, PH_QR, PH_SVD, PH_RNG, PH_SCALE_C, PH_MV_PROJ, PH_MV_ACC };
 
 // One member's share of a merged tile phase that is not copied: the member
 // plan's tile, contribution and gather arrays (device) and the shifts of its slots
@@ -141,7 +142,6 @@ struct Phase {
     std::vector<MvProjItem> mvProj;
     std::vector<MvAtom> mvAtoms;
     std::vector<MvContrib> mvContribs;
-    int64_t zeroOff = 0, zeroCount = 0;   // PH_MV_ZERO range in the workspace
     std::vector<int64_t> gtab;            // PH_TILE: column offsets of gathered right operands
     // PH_TILE of a merged plan built without copying: per member, the source
     // phase (host, uploaded with its plan) and the member's shifts; the
@@ -152,6 +152,8 @@ struct Phase {
     int segTiles = 0, segBlocks[3] = {0, 0, 0};   // tiles of a segmented phase, workgroups of its MFMA launch
     int nLong = 0;          // leading tiles whose units are split over a workgroup (order_tiles)
     int mvK = 0, ldx = 0, ldy = 0;
+    bool mvTrans = false;
+    int mvBig = 0;          // leading projections of more than kMvBigRows rows (set by upload)
     void* dAux = nullptr;
     int qrK = 0;            // panel width of the QR phase
     int qrClassEnd[4] = {0, 0, 0, 0};   // QR tasks sorted by panel class at upload (see launch_qr_phase)
@@ -275,8 +277,8 @@ public:
 
     // Y (n x k, ld ldy) := alpha op(H) X + beta Y, H in SLOT_A with layout L.
     Plan* matvec(const Layout& L, bool trans, int k, int ldx, int ldy);
-    // Streaming form of the non-transposed product for k <= 8.
-    Plan* matvecStream(const Layout& L, int k, int ldx, int ldy);
+    // Streaming form for k <= 8.
+    Plan* matvecStream(const Layout& L, bool trans, int k, int ldx, int ldy);
 
     // C := alpha A B with randomized sum-sketch compression of every admissible
     // block (sketch width kS = maxRank + oversample), A/B/C layouts given.
