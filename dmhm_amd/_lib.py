@@ -89,6 +89,7 @@ SIGNATURES = {
                                              ctypes.c_int, _hp]),
     "dmhm_hmat_destroy": (ctypes.c_int, [_h]),
     "dmhm_hmat_info": (ctypes.c_int, [_h, ctypes.POINTER(Info)]),
+    "dmhm_hmat_shape": (ctypes.c_int, [_h, ctypes.POINTER(ctypes.c_int), ctypes.POINTER(ctypes.c_int)]),
     "dmhm_hmat_block_counts": (ctypes.c_int, [_h, _llp, _llp, ctypes.c_int]),
     "dmhm_hmat_set_to_random": (ctypes.c_int, [_h, ctypes.c_uint64]),
     "dmhm_hmat_multiply_dense": (ctypes.c_int, [_h, ctypes.c_char, ctypes.c_double, ctypes.c_void_p,

@@ -23,6 +23,59 @@ static thread_local std::string g_lastError;
 
 Library g_lib;
 
+DevicePool& device_pool()
+{
+    // Never destroyed: matrices may outlive static destruction.
+    static DevicePool* p = new DevicePool();
+    return *p;
+}
+
+void* DevicePool::get(size_t bytes)
+{
+    bytes = (std::max<size_t>(bytes, 1) + 255) & ~size_t(255);
+    std::lock_guard<std::mutex> lk(mu_);
+    auto it = held_.lower_bound(bytes);
+    if (it != held_.end() && it->first - bytes <= bytes / 4) {
+        void* p = it->second;
+        holding_ -= it->first;
+        held_.erase(it);
+        return p;
+    }
+    void* p = nullptr;
+    hipError_t e = hipMalloc(&p, bytes);
+    if (e == hipErrorOutOfMemory && !held_.empty()) {
+        (void)hipGetLastError();
+        for (auto& h : held_) { size_.erase(h.second); (void)hipFree(h.second); }
+        held_.clear();
+        holding_ = 0;
+        e = hipMalloc(&p, bytes);
+    }
+    HIPCHECK(e);
+    size_[p] = bytes;
+    return p;
+}
+
+void DevicePool::put(void* p)
+{
+    std::lock_guard<std::mutex> lk(mu_);
+    const size_t bytes = size_.at(p);
+    if (g_lib.ready && bytes <= kBlockMax && holding_ + bytes <= kHoldMax) {
+        held_.emplace(bytes, p);
+        holding_ += bytes;
+        return;
+    }
+    size_.erase(p);
+    (void)hipFree(p);
+}
+
+void DevicePool::trim()
+{
+    std::lock_guard<std::mutex> lk(mu_);
+    for (auto& h : held_) { size_.erase(h.second); (void)hipFree(h.second); }
+    held_.clear();
+    holding_ = 0;
+}
+
 // Copies on the library stream and waits for them: the stream is created
 // non-blocking, so a plain hipMemcpy (null stream) would not be ordered after
 // work already queued on it (for example the zero fill of a new matrix).
@@ -140,10 +193,10 @@ dmhm_hmat_s* alloc_hmat(std::shared_ptr<GeoCtx> gc, std::shared_ptr<Layout> lay,
     std::unique_ptr<dmhm_hmat_s> h(new dmhm_hmat_s());
     h->gc = gc; h->lay = lay; h->prec = prec; h->maxRank = maxRank;
     const size_t bytes = std::max<size_t>(lay->totalElems() * h->esize(), 256);
-    HIPCHECK(hipMalloc(&h->vals, bytes));
+    h->vals = device_pool().get(bytes);
     HIPCHECK(hipMemsetAsync(h->vals, 0, bytes, g_lib.stream));
     const size_t rb = std::max<size_t>(lay->nLowRank() * sizeof(int), 4);
-    HIPCHECK(hipMalloc((void**)&h->ranks, rb));
+    h->ranks = static_cast<int*>(device_pool().get(rb));
     HIPCHECK(hipMemsetAsync(h->ranks, 0, rb, g_lib.stream));
     return h.release();
 }
@@ -1557,6 +1610,7 @@ int dmhm_finalize(void)
         (void)hipHostFree(g_lib.hReadback);
         (void)hipStreamDestroy(g_lib.stream);
         g_lib.ready = false;
+        device_pool().trim();
     });
 }
 
@@ -1673,6 +1727,15 @@ int dmhm_hmat_destroy(dmhm_hmat h)
         if (!h) return;
         if (g_lib.ready) HIPCHECK(hipStreamSynchronize(g_lib.stream));
         delete h;
+    });
+}
+
+int dmhm_hmat_shape(dmhm_hmat h, int* n, int* precision)
+{
+    return guard([&] {
+        if (!h || !n || !precision) throw Error(DMHM_EINVAL, "null pointer");
+        *n = h->geo().n;
+        *precision = h->prec;
     });
 }
 

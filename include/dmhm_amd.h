@@ -114,8 +114,11 @@ typedef struct {
     long long sumRank;           /* sum of current low-rank block ranks  */
     int maxBlockRank;
 } dmhm_info;
-/* Height/Width/NumLevels/MaxRank/StronglyAdmissible (hmat2d.hpp:96-104). */
+/* Height/Width/NumLevels/MaxRank/StronglyAdmissible (hmat2d.hpp:96-104). Reads
+ * the ranks back from the device. */
 int dmhm_hmat_info(dmhm_hmat h, dmhm_info* info);
+/* Height and precision alone, without touching the device. */
+int dmhm_hmat_shape(dmhm_hmat h, int* n, int* precision);
 /* Dense/low-rank counts per level (levels <= maxLevels). */
 int dmhm_hmat_block_counts(dmhm_hmat h, long long* dense, long long* lowRank, int maxLevels);
 

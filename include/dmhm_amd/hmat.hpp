@@ -186,8 +186,13 @@ public:
 
     void SetToRandom() { detail::check(dmhm_hmat_set_to_random(need(), next_seed())); }
 
-    int Height() const { return info().n; }
-    int Width() const { return info().n; }
+    int Height() const
+    {
+        int n = 0, precision = 0;
+        detail::check(dmhm_hmat_shape(need(), &n, &precision));
+        return n;
+    }
+    int Width() const { return Height(); }
     int NumLevels() const { return info().numLevels; }
     int MaxRank() const { return info().maxRank; }
     int SourceOffset() const { return 0; }
