@@ -1,6 +1,7 @@
 // gfx950 tile GEMM engine: grouped output-owned small GEMMs (H*X, sub-H
 // products, projections, dense-leaf accumulation, factor formation).
 #include <climits>
+#include <cstddef>
 #include "kcommon.hpp"
 
 namespace dmhm {
@@ -418,6 +419,29 @@ struct MfFrag {
     int qc;
 };
 
+// Records as whole vectors: loads by field (single bytes among them) are
+// issued one after another as their fields are used.
+typedef uint32_t mf_u2 __attribute__((ext_vector_type(2), aligned(8)));
+typedef uint32_t mf_u4 __attribute__((ext_vector_type(4), aligned(8)));
+static_assert(sizeof(Tile) == 56 && offsetof(Tile, k) == 16 && offsetof(Tile, koff) == 32 &&
+              offsetof(Tile, gather) == 48 && offsetof(Tile, slot) == 44, "tile record layout");
+static_assert(sizeof(Contrib) == 40 && offsetof(Contrib, ldl) == 16 && offsetof(Contrib, lslot) == 32 &&
+              offsetof(Contrib, flags) == 35, "contribution record layout");
+__device__ __forceinline__ int64_t mf_i64(uint32_t lo, uint32_t hi) { return (int64_t)((uint64_t)hi << 32 | lo); }
+__device__ __forceinline__ Tile mf_tile(const Tile* __restrict__ p)
+{
+    const mf_u4* v = reinterpret_cast<const mf_u4*>(p);
+    const mf_u4 a = v[0], b = v[1], c = v[2];
+    Tile t;
+    t.gather = (int)reinterpret_cast<const mf_u2*>(p)[6][0];
+    t.off = mf_i64(a[0], a[1]); t.ld = (int)a[2]; t.m = (int)a[3];
+    t.k = (int)b[0]; t.mrank = (int)b[1]; t.krank = (int)b[2]; t.moff = (int)b[3];
+    t.koff = (int)c[0]; t.cb = (int)c[1]; t.ce = (int)c[2];
+    t.slot = (uint8_t)c[3]; t.mslot = (uint8_t)(c[3] >> 8); t.kslot = (uint8_t)(c[3] >> 16);
+    t.flags = (uint8_t)(c[3] >> 24);
+    return t;
+}
+
 // One unit of a tile: walks the tile's contributions 64 at a time, one record
 // per lane, and within them by form (which operands have the inner dimension
 // contiguous; whole chunks, then the remainders of inner dimensions that 16
@@ -436,8 +460,8 @@ struct MfUnit {
     int64_t gcol[CB];           // offsets of the unit's columns in gathered right operands
     // lane records
     int64_t dl, dr;
-    int dldl, dldr, dq;
-    uint32_t dmeta;
+    int dldl, dldr, dq, dqrank;
+    uint32_t dmeta;             // left, right and rank slot, flags (bytes)
     float dalpha;
     Acc acc[RB][CB];
 
@@ -495,7 +519,7 @@ struct MfUnit {
                     else p = 16 * mine;
                 }
                 const uint32_t meta = __builtin_amdgcn_readlane(dmeta, i);
-                const int fl = (meta >> 16) & 255;
+                const int fl = meta >> 24;
                 const float ca = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(dalpha), i));
                 a = (fl & CF_RUNTIME_ALPHA) ? alpha * T(ca) : (fl & CF_RUNTIME_BETA) ? beta * T(ca) : T(ca);
                 ldl = __builtin_amdgcn_readlane(dldl, i);
@@ -548,7 +572,7 @@ struct MfUnit {
             left &= left - 1;
             const int q = __builtin_amdgcn_readlane(dq, i);
             const uint32_t meta = __builtin_amdgcn_readlane(dmeta, i);
-            const int fl = (meta >> 16) & 255;
+            const int fl = meta >> 24;
             const float ca = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(dalpha), i));
             const int64_t ldl = __builtin_amdgcn_readlane(dldl, i), ldr = __builtin_amdgcn_readlane(dldr, i);
             const bool tL = fl & CF_TRANS_L, tR = fl & CF_TRANS_R;
@@ -580,18 +604,38 @@ struct MfUnit {
         }
     }
 
+    // Issues the loads of the lane's record among the 64 from c0 on.
+    __device__ __forceinline__ void record(const Tile& tl, const Contrib* __restrict__ cs, int c0)
+    {
+        if (tl.cb == tl.ce) return;
+        const Contrib* C = cs + min(c0 + 16 * lk + li, tl.ce - 1);
+        const mf_u4 x = reinterpret_cast<const mf_u4*>(C)[0], y = reinterpret_cast<const mf_u4*>(C)[1];
+        const mf_u2 z = reinterpret_cast<const mf_u2*>(C)[4];
+        dl = mf_i64(x[0], x[1]); dr = mf_i64(x[2], x[3]);
+        dldl = (int)y[0]; dldr = (int)y[1]; dq = (int)y[2]; dqrank = (int)y[3];
+        dmeta = z[0];
+        dalpha = __int_as_float((int)z[1]);
+    }
+
+    // record() has been called for the first 64.
     __device__ __forceinline__ void contributions(const Tile& tl, const Contrib* __restrict__ cs)
     {
         const int lane = 16 * lk + li;
         for (int c0 = tl.cb; c0 < tl.ce; c0 += 64) {
-            const int c = c0 + lane;
-            const bool in = c < tl.ce;
-            const Contrib& C = cs[in ? c : tl.ce - 1];
-            dl = C.loff; dr = C.roff; dldl = C.ldl; dldr = C.ldr; dalpha = C.alpha;
-            dmeta = (uint32_t)C.lslot | (uint32_t)C.rslot << 8 | (uint32_t)C.flags << 16;
-            dq = contrib_q(b, C);
+            if (c0 != tl.cb) record(tl, cs, c0);
+            const bool in = c0 + lane < tl.ce;
+            if (dqrank >= 0) {
+                // The slots that have ranks, picked per lane without a load.
+                const uint32_t sl = (dmeta >> 16) & 255;
+                const int* r = b.rank(SLOT_A);
+                r = sl == SLOT_B ? b.rank(SLOT_B) : r;
+                r = sl == SLOT_C ? b.rank(SLOT_C) : r;
+                r = sl == SLOT_X ? b.rank(SLOT_X) : r;
+                r = sl == SLOT_WIDTH ? b.rank(SLOT_WIDTH) : r;
+                dq = min(dq, r[dqrank]);
+            }
             const bool mine = in && dq > 0 && (S == 1 || byChunk || (lane & (S - 1)) == w);
-            const bool pl = C.flags & CF_TRANS_L, pr = !(C.flags & CF_TRANS_R);
+            const bool pl = dmeta >> 24 & CF_TRANS_L, pr = !(dmeta >> 24 & CF_TRANS_R);
             const bool any = (pl && !pr) || (RB > 1 && !pl && m < 2) || (CB > 1 && !pr && n < 2);
             const bool whole = mine && !any && dq >= 16, rest = mine && !any && (dq & 15);
             run<false, true, false>(__ballot(whole && !pl && pr));
@@ -613,13 +657,17 @@ __device__ __forceinline__ void mfma_body(const BV& b, const Tile& tl, const Con
 {
     static_assert(MODE == 0 || sizeof(T) == 4, "the BF16 mode reads FP32 operands");
     static_assert(S == 1 || S == 4, "one wave or the four waves of a workgroup per unit");
+    const int row0 = ur * 16 * RB, col0 = uc * 16 * CB;
+    const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+    MfUnit<T, MODE, RB, CB, S, BV> u{b, alpha, beta, w, li, lk, row0, col0, 0, 0, S > 1 && tl.ce - tl.cb < S, 0};
+    // The first records' loads are in flight while the ranks are read.
+    u.record(tl, cs, tl.cb);
     int m = tl.m, n = tl.k;
     if (tl.mrank >= 0) m = min(m, max(0, b.rank(tl.mslot)[tl.mrank] - tl.moff));
     if (tl.krank >= 0) n = min(n, max(0, b.rank(tl.kslot)[tl.krank] - tl.koff));
-    const int row0 = ur * 16 * RB, col0 = uc * 16 * CB;
     if (m <= row0 || n <= col0) return;         // uniform over the waves that share the unit
-    const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
-    MfUnit<T, MODE, RB, CB, S, BV> u{b, alpha, beta, w, li, lk, row0, col0, m, n, S > 1 && tl.ce - tl.cb < S, 0};
+    u.m = m;
+    u.n = n;
 #pragma unroll
     for (int cb = 0; cb < CB; ++cb)
         u.gcol[cb] = tl.gather >= 0 ? gtab[tl.gather + min(col0 + mf_row<CB>(cb, li), n - 1)] : 0;
@@ -702,11 +750,11 @@ __device__ __forceinline__ void mfma_unit(const BV& b, const Tile* __restrict__ 
     if (ALL || g < nLong * per) {
         const int id = g / per, sub = g - id * per;
         if (id >= ntiles) return;
-        mfma_body<T, MODE, RB, CB, 4>(b, tiles[id], cs, gtab, sub / gr.uc, sub % gr.uc, w, alpha, beta);
+        mfma_body<T, MODE, RB, CB, 4>(b, mf_tile(tiles + id), cs, gtab, sub / gr.uc, sub % gr.uc, w, alpha, beta);
     } else {
         const int u = (g - nLong * per) * 4 + w, at = u / per, id = nLong + at, sub = u - at * per;
         if (id >= ntiles) return;
-        mfma_body<T, MODE, RB, CB, 1>(b, tiles[id], cs, gtab, sub / gr.uc, sub % gr.uc, w, alpha, beta);
+        mfma_body<T, MODE, RB, CB, 1>(b, mf_tile(tiles + id), cs, gtab, sub / gr.uc, sub % gr.uc, w, alpha, beta);
     }
 }
 
