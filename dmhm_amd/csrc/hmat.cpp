@@ -214,11 +214,13 @@ static Bases bases_for(dmhm_hmat_s* A, dmhm_hmat_s* B, dmhm_hmat_s* C, void* X, 
 
 // Tile-engine candidates per execution slot (FP64, FP32, FP32 with BF16
 // operands allowed); FP32 engines stay candidates in the BF16 slot, since a
-// more precise engine that is also faster is the better choice there.
-static const int kTuneCands[3][3] = {{TILE_LDS, TILE_MFMA, -1},
-                                     {TILE_LDS, TILE_MFMA, -1},
-                                     {TILE_LDS, TILE_MFMA, TILE_MFMA_BF16}};
-static const int kTuneCount[3] = {2, 2, 3};
+// more precise engine that is also faster is the better choice there. The LDS
+// engine runs only when it is forced: timed against it per phase, the MFMA
+// engine was the faster one (256^2 inversion 435.7 ms with both as candidates,
+// 434.3 with MFMA alone; 64^2 9.84 and 9.75 ms; products equal), and a phase
+// with one candidate is not timed.
+static const int kTuneCands[3][2] = {{TILE_MFMA, -1}, {TILE_MFMA, -1}, {TILE_MFMA, TILE_MFMA_BF16}};
+static const int kTuneCount[3] = {1, 1, 2};
 
 // Launches a TILE phase with its engine. Autotuning (no engine forced): the
 // first run of a phase in a slot is a warm-up with the first candidate (its
@@ -245,6 +247,10 @@ static void run_tile_phase(Phase& ph, const Bases& b, T alpha, T beta)
             if (sg.src != tp) { tp = &ph; break; }
     }
     const float per = ph.segSrc.empty() || tp == &ph ? 1.0f : (float)ph.segSrc.size();
+    if (kTuneCount[slot] == 1) {
+        launch_tile_phase<T>(ph, b, alpha, beta, s, kTuneCands[slot][0]);
+        return;
+    }
     Phase::Tune& t = tp->tune[slot];
     if (t.choice >= 0) {
         launch_tile_phase<T>(ph, b, alpha, beta, s, t.choice);

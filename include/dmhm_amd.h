@@ -406,9 +406,9 @@ int dmhm_hmat_rank_features(dmhm_hmat A, float* out, int count);
 int dmhm_last_product_stats(long long* out);
 
 /* Tile engine of the grouped small GEMMs (measurement and test support, no
- * counterpart in the reference): -1 autotunes every tile phase (each phase
- * times the candidate engines on its first runs and keeps the fastest; the
- * default), 0 the LDS-staged vector-FMA kernel, 1 the MFMA kernel, 3 the
+ * counterpart in the reference): -1 the engine of each phase's kind (the
+ * MFMA kernel; where BF16 is allowed, each phase times it against the BF16 one
+ * on its first runs and keeps the faster; the default), 0 the LDS-staged vector-FMA kernel, 1 the MFMA kernel, 3 the
  * MFMA kernel with BF16 operands where BF16 is allowed (the FP32 steps of a
  * mixed Schulz inversion); 2 and 4 select the same kernels as 1 and 3.
  * DMHM_TILE_ENGINE=auto|lds|mfma|mfma_pf|bf16|bf16_pf sets it at dmhm_init. */
