@@ -214,10 +214,13 @@ __global__ void __launch_bounds__(64 * NWV) qr_split_kernel(Bases b, const QrTas
             const double xn2 = wave_sum_uniform(s);
             const double alpha = bcast(xj, j & 63);
             double t = 0.0, scale = 0.0, beta = alpha;
-            if (xn2 > 0.0 && alpha * alpha + xn2 > kTinyColumn) {
-                beta = -copysign(sqrt(alpha * alpha + xn2), alpha);
-                t = (beta - alpha) / beta;
-                scale = 1.0 / (alpha - beta);
+            const double n2 = fma(alpha, alpha, xn2);
+            if (xn2 > 0.0 && n2 > kTinyColumn) {
+                // beta = -sgn(alpha) |column|, t = (beta - alpha) / beta, scale = 1 / (alpha - beta).
+                const double rs = rsq_nr(n2), nrm = n2 * rs;
+                beta = -copysign(nrm, alpha);
+                t = fma(fabs(alpha), rs, 1.0);
+                scale = copysign(rcp_nr(fabs(alpha) + nrm), alpha);
             }
 #pragma unroll
             for (int r = 0; r < RR; ++r) {

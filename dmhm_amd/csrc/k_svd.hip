@@ -25,18 +25,6 @@ namespace dmhm {
 // reciprocal square roots are the hardware estimates (v_rcp_f64, v_rsq_f64)
 // refined by two Newton steps each: a shorter dependent chain than IEEE
 // division and square root, and c^2 + s^2 = 1 to rounding either way.
-__device__ inline double rcp_nr(double x)
-{
-    double r = __builtin_amdgcn_rcp(x);
-    r = fma(r, fma(-x, r, 1.0), r);
-    return fma(r, fma(-x, r, 1.0), r);
-}
-__device__ inline double rsq_nr(double x)
-{
-    double y = __builtin_amdgcn_rsq(x);
-    y = fma(0.5 * y, fma(-x * y, y, 1.0), y);
-    return fma(0.5 * y, fma(-x * y, y, 1.0), y);
-}
 __device__ inline void jacobi_rotation(double al, double be, double ga, double& cs, double& sn)
 {
     const double d0 = be - al, g0 = 2.0 * ga;

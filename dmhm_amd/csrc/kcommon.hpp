@@ -81,6 +81,22 @@ __device__ inline double bcast(double v, int l)
     return __hiloint2double(hi, lo);
 }
 
+// 1 / x and 1 / sqrt(x) from the hardware estimates (v_rcp_f64, v_rsq_f64) and
+// two Newton steps each: a shorter dependent chain than IEEE division and
+// square root, to rounding.
+__device__ inline double rcp_nr(double x)
+{
+    double r = __builtin_amdgcn_rcp(x);
+    r = fma(r, fma(-x, r, 1.0), r);
+    return fma(r, fma(-x, r, 1.0), r);
+}
+__device__ inline double rsq_nr(double x)
+{
+    double y = __builtin_amdgcn_rsq(x);
+    y = fma(0.5 * y, fma(-x * y, y, 1.0), y);
+    return fma(0.5 * y, fma(-x * y, y, 1.0), y);
+}
+
 template <typename T> struct VecOf;
 template <> struct VecOf<float> { typedef float type __attribute__((ext_vector_type(4))); };
 template <> struct VecOf<double> { typedef double type __attribute__((ext_vector_type(2))); };
