@@ -14,7 +14,7 @@
 //
 // Here three H-matrices of the standard layout share one allocation (the
 // arena): X (the inverse being formed, A above), W (the working copy, B above)
-// and K (copies of the blocks a step overwrites). The recursion needs no
+// and K (copies of the blocks a row scaling overwrites). The recursion needs no
 // copies: inverting the diagonal child c of a node works on W's own block c,
 // which the parent no longer reads once it is inverted. Every step's
 // products are independent (distinct outputs, inputs not written in the
@@ -134,7 +134,7 @@ public:
         auto ch = [&](int i, int j) { return g_.child(b, i, j); };
         // X := 0 on the node (its diagonal children are then written by the
         // recursion; the identity's off-diagonal blocks are zero).
-        ranges({{MX, MX, b}}, true, true);
+        ranges({{MX, MX, b}}, true);
         for (int l = 0; l < nc; ++l) {
             invert(ch(l, l));
             // Row l scaled by the new pivot inverse X_ll; the right operands
@@ -147,31 +147,24 @@ public:
                 cp.push_back({m, ch(l, j)});
                 pr.push_back({ch(l, l), ch(l, j), ch(l, j), MX, MK, m});
             }
-            copies_to_k(cp, true);
+            copies_to_k(cp);
             plan(pr, Planner::HH_PRODUCT, 1.0, 0.0);
             if (l == nc - 1) break;
-            // Elimination below the pivot (update form, C_old from K).
-            cp.clear();
+            // Elimination below the pivot (update form, in place: a plan reads
+            // every C_old before its SVD and formation phases write C).
             pr.clear();
             for (int i = l + 1; i < nc; ++i)
                 for (int j = 0; j < nc; ++j) {
                     const int m = j <= l ? MX : MW;
-                    cp.push_back({m, ch(i, j)});
                     pr.push_back({ch(i, l), ch(l, j), ch(i, j), MW, m, m});
                 }
-            copies_to_k(cp, false);
             plan(pr, Planner::HH_UPDATE, -1.0, 1.0);
         }
         // Back substitution.
         for (int l = nc - 1; l >= 1; --l) {
-            std::vector<std::pair<int, int>> cp;
             std::vector<Prod> pr;
             for (int i = l - 1; i >= 0; --i)
-                for (int j = 0; j < nc; ++j) {
-                    cp.push_back({MX, ch(i, j)});
-                    pr.push_back({ch(i, l), ch(l, j), ch(i, j), MW, MX, MX});
-                }
-            copies_to_k(cp, false);
+                for (int j = 0; j < nc; ++j) pr.push_back({ch(i, l), ch(l, j), ch(i, j), MW, MX, MX});
             plan(pr, Planner::HH_UPDATE, -1.0, 1.0);
         }
     }
@@ -181,8 +174,8 @@ private:
     int64_t rnk(int m) const { return m * P_.memberRanks; }
 
     // Copies (src member -> dst member) or zero fills (dst member) of whole
-    // subtrees: values (the dense pool only if withDense) and ranks.
-    void ranges(const std::vector<std::array<int, 3>>& items, bool fill, bool withDense)
+    // subtrees: values and ranks.
+    void ranges(const std::vector<std::array<int, 3>>& items, bool fill)
     {
         DinvStep st;
         st.kind = DinvStep::RANGES;
@@ -196,7 +189,7 @@ private:
                 P_.ranges.push_back({so + a, dof + a, e - a});
                 st.maxVal = std::max(st.maxVal, e - a);
             };
-            if (withDense) add(s.d0, s.d1);
+            add(s.d0, s.d1);
             add(s.u0, s.u1);
             add(s.v0, s.v1);
         }
@@ -212,11 +205,11 @@ private:
         if (st.nVal + st.nRank > 0) P_.steps.push_back(std::move(st));
     }
 
-    void copies_to_k(const std::vector<std::pair<int, int>>& cp, bool withDense)
+    void copies_to_k(const std::vector<std::pair<int, int>>& cp)
     {
         std::vector<std::array<int, 3>> items;
         for (const auto& c : cp) items.push_back({c.first, MK, c.second});
-        ranges(items, false, withDense);
+        ranges(items, false);
     }
 
     void plan(const std::vector<Prod>& prods, int mode, double alpha, double beta)
@@ -236,7 +229,7 @@ private:
             part.val[SLOT_A] = val(p.mA); part.rank[SLOT_A] = rnk(p.mA);
             part.val[SLOT_B] = val(p.mB); part.rank[SLOT_B] = rnk(p.mB);
             part.val[SLOT_C] = val(p.mC); part.rank[SLOT_C] = rnk(p.mC);
-            part.val[SLOT_X] = val(MK); part.rank[SLOT_X] = rnk(MK);
+            part.val[SLOT_X] = val(p.mC); part.rank[SLOT_X] = rnk(p.mC);
             parts.push_back(part);
         }
         DinvStep st;

@@ -536,7 +536,6 @@ static void multiply_hmat_update(double alpha, dmhm_hmat_s* A, dmhm_hmat_s* B, d
     const int maxRank = C->maxRank;
     for (int c : C->lay->cap)
         if (c > 64) throw Error(DMHM_EINVAL, "low-rank capacity above 64 in a product");
-    std::unique_ptr<dmhm_hmat_s> Cold(copy_hmat(C, C->prec));
     const int over = o.oversample > 0 ? o.oversample : 4;
     const std::string key = "hhu:" + std::to_string(A->lay->id) + ":" + std::to_string(B->lay->id) + ":" +
                             std::to_string(C->lay->id) + ":" + std::to_string(maxRank) + ":" + std::to_string(over) +
@@ -548,8 +547,10 @@ static void multiply_hmat_update(double alpha, dmhm_hmat_s* A, dmhm_hmat_s* B, d
         return pl.hhProduct(*A->lay, *B->lay, *C->lay, maxRank, over, Planner::HH_UPDATE);
     });
     ensure_ws(p, A->esize());
-    Bases b = bases_for(A, B, C, Cold->vals, nullptr);
-    b.rank[SLOT_X] = Cold->ranks;
+    // C_old is C itself: the plan reads each block's old factors before its SVD
+    // and formation phases write the new ones.
+    Bases b = bases_for(A, B, C, C->vals, nullptr);
+    b.rank[SLOT_X] = C->ranks;
     TruncPolicy pol{o.tolMode, o.relTol};
     if (A->prec == DMHM_F64) run_plan<double>(p, b, alpha, beta, pol, o.seed);
     else run_plan<float>(p, b, (float)alpha, (float)beta, pol, o.seed);
@@ -2512,7 +2513,14 @@ void Plan::upload()
             for (const auto& t : ph.svd) ph.svdK = std::max(ph.svdK, t.k);
             src = ph.svd.data(); bytes = ph.svd.size() * sizeof(SvdTask);
         }
-        if (ph.kind == PH_RNG && !ph.rng.empty()) { src = ph.rng.data(); bytes = ph.rng.size() * sizeof(RngTask); }
+        std::vector<RngChunk> chunks;
+        if (ph.kind == PH_RNG && !ph.rng.empty()) {
+            for (const RngTask& t : ph.rng)
+                for (int64_t e = 0, n = (int64_t)t.m * t.k; e < n; e += kRngChunk)
+                    chunks.push_back({t.off, e, t.stream, (int32_t)std::min<int64_t>(kRngChunk, n - e), 0});
+            ph.rngChunks = (int)chunks.size();
+            src = chunks.data(); bytes = chunks.size() * sizeof(RngChunk);
+        }
         if (ph.kind == PH_MV_PROJ && !ph.mvProj.empty()) {
             // Tallest first: a workgroup's each, then a wave's each.
             std::stable_sort(ph.mvProj.begin(), ph.mvProj.end(),
@@ -2529,7 +2537,7 @@ void Plan::upload()
                                    hipMemcpyHostToDevice));
             std::vector<MvContrib>().swap(ph.mvContribs);
         }
-        if (src) {
+        if (src && bytes) {
             HIPCHECK(hipMalloc(&ph.dTasks, bytes));
             HIPCHECK(copy_sync(ph.dTasks, src, bytes, hipMemcpyHostToDevice));
         }

@@ -33,22 +33,21 @@ __device__ inline uint64_t seed_with(uint64_t seed0, const uint64_t* seedOff)
     return seed0 + (seedOff ? *seedOff * 0x9E3779B97F4A7C15ULL : 0);
 }
 template <typename T>
-__global__ void __launch_bounds__(256) rng_kernel(Bases b, const RngTask* __restrict__ tasks,
+__global__ void __launch_bounds__(256) rng_kernel(Bases b, const RngChunk* __restrict__ tasks,
                                                   uint64_t seed0, const uint64_t* seedOff)
 {
     const uint64_t seed = seed_with(seed0, seedOff);
-    const RngTask tk = tasks[blockIdx.x];
-    T* x = reinterpret_cast<T*>(b.val[SLOT_WS]) + tk.off;
-    const int64_t n = (int64_t)tk.m * tk.k;
-    for (int64_t e = threadIdx.x; e < n; e += 256) x[e] = (T)gauss_at(seed, tk.stream, (uint64_t)e);
+    const RngChunk tk = tasks[blockIdx.x];
+    T* x = reinterpret_cast<T*>(b.val[SLOT_WS]) + tk.off + tk.first;
+    for (int e = threadIdx.x; e < tk.count; e += 256) x[e] = (T)gauss_at(seed, tk.stream, (uint64_t)(tk.first + e));
 }
 
 template <typename T>
 void launch_rng_phase(const Phase& ph, const Bases& b, uint64_t seed, hipStream_t s, const uint64_t* seedOff)
 {
-    const int n = (int)ph.rng.size();
+    const int n = ph.rngChunks;
     if (n == 0) return;
-    rng_kernel<T><<<n, 256, 0, s>>>(b, static_cast<const RngTask*>(ph.dTasks), seed, seedOff);
+    rng_kernel<T><<<n, 256, 0, s>>>(b, static_cast<const RngChunk*>(ph.dTasks), seed, seedOff);
     HIP_LAUNCH_CHECK();
 }
 

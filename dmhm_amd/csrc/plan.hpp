@@ -85,6 +85,16 @@ struct RngTask {
     int32_t m, k;
     uint64_t stream;        // stream id mixed into the counter
 };
+// Up to kRngChunk consecutive entries of one sketch panel: one workgroup's
+// share (a workgroup per panel lasted as long as the largest one: 204 us per
+// 256^2 rank-16 FP64 product with panels of 64 to 4,096 rows).
+struct RngChunk {
+    int64_t off;            // workspace offset of the panel
+    int64_t first;          // first entry
+    uint64_t stream;
+    int32_t count, pad;
+};
+constexpr int kRngChunk = 1024;
 
 // Streaming H*X and H^T*X for few right-hand sides (HBM-bound): projections
 // P = V^T X per low-rank block (U^T X for H^T), then one workgroup per output
@@ -155,6 +165,7 @@ struct Phase {
     bool mvTrans = false;
     int mvBig = 0;          // leading projections of more than kMvBigRows rows (set by upload)
     void* dAux = nullptr;
+    int rngChunks = 0;      // device chunks of an RNG phase (set by upload)
     int qrK = 0;            // panel width of the QR phase
     int qrClassEnd[4] = {0, 0, 0, 0};   // QR tasks sorted by panel class at upload (see launch_qr_phase)
     int qrRegK = 0;         // widest task of classes 0..3
