@@ -21,18 +21,21 @@ namespace dmhm {
 // written as t = sgn(d) g / (|d| + sqrt(d^2 + g^2)) with d = be - al and
 // g = 2 ga. t does not change when d and g are scaled together, so both are
 // scaled by an estimate of 1 / max(|d|, |g|) first (no overflow or underflow
-// in the squares). c = 1 / sqrt(1 + t^2), s = c t. The reciprocals and
-// reciprocal square roots are the hardware estimates (v_rcp_f64, v_rsq_f64)
-// refined by two Newton steps each: a shorter dependent chain than IEEE
-// division and square root, and c^2 + s^2 = 1 to rounding either way.
+// in the squares). c = 1 / sqrt(1 + t^2), s = c t. t comes from the hardware
+// estimates (v_rcp_f64, v_rsq_f64) refined by one Newton step each, c by two:
+// an angle off by 1e-14 of itself leaves as little of the inner product, while
+// c^2 + s^2 = 1 to rounding for whatever t.
 __device__ inline void jacobi_rotation(double al, double be, double ga, double& cs, double& sn)
 {
     const double d0 = be - al, g0 = 2.0 * ga;
     const double rm = __builtin_amdgcn_rcp(fmax(fabs(d0), fabs(g0)));
     const double dd = d0 * rm, gg = g0 * rm;
     const double h = fma(dd, dd, gg * gg);
-    const double den = fabs(dd) + h * rsq_nr(h);
-    const double t = (dd >= 0.0 ? gg : -gg) * rcp_nr(den);
+    const double y = __builtin_amdgcn_rsq(h);
+    const double den = fabs(dd) + h * fma(0.5 * y, fma(-h * y, y, 1.0), y);
+    double r = __builtin_amdgcn_rcp(den);
+    r = fma(r, fma(-den, r, 1.0), r);
+    const double t = (dd >= 0.0 ? gg : -gg) * r;
     cs = rsq_nr(fma(t, t, 1.0));
     sn = cs * t;
 }
@@ -125,7 +128,10 @@ __global__ void __launch_bounds__(NT) svd_kernel(Bases b, const SvdTask* __restr
                                 Vs[p][r] = cs * vx[i] - sn * vy[i]; Vs[q][r] = sn * vx[i] + cs * vy[i];
                             }
                         }
-                        if (sub == 0) rotated = 1;
+                        // A sweep of small rotations only is the last one: with
+                        // every cosine and sine at most 1e-8 before it, the
+                        // cosines left are of the order of their products.
+                        if (sub == 0 && (fabs(sn) > 1e-8 || ga * ga > 1e-16 * (al * be))) rotated = 1;
                     }
                 }
             }
@@ -142,14 +148,21 @@ __global__ void __launch_bounds__(NT) svd_kernel(Bases b, const SvdTask* __restr
         sig[tid] = sqrt(s);
     }
     __syncthreads();
-    if (tid == 0) {
-        for (int c = 0; c < k; ++c) order[c] = c;
-        for (int a = 0; a < k; ++a) {          // selection sort, descending
-            int best = a;
-            for (int c = a + 1; c < k; ++c)
-                if (sig[order[c]] > sig[order[best]]) best = c;
-            const int tmp = order[a]; order[a] = order[best]; order[best] = tmp;
+    if (tid < k) {
+        // Descending order: a column's place is the number of columns before
+        // it (as bit patterns, a total order whatever the values; ties by index).
+        auto key = [&](int c) { return (uint64_t)__double_as_longlong(sig[c]) & ~(uint64_t(1) << 63); };
+        const uint64_t mine = key(tid);
+        int place = 0;
+#pragma unroll 8
+        for (int c = 0; c < k; ++c) {
+            const uint64_t x = key(c);
+            place += x > mine || (x == mine && c < tid);
         }
+        order[place] = tid;
+    }
+    __syncthreads();
+    if (tid == 0) {
         int keep = min(tk.maxKeep, k);
         if (tolMode == 1) {
             const double s0 = sig[order[0]];
@@ -194,9 +207,14 @@ void launch_svd_phase(const Phase& ph, const Bases& b, TruncPolicy pol, hipStrea
     const SvdTask* t = static_cast<const SvdTask*>(ph.dTasks);
     if (ph.svdK > 64) throw std::runtime_error("SVD factor wider than 64");
     // 24-column factors: 16 threads per column pair for phases of few factors
-    // (one workgroup per CU, the time is one factor's latency: 89 us against
-    // 99 us with 8 threads for 80 factors of k = 20), 8 threads beyond
-    // (120 us against 136 us for 850 factors).
+    // (one workgroup per CU, the time is one factor's latency), 8 threads
+    // beyond (a 256^2 inversion's SVDs: 55.1 ms with the line at 256 factors,
+    // 54.6 at 1,024). A factor of k = 20 takes 3 to 5 sweeps of about 1,450
+    // cycles per round: the reads, the three sums over a pair's threads, the
+    // rotation's dependent chain, the writes and a barrier. 55 us per launch of
+    // few factors and 108 us for 850; 74 and 134 us with one thread sorting the
+    // columns (43,000 of 150,000 cycles), two Newton steps per estimate and a
+    // last sweep without rotations.
     if (ph.svdK <= 24 && n < kSvdLatencyTasks) svd_kernel<T, 24, 192, 16><<<n, 192, 0, s>>>(b, t, pol.tolMode, pol.relTol);
     else if (ph.svdK <= 24) svd_kernel<T, 24, 128, 8><<<n, 128, 0, s>>>(b, t, pol.tolMode, pol.relTol);
     else if (ph.svdK <= 40) svd_kernel<T, 40, 192><<<n, 192, 0, s>>>(b, t, pol.tolMode, pol.relTol);
