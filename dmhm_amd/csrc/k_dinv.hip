@@ -141,10 +141,10 @@ __global__ __launch_bounds__(NT) void dense_inverse_kernel(const T* __restrict__
 // row maxima through scalar registers); the result is uniform.
 __device__ inline uint32_t wave_max_u32(uint32_t x)
 {
-    x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, kDppXor1, 0xF, 0xF, false));
-    x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, kDppXor2, 0xF, 0xF, false));
-    x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, kDppMirror8, 0xF, 0xF, false));
-    x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, kDppMirror16, 0xF, 0xF, false));
+    x = max(x, (uint32_t)__builtin_amdgcn_mov_dpp((int)x, kDppXor1, 0xF, 0xF, false));
+    x = max(x, (uint32_t)__builtin_amdgcn_mov_dpp((int)x, kDppXor2, 0xF, 0xF, false));
+    x = max(x, (uint32_t)__builtin_amdgcn_mov_dpp((int)x, kDppMirror8, 0xF, 0xF, false));
+    x = max(x, (uint32_t)__builtin_amdgcn_mov_dpp((int)x, kDppMirror16, 0xF, 0xF, false));
     const uint32_t a = __builtin_amdgcn_readlane(x, 0), b = __builtin_amdgcn_readlane(x, 16);
     const uint32_t c = __builtin_amdgcn_readlane(x, 32), e = __builtin_amdgcn_readlane(x, 48);
     return max(max(a, b), max(c, e));
@@ -153,7 +153,7 @@ __device__ inline uint32_t wave_max_u32(uint32_t x)
 // Inverse of one m x m leaf (m <= 64): Gauss-Jordan with partial pivoting,
 // lane = row, the 64 columns split over NWV waves (wave w holds columns
 // [w CW, (w + 1) CW) of every row in registers). Three departures from the
-// textbook form keep each step to one barrier and one LDS exchange:
+// textbook form keep a panel of CW steps to one barrier and one LDS exchange:
 // - rows are not exchanged: step k takes the largest |u(i,k)| over the rows
 //   not yet used as pivots (compared on the high word of the double: sign
 //   cleared, exponent and 20 mantissa bits, ties to the lowest row) and
@@ -162,11 +162,13 @@ __device__ inline uint32_t wave_max_u32(uint32_t x)
 // - the pivot row is not scaled by 1/u(p,k) at its step: the factor of every
 //   other row is u(i,k) / u(p,k) either way, so the scale is kept per row and
 //   applied at the store (the row's entries stay, its column-k entry is 1);
-// - the wave that owns column k chooses the pivot and publishes the pivot
-//   row's index, 1/u(p,k) and every row's factor through LDS; every wave then
-//   updates only its own columns, reading its share of the pivot row from its
-//   own lane p (v_readlane). Buffers alternate by step parity, so a step's
-//   writes never meet the previous step's reads.
+// - the wave that owns columns k .. k + CW - 1 takes all their steps on its own
+//   columns alone (they need no other wave's) and publishes the CW pivot rows'
+//   indices and every row's factors through LDS; the other waves then apply the
+//   CW steps to their own columns, reading their share of each pivot row from
+//   their own lane p (v_readlane), the next panel's wave ahead of the others.
+//   Buffers alternate by panel parity, so a panel's writes never meet the
+//   previous one's reads: one barrier per panel.
 // Padding rows and columns beyond m hold the identity; their steps (up to
 // CW - 1 in the last panel) change nothing.
 template <typename T, int NWV>
@@ -175,9 +177,8 @@ __global__ void __launch_bounds__(64 * NWV) dense_inverse_split_kernel(const T* 
                                                                       int* __restrict__ singular)
 {
     constexpr int CW = 64 / NWV;
-    static_assert(CW % 2 == 0, "step parity follows the column within a wave");
-    __shared__ double gbuf[2][64], ibuf[2];
-    __shared__ int pbuf[2];
+    __shared__ double gbuf[2][CW][64], scales[64];      // scales: of the steps' pivot rows
+    __shared__ int pivs[64], steps[64];                 // pivot row of a step, step of a row
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     double u[CW];
 #pragma unroll
@@ -185,59 +186,71 @@ __global__ void __launch_bounds__(64 * NWV) dense_inverse_split_kernel(const T* 
         const int c = w * CW + j;
         u[j] = (c < m && lane < m) ? (double)src[lane + (int64_t)c * m] : (c == lane ? 1.0 : 0.0);
     }
-    bool used = false, sing = false;
-    double scale = 1.0;
-    int stepOf = 0, pivOf = 0;      // this row's step; the pivot row of step `lane`
+    bool sing = false;
+    uint64_t used = 0;              // rows that have been pivots
     const int panels = (m + CW - 1) / CW;
 #pragma unroll 1
     for (int kb = 0; kb < panels; ++kb) {
-        const bool owner = w == kb;
+        const int par = kb & 1;
+        if (w == kb) {
+#pragma unroll
+            for (int kk = 0; kk < CW; ++kk) {
+                const double v = u[kk];
+                const uint32_t hi = used >> lane & 1 ? 0u : ((uint32_t)__double2hiint(v) & 0x7fffffffu);
+                const uint32_t mx = wave_max_u32(hi);
+                const uint64_t cand = __ballot(hi == mx) & ~used;
+                const int p = __builtin_ctzll(cand);
+                const double dd = bcast(v, p);
+                const double inv = dd == 0.0 ? 0.0 : rcp_nr(dd);
+                const double g = lane == p ? 0.0 : v * inv;
+                gbuf[par][kk][lane] = g;
+                if (lane == p) {
+                    pivs[kb * CW + kk] = p;
+                    scales[kb * CW + kk] = inv;
+                    steps[p] = kb * CW + kk;
+                }
+                sing = sing || dd == 0.0;
+                used |= uint64_t(1) << p;
+#pragma unroll
+                for (int j = 0; j < CW; ++j)
+                    u[j] = j == kk ? (lane == p ? 1.0 : -g) : fma(-g, bcast(u[j], p), u[j]);
+            }
+        }
+        __syncthreads();
+        if (w == kb) {
+            __builtin_amdgcn_s_setprio(0);
+            continue;
+        }
+        if (w == kb + 1) __builtin_amdgcn_s_setprio(3);
+        const int pl = pivs[kb * CW + lane % CW];
 #pragma unroll
         for (int kk = 0; kk < CW; ++kk) {
-            const int k = kb * CW + kk, par = kk & 1;
-            if (owner) {
-                const double v = u[kk];
-                const uint32_t hi = used ? 0u : ((uint32_t)__double2hiint(v) & 0x7fffffffu);
-                const uint32_t mx = wave_max_u32(hi);
-                const unsigned long long cand = __ballot(!used && hi == mx);
-                const int p = __builtin_amdgcn_readfirstlane(__ffsll(cand) - 1);
-                const double dd = bcast(v, p);
-                const double inv = dd == 0.0 ? 0.0 : 1.0 / dd;
-                gbuf[par][lane] = lane == p ? 0.0 : v * inv;
-                if (lane == 0) { pbuf[par] = p; ibuf[par] = inv; }
-                sing = sing || dd == 0.0;
-            }
-            __syncthreads();
-            const int p = __builtin_amdgcn_readfirstlane(pbuf[par]);
-            const double inv = ibuf[par];
-            const double g = gbuf[par][lane];
-            const bool me = lane == p;
+            const int p = __builtin_amdgcn_readlane(pl, kk);
+            const double g = gbuf[par][kk][lane];
+            used |= uint64_t(1) << p;
 #pragma unroll
-            for (int j = 0; j < CW; ++j) {
-                if (j == kk && owner) u[j] = me ? 1.0 : -g;
-                else u[j] = fma(-g, bcast(u[j], p), u[j]);
-            }
-            scale = me ? inv : scale;
-            used = used || me;
-            stepOf = me ? k : stepOf;
-            pivOf = lane == k ? p : pivOf;
+            for (int j = 0; j < CW; ++j) u[j] = fma(-g, bcast(u[j], p), u[j]);
         }
     }
     if (sing && lane == 0) atomicExch(singular, 1);
-    const bool row = lane < m && stepOf < m;
+    // A row beyond m is its own pivot in a step beyond m, or in none.
+    const int step = used >> lane & 1 ? steps[lane] : 64;
+    const double scale = step < m ? scales[step] : 0.0;
+    const bool row = lane < m && step < m;
 #pragma unroll
     for (int j = 0; j < CW; ++j) {
         const int c = w * CW + j;
-        const int pc = __builtin_amdgcn_readlane(pivOf, c);
-        if (row && c < m && pc < m) dst[stepOf + (int64_t)pc * m] = (T)(u[j] * scale);
+        if (row && c < m && pivs[c] < m) dst[step + (int64_t)pivs[c] * m] = (T)(u[j] * scale);
     }
 }
 
-// Waves of the leaf inversion (a 64 x 64 FP64 leaf: 28 us with 8 waves or
-// 16, 32 us with 4, 66 us with one wave that broadcasts the whole pivot row
-// by lane reads, against 108 us for lane = column with rows split over 8
-// waves and two barriers per step).
-constexpr int kInvWaves = 8;
+// Waves of the leaf inversion. What bounds it is the instructions of the wave
+// that owns the panel: its own steps (the pivot search and reciprocal, then a
+// lane read and an FMA per column) and the steps of the panel before it. A 64 x
+// 64 FP64 leaf: 29.0 us with a barrier and an exchange per column, 25.5 us per
+// panel of 8 columns (8 waves), 20.9 us per panel of 4 (16 waves), a launch of
+// about 4 us included; 108 us for lane = column with rows split over 8 waves.
+constexpr int kInvWaves = 16;
 
 template <typename T>
 void launch_dense_inverse(const T* src, T* dst, int m, int* singular, hipStream_t s)
