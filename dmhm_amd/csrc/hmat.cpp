@@ -2445,6 +2445,7 @@ void Plan::upload()
             // arrays must already be on the device.
             std::vector<TileSeg> segs;
             ph.segTiles = ph.segBlocks[0] = ph.segBlocks[1] = ph.segBlocks[2] = 0;
+            ph.wide = true;
             for (const auto& s : ph.segSrc) {
                 const int n = (int)s.src->tiles.size();
                 if (n > 0 && (!s.src->dTiles || !s.src->dContribs))
@@ -2456,6 +2457,7 @@ void Plan::upload()
                 for (int k = 0; k < NUM_SLOTS; ++k) { t.val[k] = s.val[k]; t.rank[k] = s.rank[k]; }
                 t.count = n;
                 t.nLong = s.src->nLong;
+                ph.wide = ph.wide && s.src->wide;
                 t.first = ph.segTiles;
                 ph.segTiles += n;
                 for (int i = 0; i < 3; ++i) {

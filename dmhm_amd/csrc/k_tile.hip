@@ -805,21 +805,32 @@ static void launch_mfma_u(const Phase& ph, const Bases& b, T alpha, T beta, hipS
 
 // Units of the launch: 32 x 32 entries (a row or column block less where the
 // tiles are narrower), one per wave but for the long tiles, where the phase
-// has tiles enough to give each of the 1,024 SIMDs two such waves, else 16 x
-// 16 split over the four waves of a workgroup: such a phase is one tile's
+// has tiles enough to give each of the 1,024 SIMDs one such wave, else 16 x 16
+// split over the four waves of a workgroup: such a phase is one tile's
 // latency, and the split cuts it (direct inversion of 64^2 at rank 8, 940
 // launches of at most a few hundred tiles: 15.4 -> 10.6 ms; of 256^2 at rank
-// 16 with its refinement: 648 -> 500 ms).
-constexpr int64_t kMfmaWaves = 2048;
+// 16 with its refinement: 648 -> 500 ms. With the line at 512, 1,024, 2,048
+// and 4,096 units: 8.20, 8.20, 8.30 and 8.46 ms, and 370, 370, 373 and 379 ms).
+// From 8,192 units of tiles that are mostly wide (Phase::wide), units of 64
+// columns: a quarter (16 rows: a sixth) fewer operand loads per MFMA and half as
+// many waves that begin with a chain of dependent loads, for two waves per SIMD
+// instead of three (H X with 64 columns on the 256^2 inverse 891 -> 846 us,
+// 256^2 FP64 product 47.0 -> 45.6 ms, FP32 3D update 9.91 -> 8.61 ms, 9.00 with
+// the line at 4,096).
+constexpr int64_t kMfmaWaves = 1024, kMfmaWide = 8192;
 
 template <typename T, int MODE>
 static void launch_mfma(const Phase& ph, const Bases& b, T alpha, T beta, hipStream_t s)
 {
     const int64_t n = ph.segSrc.empty() ? (int64_t)ph.tiles.size() : ph.segTiles;
-    const int rb = ph.maxMTile <= 16 ? 1 : 2, cb = ph.maxKTile <= 16 ? 1 : 2;
+    const int rb = ph.maxMTile <= 16 ? 1 : 2;
+    int cb = ph.maxKTile <= 16 ? 1 : 2;
     const int64_t units = n * ((ph.maxMTile + 16 * rb - 1) / (16 * rb)) * ((ph.maxKTile + 16 * cb - 1) / (16 * cb));
+    if (units >= kMfmaWide && ph.wide) cb = 4;
     if (units < kMfmaWaves) launch_mfma_u<T, MODE, 1, 1, true>(ph, b, alpha, beta, s);
     else if (rb == 1 && cb == 1) launch_mfma_u<T, MODE, 1, 1, false>(ph, b, alpha, beta, s);
+    else if (rb == 2 && cb == 4) launch_mfma_u<T, MODE, 2, 4, false>(ph, b, alpha, beta, s);
+    else if (cb == 4) launch_mfma_u<T, MODE, 1, 4, false>(ph, b, alpha, beta, s);
     else if (rb == 1) launch_mfma_u<T, MODE, 1, 2, false>(ph, b, alpha, beta, s);
     else if (cb == 1) launch_mfma_u<T, MODE, 2, 1, false>(ph, b, alpha, beta, s);
     else launch_mfma_u<T, MODE, 2, 2, false>(ph, b, alpha, beta, s);

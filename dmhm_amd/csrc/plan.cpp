@@ -64,6 +64,9 @@ void order_tiles(Phase& ph)
         cls[c].push_back(t);
     }
     ph.nLong = (int)cls[0].size();
+    int64_t by32 = 0, by64 = 0;                 // 16-column blocks in units of 32 and of 64 columns
+    for (const Tile& t : ph.tiles) { by32 += (t.k + 31) / 32 * 2; by64 += (t.k + 63) / 64 * 4; }
+    ph.wide = 8 * by64 <= 9 * by32;
     ph.tiles.clear();
     for (auto& v : cls) ph.tiles.insert(ph.tiles.end(), v.begin(), v.end());
 }

@@ -161,6 +161,7 @@ struct Phase {
     void* dSegs = nullptr;
     int segTiles = 0, segBlocks[3] = {0, 0, 0};   // tiles of a segmented phase, workgroups of its MFMA launch
     int nLong = 0;          // leading tiles whose units are split over a workgroup (order_tiles)
+    bool wide = false;      // units of 64 columns waste little on these tiles' widths (order_tiles)
     int mvK = 0, ldx = 0, ldy = 0;
     bool mvTrans = false;
     int mvBig = 0;          // leading projections of more than kMvBigRows rows (set by upload)
