@@ -41,18 +41,28 @@ void* DevicePool::get(size_t bytes)
         held_.erase(it);
         return p;
     }
+    void* p = raw(bytes);
+    size_[p] = bytes;
+    return p;
+}
+
+void* DevicePool::raw(size_t bytes)
+{
     void* p = nullptr;
     hipError_t e = hipMalloc(&p, bytes);
     if (e == hipErrorOutOfMemory && !held_.empty()) {
         (void)hipGetLastError();
-        for (auto& h : held_) { size_.erase(h.second); (void)hipFree(h.second); }
-        held_.clear();
-        holding_ = 0;
+        drop();
         e = hipMalloc(&p, bytes);
     }
     HIPCHECK(e);
-    size_[p] = bytes;
     return p;
+}
+
+void* DevicePool::outside(size_t bytes)
+{
+    std::lock_guard<std::mutex> lk(mu_);
+    return raw(bytes);
 }
 
 void DevicePool::put(void* p)
@@ -68,12 +78,17 @@ void DevicePool::put(void* p)
     (void)hipFree(p);
 }
 
-void DevicePool::trim()
+void DevicePool::drop()
 {
-    std::lock_guard<std::mutex> lk(mu_);
     for (auto& h : held_) { size_.erase(h.second); (void)hipFree(h.second); }
     held_.clear();
     holding_ = 0;
+}
+
+void DevicePool::trim()
+{
+    std::lock_guard<std::mutex> lk(mu_);
+    drop();
 }
 
 // Copies on the library stream and waits for them: the stream is created
@@ -665,7 +680,7 @@ static void rounded_update_dev(int maxRank, double alpha, int m, int n, int rA, 
     }
     job.ws.ensure(o * sizeof(double));
     HIPCHECK(copy_sync(job.ws.ptr, host.data(), o * sizeof(double), hipMemcpyHostToDevice));
-    HIPCHECK(hipMalloc((void**)&job.rank, sizeof(int)));
+    job.rank = static_cast<int*>(device_pool().outside(sizeof(int)));
     job.plan.phases.resize(5);
     Phase& q = job.plan.phases[0];
     q.kind = PH_QR;
@@ -714,7 +729,7 @@ static void compress_dense_dev(int maxRank, int m, int n, const double* D, doubl
         for (int i = 0; i < m; ++i) host[Dd + i + (size_t)j * mp] = D[i + (size_t)j * m];
     job.ws.ensure(o * sizeof(double));
     HIPCHECK(copy_sync(job.ws.ptr, host.data(), o * sizeof(double), hipMemcpyHostToDevice));
-    HIPCHECK(hipMalloc((void**)&job.rank, sizeof(int)));
+    job.rank = static_cast<int*>(device_pool().outside(sizeof(int)));
     job.plan.phases.resize(3);
     job.plan.phases[0].kind = PH_QR;
     job.plan.phases[0].qr.push_back(QrTask{Dd, R, mp, k, mp, k, SLOT_WS});
@@ -795,7 +810,7 @@ dmhm_hmat_s* copy_hmat(dmhm_hmat_s* s, int prec)
 template <typename T>
 static void upload(std::vector<T>& v, T** d)
 {
-    HIPCHECK(hipMalloc((void**)d, std::max<size_t>(v.size(), 1) * sizeof(T)));
+    *d = static_cast<T*>(device_pool().outside(std::max<size_t>(v.size(), 1) * sizeof(T)));
     if (!v.empty()) HIPCHECK(copy_sync(*d, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
 }
 
@@ -2466,21 +2481,21 @@ void Plan::upload()
                 }
                 segs.push_back(t);
             }
-            HIPCHECK(hipMalloc(&ph.dSegs, segs.size() * sizeof(TileSeg)));
+            ph.dSegs = device_pool().outside(segs.size() * sizeof(TileSeg));
             HIPCHECK(copy_sync(ph.dSegs, segs.data(), segs.size() * sizeof(TileSeg), hipMemcpyHostToDevice));
         }
         if (!ph.tiles.empty()) {
             order_tiles(ph);
-            HIPCHECK(hipMalloc(&ph.dTiles, ph.tiles.size() * sizeof(Tile)));
+            ph.dTiles = device_pool().outside(ph.tiles.size() * sizeof(Tile));
             HIPCHECK(copy_sync(ph.dTiles, ph.tiles.data(), ph.tiles.size() * sizeof(Tile), hipMemcpyHostToDevice));
         }
         if (!ph.contribs.empty()) {
-            HIPCHECK(hipMalloc(&ph.dContribs, ph.contribs.size() * sizeof(Contrib)));
+            ph.dContribs = device_pool().outside(ph.contribs.size() * sizeof(Contrib));
             HIPCHECK(copy_sync(ph.dContribs, ph.contribs.data(), ph.contribs.size() * sizeof(Contrib),
                                hipMemcpyHostToDevice));
         }
         if (!ph.gtab.empty()) {
-            HIPCHECK(hipMalloc(&ph.dGather, ph.gtab.size() * sizeof(int64_t)));
+            ph.dGather = device_pool().outside(ph.gtab.size() * sizeof(int64_t));
             HIPCHECK(copy_sync(ph.dGather, ph.gtab.data(), ph.gtab.size() * sizeof(int64_t), hipMemcpyHostToDevice));
         }
         const void* src = nullptr; size_t bytes = 0;
@@ -2533,14 +2548,14 @@ void Plan::upload()
         }
         if (ph.kind == PH_MV_ACC && !ph.mvAtoms.empty()) {
             src = ph.mvAtoms.data(); bytes = ph.mvAtoms.size() * sizeof(MvAtom);
-            HIPCHECK(hipMalloc(&ph.dAux, std::max<size_t>(ph.mvContribs.size(), 1) * sizeof(MvContrib)));
+            ph.dAux = device_pool().outside(std::max<size_t>(ph.mvContribs.size(), 1) * sizeof(MvContrib));
             if (!ph.mvContribs.empty())
                 HIPCHECK(copy_sync(ph.dAux, ph.mvContribs.data(), ph.mvContribs.size() * sizeof(MvContrib),
                                    hipMemcpyHostToDevice));
             std::vector<MvContrib>().swap(ph.mvContribs);
         }
         if (src && bytes) {
-            HIPCHECK(hipMalloc(&ph.dTasks, bytes));
+            ph.dTasks = device_pool().outside(bytes);
             HIPCHECK(copy_sync(ph.dTasks, src, bytes, hipMemcpyHostToDevice));
         }
         // Host copies of the big arrays are no longer needed (unless merged

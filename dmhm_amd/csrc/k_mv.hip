@@ -271,6 +271,7 @@ __global__ void __launch_bounds__(64 * NW) mv_acc_kernel(Bases b, const MvAtom* 
         constexpr int VW = 16 / (int)sizeof(T), LPC = 64 / VW;
         constexpr int NA = K <= 2 ? (NW == 16 ? 4 : 8) / K : 2;     // 16 waves have 128 registers each
         const int rg = i % LPC, cg = i / LPC;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");     // red[w] was written by the wave's other lanes
         for (int c0 = 0; c0 < at.m; c0 += NA * VW) {
             T acc[NA][K];
 #pragma unroll

@@ -52,7 +52,11 @@ public:
     void* get(size_t bytes);
     void put(void* p);
     void trim();
+    // Memory that is not pooled (hipFree gives it back), for plans' tables.
+    void* outside(size_t bytes);
 private:
+    void* raw(size_t bytes);
+    void drop();
     static constexpr size_t kHoldMax = size_t(4) << 30, kBlockMax = size_t(2) << 30;
     std::mutex mu_;
     std::multimap<size_t, void*> held_;
