@@ -1,10 +1,9 @@
 // gfx950 kernels of the recursive direct inversion (HMat2d/HMat3d::
 // DirectInvert, src/HMat2d/Invert-incl.hpp:17-125) and of merged plans: the
 // dense leaf inverse (hmat_tools::Invert on a Dense, src/hmat_tools/
-// Invert.cpp:14-42, there LAPACK getrf + getri), copies and fills of index
+// Invert.cpp:14-42, there LAPACK getrf + getri), and copies and fills of index
 // ranges inside one allocation (sub-matrix copies: a subtree of the block
-// tree is one contiguous range of each storage pool), and identities at
-// several workspace offsets.
+// tree is one contiguous range of each storage pool).
 #include "kcommon.hpp"
 
 namespace dmhm {
