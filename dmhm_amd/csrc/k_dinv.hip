@@ -243,6 +243,128 @@ __global__ void __launch_bounds__(64 * NWV) dense_inverse_split_kernel(const T* 
     }
 }
 
+// The same elimination for a leaf of up to 64 RR rows, worked on in memory
+// (`work`, overwritten) in panels of NB columns: the first wave takes a panel's
+// steps in registers (rows lane + 64 r) and publishes its pivots and factors,
+// then every wave applies the NB steps to whole columns in one read and one
+// write of each. One step per pass over the matrix, as dense_inverse_kernel
+// takes, is bound by that traffic through one CU. Direct inversion of 88^2 in
+// leaves of 121 points (FP64, rank 8): 89.7 -> 22.2 ms, of 120^2 in leaves of
+// 225 points 415 -> 290 ms.
+template <typename T, int RR>
+__global__ void __launch_bounds__(1024) dense_inverse_panel_kernel(T* work, T* __restrict__ dst, int m,
+                                                                   int* __restrict__ singular)
+{
+    constexpr int NB = 8, NW = 16;
+    __shared__ double G[NB][64 * RR], scales[64 * RR];
+    __shared__ int pivs[64 * RR], steps[64 * RR];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // Entry of row p of a column held as rows lane + 64 r (p uniform).
+    auto at = [&](const double (&x)[RR], int p) {
+        double v = x[0];
+#pragma unroll
+        for (int r = 1; r < RR; ++r) v = p >> 6 == r ? x[r] : v;
+        return bcast(v, p & 63);
+    };
+    uint64_t used[RR] = {};         // rows that have been pivots (kept by the first wave)
+    bool sing = false;
+#pragma unroll 1
+    for (int k0 = 0; k0 < m; k0 += NB) {
+        const int nb = min(NB, m - k0);
+        if (w == 0) {
+            double u[NB][RR];
+#pragma unroll
+            for (int j = 0; j < NB; ++j)
+#pragma unroll
+                for (int r = 0; r < RR; ++r) {
+                    const int i = lane + 64 * r;
+                    u[j][r] = j < nb && i < m ? (double)work[i + (int64_t)(k0 + j) * m] : 0.0;
+                }
+#pragma unroll
+            for (int kk = 0; kk < NB; ++kk) {
+                if (kk >= nb) continue;
+                uint32_t hi[RR], mine = 0;
+#pragma unroll
+                for (int r = 0; r < RR; ++r) {
+                    const bool open = lane + 64 * r < m && !(used[r] >> lane & 1);
+                    hi[r] = open ? (uint32_t)__double2hiint(u[kk][r]) & 0x7fffffffu : 0u;
+                    mine = max(mine, hi[r]);
+                }
+                const uint32_t mx = wave_max_u32(mine);
+                int p = -1;
+#pragma unroll
+                for (int r = 0; r < RR; ++r) {
+                    const uint64_t cand = __ballot(lane + 64 * r < m && hi[r] == mx) & ~used[r];
+                    if (p < 0 && cand) {
+                        p = 64 * r + __builtin_ctzll(cand);
+                        used[r] |= cand & (~cand + 1);
+                    }
+                }
+                p = __builtin_amdgcn_readfirstlane(p);
+                const double dd = at(u[kk], p);
+                const double inv = dd == 0.0 ? 0.0 : rcp_nr(dd);
+                sing = sing || dd == 0.0;
+                double g[RR];
+#pragma unroll
+                for (int r = 0; r < RR; ++r) {
+                    g[r] = lane + 64 * r == p ? 0.0 : u[kk][r] * inv;
+                    G[kk][lane + 64 * r] = g[r];
+                }
+                if (lane == 0) { pivs[k0 + kk] = p; scales[k0 + kk] = inv; steps[p] = k0 + kk; }
+#pragma unroll
+                for (int j = 0; j < NB; ++j) {
+                    const double x = at(u[j], p);
+#pragma unroll
+                    for (int r = 0; r < RR; ++r)
+                        u[j][r] = j == kk ? (lane + 64 * r == p ? 1.0 : -g[r]) : fma(-g[r], x, u[j][r]);
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < NB; ++j)
+#pragma unroll
+                for (int r = 0; r < RR; ++r) {
+                    const int i = lane + 64 * r;
+                    if (j < nb && i < m) work[i + (int64_t)(k0 + j) * m] = (T)u[j][r];
+                }
+        }
+        __syncthreads();
+        double g[NB][RR];
+#pragma unroll
+        for (int kk = 0; kk < NB; ++kk)
+#pragma unroll
+            for (int r = 0; r < RR; ++r) g[kk][r] = kk < nb ? G[kk][lane + 64 * r] : 0.0;
+        const int pl = pivs[k0 + min(lane, nb - 1)];
+#pragma unroll 1
+        for (int c = w; c < m; c += NW) {
+            if (c >= k0 && c < k0 + nb) continue;
+            T* col = work + (int64_t)c * m;
+            double x[RR];
+#pragma unroll
+            for (int r = 0; r < RR; ++r) x[r] = lane + 64 * r < m ? (double)col[lane + 64 * r] : 0.0;
+#pragma unroll
+            for (int kk = 0; kk < NB; ++kk) {
+                if (kk >= nb) continue;
+                const double v = at(x, __builtin_amdgcn_readlane(pl, kk));
+#pragma unroll
+                for (int r = 0; r < RR; ++r) x[r] = fma(-g[kk][r], v, x[r]);
+            }
+#pragma unroll
+            for (int r = 0; r < RR; ++r)
+                if (lane + 64 * r < m) col[lane + 64 * r] = (T)x[r];
+        }
+        __syncthreads();
+    }
+    if (sing && threadIdx.x == 0) atomicExch(singular, 1);
+    for (int c = w; c < m; c += NW) {
+        const int pc = pivs[c];
+#pragma unroll
+        for (int r = 0; r < RR; ++r) {
+            const int i = lane + 64 * r;
+            if (i < m) dst[steps[i] + (int64_t)pc * m] = (T)((double)work[i + (int64_t)c * m] * scales[steps[i]]);
+        }
+    }
+}
+
 // Waves of the leaf inversion. What bounds it is the instructions of the wave
 // that owns the panel: its own steps (the pivot search and reciprocal, then a
 // lane read and an FMA per column) and the steps of the panel before it. A 64 x
@@ -251,12 +373,19 @@ __global__ void __launch_bounds__(64 * NWV) dense_inverse_split_kernel(const T* 
 // about 4 us included; 108 us for lane = column with rows split over 8 waves.
 constexpr int kInvWaves = 16;
 
+// `src` is overwritten (m in 65 .. 256).
 template <typename T>
-void launch_dense_inverse(const T* src, T* dst, int m, int* singular, hipStream_t s)
+void launch_dense_inverse(T* src, T* dst, int m, int* singular, hipStream_t s)
 {
     if (m <= 0) return;
     if (m <= 64) {
         dense_inverse_split_kernel<T, kInvWaves><<<1, 64 * kInvWaves, 0, s>>>(src, dst, m, singular);
+        HIP_LAUNCH_CHECK();
+        return;
+    }
+    if (m <= 256) {
+        if (m <= 128) dense_inverse_panel_kernel<T, 2><<<1, 1024, 0, s>>>(src, dst, m, singular);
+        else dense_inverse_panel_kernel<T, 4><<<1, 1024, 0, s>>>(src, dst, m, singular);
         HIP_LAUNCH_CHECK();
         return;
     }
@@ -271,7 +400,7 @@ void launch_dense_inverse(const T* src, T* dst, int m, int* singular, hipStream_
 #define INST(T)                                                                                          \
     template void launch_copy_ranges<T>(const T*, T*, const CopyRange*, int, int64_t, bool, hipStream_t); \
     template void launch_arena_ranges<T>(T*, int*, const CopyRange*, int, int, int64_t, bool, hipStream_t); \
-    template void launch_dense_inverse<T>(const T*, T*, int, int*, hipStream_t);
+    template void launch_dense_inverse<T>(T*, T*, int, int*, hipStream_t);
 INST(double)
 INST(float)
 template void launch_copy_ranges<int>(const int*, int*, const CopyRange*, int, int64_t, bool, hipStream_t);

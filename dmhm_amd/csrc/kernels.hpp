@@ -76,7 +76,7 @@ template <typename T> void launch_arena_ranges(T* vals, int* ranks, const CopyRa
                                                int64_t maxLen, bool fill, hipStream_t s);
 // dst (m x m, ld m) = inverse of src (Gauss-Jordan, partial pivoting); a zero
 // pivot sets *singular (device int).
-template <typename T> void launch_dense_inverse(const T* src, T* dst, int m, int* singular, hipStream_t s);
+template <typename T> void launch_dense_inverse(T* src, T* dst, int m, int* singular, hipStream_t s);
 
 // Vector utilities for the power iteration (EstimateTwoNorm).
 template <typename T> void launch_sumsq(const T* x, int64_t n, double* out, hipStream_t s);

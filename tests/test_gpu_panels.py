@@ -43,8 +43,9 @@ def test_rounded_update_at_panel_edges(m, n, k, graded):
     assert np.linalg.norm(U @ V.T - want) <= tol * np.linalg.norm(U0) * np.linalg.norm(V0)
 
 
-# Panels of 4 columns: one short, whole, one over, and the largest leaf.
-@pytest.mark.parametrize("m", [1, 3, 4, 5, 31, 60, 61, 63, 64])
+# Panels of 4 columns (of 8 beyond 64 rows): one short, whole, one over, and
+# the first and last size of each kernel.
+@pytest.mark.parametrize("m", [1, 3, 4, 5, 31, 60, 61, 63, 64, 65, 72, 127, 128, 129, 255, 256, 257])
 def test_leaf_inverse_at_panel_edges(m):
     print("case", m, flush=True)
     rng = np.random.default_rng(m)
