@@ -64,18 +64,17 @@ void launch_copy_ranges(const T* src, T* dst, const CopyRange* ranges, int count
 // at step k the pivot row p (largest |a(i,k)|, i >= k) is swapped into row k,
 // then every entry is updated from the saved column k and the scaled row k;
 // the row swaps are undone as column swaps in reverse order at the end. The
-// matrix is held in LDS when `inLds` (loaded from src, stored to dst), else
-// worked on in dst (copied from src first). A zero pivot sets *singular.
+// matrix is worked on in dst (copied from src first). A zero pivot sets *singular.
 template <typename T, int NT>
 __global__ __launch_bounds__(NT) void dense_inverse_kernel(const T* __restrict__ src, T* __restrict__ dst, int m,
-                                                           bool inLds, int* __restrict__ singular)
+                                                           int* __restrict__ singular)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     T* col = reinterpret_cast<T*>(smem);              // saved column k (m)
     T* row = col + m;                                 // scaled row k (m)
     int* piv = reinterpret_cast<int*>(row + m);       // pivot rows (m)
     __shared__ int pivot;
-    T* a = inLds ? reinterpret_cast<T*>(piv + ((m + 3) & ~3)) : dst;
+    T* a = dst;
     const int tid = threadIdx.x;
     const int mm = m * m;
     for (int e = tid; e < mm; e += NT) a[e] = src[e];
@@ -132,8 +131,6 @@ __global__ __launch_bounds__(NT) void dense_inverse_kernel(const T* __restrict__
             }
         __syncthreads();
     }
-    if (inLds)
-        for (int e = tid; e < mm; e += NT) dst[e] = a[e];
 }
 
 // Largest unsigned value over the wave (DPP within rows of 16, then the four
@@ -391,10 +388,8 @@ void launch_dense_inverse(T* src, T* dst, int m, int* singular, hipStream_t s)
         return;
     }
     const size_t vecs = 2 * (size_t)m * sizeof(T) + (((size_t)m + 3) & ~size_t(3)) * sizeof(int);
-    const size_t full = vecs + (size_t)m * m * sizeof(T);
-    const bool inLds = full <= 64 * 1024;
     if (vecs > 64 * 1024) throw std::invalid_argument("dense leaf too large to invert");
-    dense_inverse_kernel<T, 512><<<1, 512, inLds ? full : vecs, s>>>(src, dst, m, inLds, singular);
+    dense_inverse_kernel<T, 512><<<1, 512, vecs, s>>>(src, dst, m, singular);
     HIP_LAUNCH_CHECK();
 }
 
