@@ -2,6 +2,7 @@
 // products, projections, dense-leaf accumulation, factor formation).
 #include <climits>
 #include <cstddef>
+#include "chunks.hpp"
 #include "kcommon.hpp"
 
 namespace dmhm {
@@ -455,8 +456,7 @@ struct MfUnit {
     T alpha, beta;
     int w, li, lk;
     int row0, col0, m, n;       // the unit's first row and column, the tile's extent
-    bool byChunk;               // S waves split chunks, not contributions
-    int turn;                   // chunks dealt so far (byChunk)
+    ChunkWalk<S> walk;          // byChunk: S waves split chunks, not contributions
     int64_t gcol[CB];           // offsets of the unit's columns in gathered right operands
     // lane records
     int64_t dl, dr;
@@ -499,25 +499,11 @@ struct MfUnit {
     {
         GPtr<T> L[RB], R[CB];
         int64_t ldl = 0, ldr = 0;
-        int q = 0, p = 0;
         T a = T(0);
+        walk.start();
         // Moves to the wave's next chunk; at the end it stays on the last one.
         auto next = [&]() -> bool {
-            const int last = p;
-            p += TAIL ? 16 : byChunk ? 16 * S : 16;
-            while (TAIL ? p >= q : p + 16 > q) {
-                if (left == 0) { p = last; return false; }
-                const int i = __builtin_ctzll(left);
-                left &= left - 1;
-                q = __builtin_amdgcn_readlane(dq, i);
-                if (TAIL) p = q & ~15;
-                else p = 0;
-                if (S > 1 && byChunk) {
-                    const int mine = (w - turn) & (S - 1);      // this wave's first chunk of the contribution
-                    turn += TAIL ? 1 : q >> 4;
-                    if (TAIL) p = mine == 0 ? p : q;
-                    else p = 16 * mine;
-                }
+            return walk.template next<TAIL>(left, [&](int i) { return __builtin_amdgcn_readlane(dq, i); }, [&](int i) {
                 const uint32_t meta = __builtin_amdgcn_readlane(dmeta, i);
                 const int fl = meta >> 24;
                 const float ca = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(dalpha), i));
@@ -529,14 +515,13 @@ struct MfUnit {
                                     row0, m, li, lk, L);
                 mf_lanes<T, PR, CB>((GPtr<T>)(b.template val<const T>((meta >> 8) & 255) + lane_i64(dr, i)), ldr,
                                     fl & CF_GATHER_R, gcol, col0, n, li, lk, R);
-            }
-            return true;
+            });
         };
         auto fetch = [&](Frag& f) {
             f.a = a;
-            f.qc = q - p;
-            mf_issue<T, PL, TAIL, RB>(L, ldl, p, f.qc, lk, f.l);
-            mf_issue<T, PR, TAIL, CB>(R, ldr, p, f.qc, lk, f.r);
+            f.qc = walk.q - walk.p;
+            mf_issue<T, PL, TAIL, RB>(L, ldl, walk.p, f.qc, lk, f.l);
+            mf_issue<T, PR, TAIL, CB>(R, ldr, walk.p, f.qc, lk, f.r);
         };
         auto use = [&](Frag& f) {
             mf_finish<T, PL, TAIL, RB>(f.l, row0, m, f.qc, li, lk);
@@ -582,7 +567,7 @@ struct MfUnit {
             f.a = (fl & CF_RUNTIME_ALPHA) ? alpha * T(ca) : (fl & CF_RUNTIME_BETA) ? beta * T(ca) : T(ca);
 #pragma unroll 1
             for (int p = 0; p < q; p += 16) {
-                if (S > 1 && byChunk && (turn++ & (S - 1)) != w) continue;
+                if (S > 1 && walk.byChunk && (walk.turn++ & (S - 1)) != w) continue;
 #pragma unroll
                 for (int s = 0; s < 4; ++s) {
                     const int k = p + mf_k<T>(s, lk), kc = min(k, q - 1);
@@ -634,7 +619,7 @@ struct MfUnit {
                 r = sl == SLOT_WIDTH ? b.rank(SLOT_WIDTH) : r;
                 dq = min(dq, r[dqrank]);
             }
-            const bool mine = in && dq > 0 && (S == 1 || byChunk || (lane & (S - 1)) == w);
+            const bool mine = in && dq > 0 && (S == 1 || walk.byChunk || (lane & (S - 1)) == w);
             const bool pl = dmeta >> 24 & CF_TRANS_L, pr = !(dmeta >> 24 & CF_TRANS_R);
             const bool any = (pl && !pr) || (RB > 1 && !pl && m < 2) || (CB > 1 && !pr && n < 2);
             const bool whole = mine && !any && dq >= 16, rest = mine && !any && (dq & 15);
@@ -659,7 +644,8 @@ __device__ __forceinline__ void mfma_body(const BV& b, const Tile& tl, const Con
     static_assert(S == 1 || S == 4, "one wave or the four waves of a workgroup per unit");
     const int row0 = ur * 16 * RB, col0 = uc * 16 * CB;
     const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
-    MfUnit<T, MODE, RB, CB, S, BV> u{b, alpha, beta, w, li, lk, row0, col0, 0, 0, S > 1 && tl.ce - tl.cb < S, 0};
+    MfUnit<T, MODE, RB, CB, S, BV> u{b, alpha, beta, w, li, lk, row0, col0, 0, 0,
+                                      {w, S > 1 && tl.ce - tl.cb < S}};
     // The first records' loads are in flight while the ranks are read.
     u.record(tl, cs, tl.cb);
     int m = tl.m, n = tl.k;
