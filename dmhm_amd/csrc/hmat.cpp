@@ -30,66 +30,21 @@ DevicePool& device_pool()
     return *p;
 }
 
-void* DevicePool::get(size_t bytes)
-{
-    bytes = (std::max<size_t>(bytes, 1) + 255) & ~size_t(255);
-    std::lock_guard<std::mutex> lk(mu_);
-    auto it = held_.lower_bound(bytes);
-    if (it != held_.end() && it->first - bytes <= bytes / 4) {
-        void* p = it->second;
-        holding_ -= it->first;
-        held_.erase(it);
-        return p;
-    }
-    void* p = raw(bytes);
-    size_[p] = bytes;
-    return p;
-}
-
-void* DevicePool::raw(size_t bytes)
+void* HipMemory::alloc(size_t bytes)
 {
     void* p = nullptr;
-    hipError_t e = hipMalloc(&p, bytes);
-    if (e == hipErrorOutOfMemory && !held_.empty()) {
+    const hipError_t e = hipMalloc(&p, bytes);
+    if (e == hipErrorOutOfMemory) {
         (void)hipGetLastError();
-        drop();
-        e = hipMalloc(&p, bytes);
+        return nullptr;
     }
     HIPCHECK(e);
     return p;
 }
 
-void* DevicePool::outside(size_t bytes)
-{
-    std::lock_guard<std::mutex> lk(mu_);
-    return raw(bytes);
-}
+void HipMemory::free(void* p) { (void)hipFree(p); }
 
-void DevicePool::put(void* p)
-{
-    std::lock_guard<std::mutex> lk(mu_);
-    const size_t bytes = size_.at(p);
-    if (g_lib.ready && bytes <= kBlockMax && holding_ + bytes <= kHoldMax) {
-        held_.emplace(bytes, p);
-        holding_ += bytes;
-        return;
-    }
-    size_.erase(p);
-    (void)hipFree(p);
-}
-
-void DevicePool::drop()
-{
-    for (auto& h : held_) { size_.erase(h.second); (void)hipFree(h.second); }
-    held_.clear();
-    holding_ = 0;
-}
-
-void DevicePool::trim()
-{
-    std::lock_guard<std::mutex> lk(mu_);
-    drop();
-}
+void HipMemory::short_of_memory() { throw Error(DMHM_ENOMEM, std::string("hipMalloc: ") + hipGetErrorString(hipErrorOutOfMemory)); }
 
 // Copies on the library stream and waits for them: the stream is created
 // non-blocking, so a plain hipMemcpy (null stream) would not be ordered after
@@ -1614,6 +1569,7 @@ int dmhm_init(int device)
         if (!g_lib.tuneEv) g_lib.tuneEv = new EventPair();
         g_lib.device = device;
         g_lib.ready = true;
+        device_pool().open();
     });
 }
 
@@ -1632,7 +1588,7 @@ int dmhm_finalize(void)
         (void)hipHostFree(g_lib.hReadback);
         (void)hipStreamDestroy(g_lib.stream);
         g_lib.ready = false;
-        device_pool().trim();
+        device_pool().close();
     });
 }
 

@@ -3,7 +3,6 @@
 // with their plan caches, device H-matrix storage, and the plan runner.
 #pragma once
 #include <hip/hip_runtime.h>
-#include <unordered_map>
 #include <cstdint>
 #include <functional>
 #include <map>
@@ -17,6 +16,7 @@
 #include "geometry.hpp"
 #include "kernels.hpp"
 #include "plan.hpp"
+#include "pool.hpp"
 
 namespace dmhm {
 
@@ -33,36 +33,12 @@ struct Error : std::runtime_error {
                         std::string(#x) + ": " + hipGetErrorString(e_));                  \
     } while (0)
 
-// ---------------------------------------------------------------------------
-// Library state: one device, one stream (default priority), a growing
-// workspace and per-geometry plan caches.
-// ---------------------------------------------------------------------------
-// Device memory of destroyed matrices and buffers, kept for the next ones: a
-// product or a copy per step of a user's loop otherwise pays hipMalloc and
-// hipFree (about 0.1 ms each, and a device synchronisation) every time. At most
-// kHoldMax bytes are held, in blocks of at most kBlockMax; a request takes the
-// smallest held block that is at most a quarter larger. All work of the library
-// is ordered on one stream, so a block's old users are done before its new
-// ones start. Everything held is freed by dmhm_finalize and before an
-// allocation is reported as failed. Batch of 24 products and applications
-// (FP32, 48^2 and 64^2): 22 ms
-// without, 12.4 with.
-class DevicePool {
-public:
-    void* get(size_t bytes);
-    void put(void* p);
-    void trim();
-    // Memory that is not pooled (hipFree gives it back), for plans' tables.
-    void* outside(size_t bytes);
-private:
-    void* raw(size_t bytes);
-    void drop();
-    static constexpr size_t kHoldMax = size_t(4) << 30, kBlockMax = size_t(2) << 30;
-    std::mutex mu_;
-    std::multimap<size_t, void*> held_;
-    std::unordered_map<void*, size_t> size_;    // every block handed out or held
-    size_t holding_ = 0;
+struct HipMemory {
+    static void* alloc(size_t bytes);
+    static void free(void* p);
+    [[noreturn]] static void short_of_memory();
 };
+using DevicePool = BlockPool<HipMemory>;
 DevicePool& device_pool();
 
 struct DeviceBuffer {
@@ -79,6 +55,10 @@ struct DeviceBuffer {
 
 struct GeoCtx;
 
+// ---------------------------------------------------------------------------
+// Library state: one device, one stream (default priority), a growing
+// workspace and per-geometry plan caches.
+// ---------------------------------------------------------------------------
 struct EventPair {
     hipEvent_t a = nullptr, b = nullptr;
     EventPair() { HIPCHECK(hipEventCreate(&a)); HIPCHECK(hipEventCreate(&b)); }
