@@ -74,6 +74,7 @@ _hp = ctypes.POINTER(ctypes.c_void_p)
 SIGNATURES = {
     "dmhm_init": (ctypes.c_int, [ctypes.c_int]),
     "dmhm_finalize": (ctypes.c_int, []),
+    "dmhm_trim": (ctypes.c_int, []),
     "dmhm_last_error": (ctypes.c_char_p, []),
     "dmhm_synchronize": (ctypes.c_int, []),
     "dmhm_build_natural_to_hierarchical_map": (ctypes.c_int, [ctypes.c_int, _ip, ctypes.c_int, _ip]),
@@ -201,3 +202,9 @@ def init(device=0):
     if not _initialized:
         check(load().dmhm_init(device))
         _initialized = True
+
+
+def trim():
+    """dmhm_trim: device memory held for the next matrices goes back to the
+    device, for other allocators of the process (torch's)."""
+    check(load().dmhm_trim())

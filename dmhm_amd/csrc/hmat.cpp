@@ -1594,6 +1594,11 @@ int dmhm_finalize(void)
 
 const char* dmhm_last_error(void) { return g_lastError.c_str(); }
 
+int dmhm_trim(void)
+{
+    return guard([&] { require_ready(); device_pool().trim(); });
+}
+
 int dmhm_synchronize(void)
 {
     return guard([&] { require_ready(); HIPCHECK(hipStreamSynchronize(g_lib.stream)); });

@@ -15,7 +15,7 @@ namespace dmhm {
 // kHoldMax bytes are held, in blocks of at most kBlockMax; a request takes the
 // smallest held block that is at most a quarter larger. All work of the library
 // is ordered on one stream, so a block's old users are done before its new
-// ones start. Everything held is given back by trim, by close
+// ones start. Everything held is given back by trim (dmhm_trim), by close
 // (dmhm_finalize) and before an allocation is reported as failed; a block that
 // outlives a close, whose device may then no longer be the library's, is given
 // back when it is put. Batch of 24 products and applications (FP32, 48^2 and

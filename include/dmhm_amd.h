@@ -55,6 +55,12 @@ typedef struct dmhm_hbatch_s* dmhm_hbatch;
  * RNG seeding are replaced by per-handle seeds). */
 int dmhm_init(int device);
 int dmhm_finalize(void);
+/* Gives device memory that the library holds for reuse back to the device
+ * (no counterpart in the reference). Destroyed matrices of up to 2 GiB leave
+ * at most 4 GiB in all allocated, for the next ones; the library gives it back
+ * by itself in dmhm_finalize and before one of its own allocations fails, but
+ * cannot see that another allocator in the process runs short. */
+int dmhm_trim(void);
 const char* dmhm_last_error(void);
 /* Device synchronisation point used by benchmarks. */
 int dmhm_synchronize(void);
@@ -105,6 +111,7 @@ int dmhm_hmat_create_from_csr(int dim, const int* sizes, int numLevels, int maxR
 int dmhm_hmat_create_zero(int dim, const int* sizes, int numLevels, int maxRank, int strong,
                           int precision, dmhm_hmat* out);
 
+/* The memory may be held for the next matrix (dmhm_trim). */
 int dmhm_hmat_destroy(dmhm_hmat h);
 
 typedef struct {
