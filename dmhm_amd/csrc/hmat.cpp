@@ -518,7 +518,12 @@ static void multiply_hmat_update(double alpha, dmhm_hmat_s* A, dmhm_hmat_s* B, d
     });
     ensure_ws(p, A->esize());
     // C_old is C itself: the plan reads each block's old factors before its SVD
-    // and formation phases write the new ones.
+    // and formation phases write the new ones. An operand that is C as well is
+    // read for other blocks too, after they are written: it is copied.
+    std::unique_ptr<dmhm_hmat_s> operand;
+    if (A->vals == C->vals || B->vals == C->vals) operand.reset(copy_hmat(C, C->prec));
+    if (A->vals == C->vals) A = operand.get();
+    if (B->vals == C->vals) B = operand.get();
     Bases b = bases_for(A, B, C, C->vals, nullptr);
     b.rank[SLOT_X] = C->ranks;
     TruncPolicy pol{o.tolMode, o.relTol};

@@ -186,7 +186,7 @@ int dmhm_hmat_multiply_hmat(double alpha, dmhm_hmat A, dmhm_hmat B, dmhm_hmat* C
 /* C := alpha A B + beta C, HMat2d::Multiply(alpha, B, beta, C)
  * (src/HMat2d/MultiplyHMat-incl.hpp:189-380). C keeps its geometry; every
  * admissible block of C is recompressed from a sketch of the exact
- * alpha A B + beta C restricted to it. */
+ * alpha A B + beta C restricted to it. A and B may be C (it is copied then). */
 int dmhm_hmat_multiply_hmat_update(double alpha, dmhm_hmat A, dmhm_hmat B, double beta, dmhm_hmat C,
                                    const dmhm_hh_opts* opts);
 

@@ -1,6 +1,6 @@
 """The update form C := alpha A B + beta C in place: against numpy where no
 block is truncated (rank(A B) + rank(C) at most maxRank), with C's subtrees cut
-into one workspace batch each. FP64, 1e-11 relative
+into one workspace batch each, and with C as an operand. FP64, 1e-11 relative
 to the entries summed: n roundings per product and the conditioning of a
 Gaussian sketch with four columns to spare."""
 import os
@@ -41,6 +41,17 @@ def check_update(sizes, levels, strong):
     C.UpdateWith(0.0, C.Copy())             # standard layout, as products have
     A.Multiply(-0.5, B, 2.0, C)
     assert close(C.to_dense(), -0.5 * a @ b + 2.0 * c, np.abs(a) @ np.abs(b) + np.abs(c)), (sizes, strong)
+
+
+@pytest.mark.parametrize("which", ["A", "B", "AB"])
+@pytest.mark.parametrize("case", CASES, ids=[str(c) for c in CASES])
+def test_operand_is_the_result(case, which):
+    (A, a), (C, c) = (operand(*case, s, 4) for s in range(2))
+    C.UpdateWith(0.0, C.Copy())
+    L, l = (C, c) if "A" in which else (A, a)
+    R, r = (C, c) if "B" in which else (A, a)
+    L.Multiply(-0.5, R, 2.0, C)
+    assert close(C.to_dense(), -0.5 * l @ r + 2.0 * c, np.abs(l) @ np.abs(r) + np.abs(c))
 
 
 def test_one_batch_per_subtree():
