@@ -2,12 +2,7 @@
 // kernel walks them; plain index arithmetic, shared with host code.
 #pragma once
 #include <cstdint>
-
-#ifdef __HIPCC__
-#define DMHM_HD __host__ __device__ inline __attribute__((always_inline))
-#else
-#define DMHM_HD inline
-#endif
+#include "hostdev.hpp"
 
 namespace dmhm {
 

@@ -15,31 +15,6 @@ namespace dmhm {
 // ---------------------------------------------------------------------------
 // KMAX bounds k (LDS sized for it); NT threads, TPP (a power of two <= 8)
 // per column pair.
-// Rotation (c, s) of a column pair with squared norms al, be and inner
-// product ga that makes the pair orthogonal: t = tan(theta) is the root of
-// t^2 + 2 zeta t - 1 = 0 of smaller magnitude, zeta = (be - al) / (2 ga),
-// written as t = sgn(d) g / (|d| + sqrt(d^2 + g^2)) with d = be - al and
-// g = 2 ga. t does not change when d and g are scaled together, so both are
-// scaled by an estimate of 1 / max(|d|, |g|) first (no overflow or underflow
-// in the squares). c = 1 / sqrt(1 + t^2), s = c t. t comes from the hardware
-// estimates (v_rcp_f64, v_rsq_f64) refined by one Newton step each, c by two:
-// an angle off by 1e-14 of itself leaves as little of the inner product, while
-// c^2 + s^2 = 1 to rounding for whatever t.
-__device__ inline void jacobi_rotation(double al, double be, double ga, double& cs, double& sn)
-{
-    const double d0 = be - al, g0 = 2.0 * ga;
-    const double rm = __builtin_amdgcn_rcp(fmax(fabs(d0), fabs(g0)));
-    const double dd = d0 * rm, gg = g0 * rm;
-    const double h = fma(dd, dd, gg * gg);
-    const double y = __builtin_amdgcn_rsq(h);
-    const double den = fabs(dd) + h * fma(0.5 * y, fma(-h * y, y, 1.0), y);
-    double r = __builtin_amdgcn_rcp(den);
-    r = fma(r, fma(-den, r, 1.0), r);
-    const double t = (dd >= 0.0 ? gg : -gg) * r;
-    cs = rsq_nr(fma(t, t, 1.0));
-    sn = cs * t;
-}
-
 template <typename T, int KMAX, int NT, int TPP = 8>
 __global__ void __launch_bounds__(NT) svd_kernel(Bases b, const SvdTask* __restrict__ tasks,
                                                  int tolMode, double relTol)
@@ -119,7 +94,7 @@ __global__ void __launch_bounds__(NT) svd_kernel(Bases b, const SvdTask* __restr
                     ga = group_sum<TPP>(ga);
                     if (ga * ga > 1e-30 * (al * be) && fabs(ga) > froTol) {
                         double cs, sn;
-                        jacobi_rotation(al, be, ga, cs, sn);
+                        jacobi_rotation<HwEst>(al, be, ga, cs, sn);
 #pragma unroll
                         for (int i = 0; i < RPT; ++i) {
                             const int r = sub + i * TPP;

@@ -9,6 +9,7 @@
 #include <stdexcept>
 #include <string>
 #include "kernels.hpp"
+#include "refine.hpp"
 
 namespace dmhm {
 
@@ -81,21 +82,14 @@ __device__ inline double bcast(double v, int l)
     return __hiloint2double(hi, lo);
 }
 
-// 1 / x and 1 / sqrt(x) from the hardware estimates (v_rcp_f64, v_rsq_f64) and
-// two Newton steps each: a shorter dependent chain than IEEE division and
-// square root, to rounding.
-__device__ inline double rcp_nr(double x)
-{
-    double r = __builtin_amdgcn_rcp(x);
-    r = fma(r, fma(-x, r, 1.0), r);
-    return fma(r, fma(-x, r, 1.0), r);
-}
-__device__ inline double rsq_nr(double x)
-{
-    double y = __builtin_amdgcn_rsq(x);
-    y = fma(0.5 * y, fma(-x * y, y, 1.0), y);
-    return fma(0.5 * y, fma(-x * y, y, 1.0), y);
-}
+// The hardware's estimates (v_rcp_f64, v_rsq_f64), and 1 / x and 1 / sqrt(x)
+// from them.
+struct HwEst {
+    static __device__ double rcp(double x) { return __builtin_amdgcn_rcp(x); }
+    static __device__ double rsq(double x) { return __builtin_amdgcn_rsq(x); }
+};
+__device__ inline double rcp_nr(double x) { return refined_rcp<HwEst>(x); }
+__device__ inline double rsq_nr(double x) { return refined_rsq<HwEst>(x); }
 
 template <typename T> struct VecOf;
 template <> struct VecOf<float> { typedef float type __attribute__((ext_vector_type(4))); };
