@@ -103,10 +103,13 @@ __global__ void __launch_bounds__(NT) svd_kernel(Bases b, const SvdTask* __restr
                                 Vs[p][r] = cs * vx[i] - sn * vy[i]; Vs[q][r] = sn * vx[i] + cs * vy[i];
                             }
                         }
-                        // A sweep of small rotations only is the last one: with
-                        // every cosine and sine at most 1e-8 before it, the
-                        // cosines left are of the order of their products.
-                        if (sub == 0 && (fabs(sn) > 1e-8 || ga * ga > 1e-16 * (al * be))) rotated = 1;
+                        // A sweep of rotations by at most tau, of pairs whose
+                        // cosine is at most tau, is the last one: a pair it made
+                        // orthogonal is met again by the 2 (k - 2) rotations of
+                        // its columns with others, each of which adds at most
+                        // 2 tau^2 to its cosine. tau = 2e-9 leaves 1e-15 at k =
+                        // 64, what a sweep without rotations would find.
+                        if (sub == 0 && (fabs(sn) > 2e-9 || ga * ga > 4e-18 * (al * be))) rotated = 1;
                     }
                 }
             }
