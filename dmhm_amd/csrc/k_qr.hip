@@ -228,13 +228,7 @@ __global__ void __launch_bounds__(64 * NWV) qr_split_kernel(Bases b, const QrTas
             const double alpha = bcast(xj, j & 63);
             double t = 0.0, scale = 0.0, beta = alpha;
             const double n2 = fma(alpha, alpha, xn2);
-            if (xn2 > 0.0 && n2 > kTinyColumn) {
-                // beta = -sgn(alpha) |column|, t = (beta - alpha) / beta, scale = 1 / (alpha - beta).
-                const double rs = rsq_nr(n2), nrm = n2 * rs;
-                beta = -copysign(nrm, alpha);
-                t = fma(fabs(alpha), rs, 1.0);
-                scale = copysign(rcp_nr(fabs(alpha) + nrm), alpha);
-            }
+            if (xn2 > 0.0 && n2 > kTinyColumn) householder<HwEst>(alpha, n2, t, scale, beta);
 #pragma unroll
             for (int r = 0; r < RR; ++r) {
                 const int i = lane + 64 * r;
@@ -410,13 +404,7 @@ __global__ void __launch_bounds__(KMAX * 8) qr_group_kernel(Bases b, const QrTas
             const double dot = group_sum<LPC>(xa[0] + xa[1]);
             double t = 0.0, scale = 0.0, beta = alpha;
             const double n2 = fma(alpha, alpha, xn2);
-            if (xn2 > 0.0 && n2 > kTinyColumn) {
-                // beta = -sgn(alpha) |column|, t = (beta - alpha) / beta, scale = 1 / (alpha - beta).
-                const double rs = rsq_nr(n2), nrm = n2 * rs;
-                beta = -copysign(nrm, alpha);
-                t = fma(fabs(alpha), rs, 1.0);
-                scale = copysign(rcp_nr(fabs(alpha) + nrm), alpha);
-            }
+            if (xn2 > 0.0 && n2 > kTinyColumn) householder<HwEst>(alpha, n2, t, scale, beta);
             const double d = fma(scale, dot, aj);       // v . (this column)
             if (c > j) {
                 const double f = t * d, fs = f * scale;

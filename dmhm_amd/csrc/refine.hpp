@@ -24,6 +24,26 @@ DMHM_HD double refined_rsq(double x)
     return fma(0.5 * y, fma(-x * y, y, 1.0), y);
 }
 
+// sqrt(x) for x > 0 from y, its refined reciprocal: x y is off by 3 u, the
+// residual x - s^2, exact to its rounding, takes that back to one rounding.
+DMHM_HD double refined_sqrt(double x, double y)
+{
+    const double s = x * y;
+    return fma(fma(-s, s, x), 0.5 * y, s);
+}
+
+// Householder reflector I - tau v v^T, v = (1, scale x), of a column (alpha, x)
+// of squared norm n2 = alpha^2 + x^T x: beta = -sgn(alpha) |column| (what it
+// makes of alpha), tau = (beta - alpha) / beta, scale = 1 / (alpha - beta).
+template <typename Est>
+DMHM_HD void householder(double alpha, double n2, double& tau, double& scale, double& beta)
+{
+    const double rs = refined_rsq<Est>(n2), nrm = refined_sqrt(n2, rs);
+    beta = -copysign(nrm, alpha);
+    tau = fma(fabs(alpha), rs, 1.0);
+    scale = copysign(refined_rcp<Est>(fabs(alpha) + nrm), alpha);
+}
+
 // Rotation (c, s) of a column pair with squared norms al, be and inner
 // product ga that makes the pair orthogonal: t = tan(theta) is the root of
 // t^2 + 2 zeta t - 1 = 0 of smaller magnitude, zeta = (be - al) / (2 ga),

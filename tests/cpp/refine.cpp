@@ -32,6 +32,17 @@ int main()
         bound("rcp", dmhm::refined_rcp<Est>(x), 1.0L / x, 1.01, x);
         // Half of the rounding of x y, half of that of its square, the last one.
         bound("rsq", dmhm::refined_rsq<Est>(x), 1.0L / sqrtl(x), 2.01, x);
+        // The residual's correction leaves the rounding of the sum alone.
+        bound("sqrt", dmhm::refined_sqrt(x, dmhm::refined_rsq<Est>(x)), sqrtl(x), 1.01, x);
+        // Reflector: beta one rounding; tau 2 u of a term of at most half of it
+        // and one rounding; scale beta's, the sum's and the reciprocal's.
+        const double alpha = std::sqrt(x) * unit(g);
+        double tau, scale, beta;
+        dmhm::householder<Est>(alpha, x, tau, scale, beta);
+        const long double b = -copysignl(sqrtl(x), alpha);
+        bound("beta", beta, b, 1.01, x);
+        bound("tau", tau, (b - alpha) / b, 2.02, x);
+        bound("scale", scale, 1.0L / (alpha - b), 3.03, x);
         // tan of the rotation: d (1), its scaling and g's (2), h (2), its root
         // (2 + 1), the sum (1), the reciprocal (1), the product (1).
         const double al = std::ldexp(mant(g), near(g)), be = std::ldexp(mant(g), near(g));
