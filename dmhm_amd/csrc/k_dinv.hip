@@ -289,15 +289,32 @@ __global__ void __launch_bounds__(1024) dense_inverse_panel_kernel(T* work, T* _
                     mine = max(mine, hi[r]);
                 }
                 const uint32_t mx = wave_max_u32(mine);
-                int p = -1;
+                uint64_t cand[RR];
+                int tied = 0;
 #pragma unroll
                 for (int r = 0; r < RR; ++r) {
-                    const uint64_t cand = __ballot(lane + 64 * r < m && hi[r] == mx) & ~used[r];
-                    if (p < 0 && cand) {
-                        p = 64 * r + __builtin_ctzll(cand);
-                        used[r] |= cand & (~cand + 1);
-                    }
+                    cand[r] = __ballot(lane + 64 * r < m && hi[r] == mx) & ~used[r];
+                    tied += __popcll(cand[r]);
                 }
+                if (tied > 1) {                 // equal to 20 bits: the low words decide
+                    uint32_t lo[RR];
+                    mine = 0;
+#pragma unroll
+                    for (int r = 0; r < RR; ++r) {
+                        lo[r] = (uint32_t)__double2loint(u[kk][r]);
+                        mine = cand[r] >> lane & 1 ? max(mine, lo[r]) : mine;
+                    }
+                    const uint32_t ml = wave_max_u32(mine);
+#pragma unroll
+                    for (int r = 0; r < RR; ++r) cand[r] &= __ballot(lo[r] == ml);
+                }
+                int p = -1;
+#pragma unroll
+                for (int r = 0; r < RR; ++r)
+                    if (p < 0 && cand[r]) {
+                        p = 64 * r + __builtin_ctzll(cand[r]);
+                        used[r] |= cand[r] & (~cand[r] + 1);
+                    }
                 p = __builtin_amdgcn_readfirstlane(p);
                 const double dd = at(u[kk], p);
                 const double inv = dd == 0.0 ? 0.0 : rcp_nr(dd);
