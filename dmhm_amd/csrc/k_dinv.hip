@@ -8,18 +8,9 @@
 
 namespace dmhm {
 
-// dst[d + e] = src[s + e] (copy) or dst[d + e] = 0 (fill, src unused) for
-// every range (s, d, len); blockIdx.y selects the range.
-template <typename T, bool FILL>
-__global__ void ranges_kernel(const T* __restrict__ src, T* __restrict__ dst, const CopyRange* __restrict__ rs)
-{
-    const CopyRange r = rs[blockIdx.y];
-    for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < r.len; e += (int64_t)gridDim.x * blockDim.x)
-        dst[r.dst + e] = FILL ? T(0) : src[r.src + e];
-}
-
-// The value ranges (blockIdx.y < nVal) and the rank ranges of one step in
-// one launch.
+// vals[d + e] = vals[s + e] (copy) or vals[d + e] = 0 (fill) for every range
+// (s, d, len) of one step, the value ranges (blockIdx.y < nVal) and the rank
+// ranges in one launch.
 template <typename T, bool FILL>
 __global__ void ranges2_kernel(T* __restrict__ vals, int* __restrict__ ranks, const CopyRange* __restrict__ rs, int nVal)
 {
@@ -44,18 +35,6 @@ void launch_arena_ranges(T* vals, int* ranks, const CopyRange* ranges, int nVal,
     const dim3 grid((unsigned)std::min<int64_t>((maxLen + 255) / 256, 2048), (unsigned)count);
     if (fill) ranges2_kernel<T, true><<<grid, 256, 0, s>>>(vals, ranks, ranges, nVal);
     else ranges2_kernel<T, false><<<grid, 256, 0, s>>>(vals, ranks, ranges, nVal);
-    HIP_LAUNCH_CHECK();
-}
-
-template <typename T>
-void launch_copy_ranges(const T* src, T* dst, const CopyRange* ranges, int count, int64_t maxLen, bool fill,
-                        hipStream_t s)
-{
-    if (count <= 0 || maxLen <= 0) return;
-    if (count > 65535) throw std::invalid_argument("too many ranges in one launch");
-    const dim3 grid((unsigned)std::min<int64_t>((maxLen + 255) / 256, 2048), (unsigned)count);
-    if (fill) ranges_kernel<T, true><<<grid, 256, 0, s>>>(src, dst, ranges);
-    else ranges_kernel<T, false><<<grid, 256, 0, s>>>(src, dst, ranges);
     HIP_LAUNCH_CHECK();
 }
 
@@ -411,11 +390,9 @@ void launch_dense_inverse(T* src, T* dst, int m, int* singular, hipStream_t s)
 }
 
 #define INST(T)                                                                                          \
-    template void launch_copy_ranges<T>(const T*, T*, const CopyRange*, int, int64_t, bool, hipStream_t); \
     template void launch_arena_ranges<T>(T*, int*, const CopyRange*, int, int, int64_t, bool, hipStream_t); \
     template void launch_dense_inverse<T>(T*, T*, int, int*, hipStream_t);
 INST(double)
 INST(float)
-template void launch_copy_ranges<int>(const int*, int*, const CopyRange*, int, int64_t, bool, hipStream_t);
 
 } // namespace dmhm

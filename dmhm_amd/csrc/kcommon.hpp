@@ -82,18 +82,12 @@ __device__ inline double bcast(double v, int l)
     return __hiloint2double(hi, lo);
 }
 
-// The hardware's estimates (v_rcp_f64, v_rsq_f64), and 1 / x and 1 / sqrt(x)
-// from them.
+// The hardware's estimates (v_rcp_f64, v_rsq_f64), and 1 / x from them.
 struct HwEst {
     static __device__ double rcp(double x) { return __builtin_amdgcn_rcp(x); }
     static __device__ double rsq(double x) { return __builtin_amdgcn_rsq(x); }
 };
 __device__ inline double rcp_nr(double x) { return refined_rcp<HwEst>(x); }
-__device__ inline double rsq_nr(double x) { return refined_rsq<HwEst>(x); }
-
-template <typename T> struct VecOf;
-template <> struct VecOf<float> { typedef float type __attribute__((ext_vector_type(4))); };
-template <> struct VecOf<double> { typedef double type __attribute__((ext_vector_type(2))); };
 
 // Grid of a grid-stride elementwise launch over n elements.
 inline int grid_for(int64_t n) { return (int)std::min<int64_t>((n + 255) / 256, 8192); }

@@ -21,7 +21,7 @@ struct TruncPolicy {
 // through LDS (vector FMA); TILE_MFMA, the wave-per-unit MFMA kernel in the
 // storage precision; TILE_MFMA_BF16, the same with FP32 operands rounded to
 // BF16 and FP32 accumulation (FP64 storage falls back to TILE_MFMA). The MFMA
-// kernel always prefetches; the _PF values name the same engines.
+// kernel has one form; the _PF values name the same engines.
 enum TileEngine { TILE_LDS = 0, TILE_MFMA = 1, TILE_MFMA_PF = 2, TILE_MFMA_BF16 = 3, TILE_MFMA_BF16_PF = 4,
                   TILE_ENGINES = 5 };
 template <typename T>
@@ -65,17 +65,15 @@ template <typename T> void launch_swap_lowrank(const T* src, T* dst, const int64
                                                hipStream_t s);
 void launch_permute_int(const int* src, int* dst, const int* perm, int count, hipStream_t s);
 
-// Direct inversion and merged plans (k_dinv.hip). Ranges are element ranges
-// of one allocation: dst[d + e] = src[s + e] for e < len.
+// Direct inversion (k_dinv.hip). Ranges are element ranges of one allocation:
+// x[dst + e] = x[src + e] for e < len.
 struct CopyRange { int64_t src, dst, len; };
-template <typename T> void launch_copy_ranges(const T* src, T* dst, const CopyRange* ranges, int count,
-                                              int64_t maxLen, bool fill, hipStream_t s);
 // Value ranges (the first nVal) and rank ranges of one allocation pair in one
 // launch; maxLen bounds every range's length.
 template <typename T> void launch_arena_ranges(T* vals, int* ranks, const CopyRange* ranges, int nVal, int nRank,
                                                int64_t maxLen, bool fill, hipStream_t s);
 // dst (m x m, ld m) = inverse of src (Gauss-Jordan, partial pivoting); a zero
-// pivot sets *singular (device int).
+// pivot sets *singular (device int). src is overwritten where m is 65 .. 256.
 template <typename T> void launch_dense_inverse(T* src, T* dst, int m, int* singular, hipStream_t s);
 
 // Vector utilities for the power iteration (EstimateTwoNorm).

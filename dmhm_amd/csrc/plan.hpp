@@ -276,7 +276,7 @@ struct PlanPart {
 Plan* merge_plans(const std::vector<PlanPart>& parts, bool segmentTiles = false);
 
 // Host-side bounds check of a plan that has not been uploaded: every operand,
-// output, QR panel, SVD factor, sketch panel and identity of every task lies
+// output, QR panel, SVD factor and sketch panel of every task lies
 // inside its slot (slotElems[slot] elements; SLOT_WS: the plan's workspace)
 // and every rank index inside rankElems[slot]. Returns an empty string or the
 // first violation.

@@ -639,7 +639,8 @@ class HBatch:
 
 def check_direct_invert_program(dim, sizes, num_levels, max_rank, strong, oversample=4):
     """Host only: lowers the direct inversion of a geometry at max_rank and
-    checks every task's bounds. Returns the program's counts."""
+    checks every task's bounds. Returns the program's counts (identity_phases
+    is 0: products form no identities)."""
     sz = np.zeros(3, dtype=np.int32)
     sz[:len(sizes)] = sizes
     st = np.zeros(7, dtype=np.int64)

@@ -310,7 +310,8 @@ int dmhm_hmat_direct_invert(dmhm_hmat h, const dmhm_hh_opts* opts);
 /* Host only (no GPU needed): lowers the direct inversion of a geometry at
  * rank maxRank and checks that every task of the program stays inside its
  * buffers. stats[7]: sub-matrix products, merged plans, steps, dense leaf
- * inversions, workspace elements, plan phases (launches), identity phases.
+ * inversions, workspace elements, plan phases (launches), 0 (products form
+ * no identities).
  * DMHM_EINVAL names the first violation. No reference counterpart. */
 int dmhm_check_direct_invert_program(int dim, const int* sizes, int numLevels, int maxRank, int strong,
                                      int oversample, long long* stats);
