@@ -273,8 +273,8 @@ template void run_plan<double>(Plan&, const Bases&, double, double, TruncPolicy,
 template void run_plan<float>(Plan&, const Bases&, float, float, TruncPolicy, uint64_t);
 
 // Workspace budget (elements) of one H*H batch: 2^33 (64 GiB in FP64) by
-// default, which keeps the 256^2 rank-16 product in 2-3 batches (103 ms FP64,
-// against 116 ms with 2^31 and 185 ms with 2^29); DMHM_HH_BATCH_ELEMS
+// default, which keeps the 256^2 rank-16 product in two batches (45.4 ms FP64,
+// against 47.6 ms with 2^31 and 61.7 ms with 2^29); DMHM_HH_BATCH_ELEMS
 // overrides it (plans built before a change keep theirs).
 int64_t hh_batch_budget()
 {

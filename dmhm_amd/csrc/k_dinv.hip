@@ -226,8 +226,9 @@ __global__ void __launch_bounds__(64 * NWV) dense_inverse_split_kernel(const T* 
 // write of each. One step per pass over the matrix, as dense_inverse_kernel
 // takes, is bound by that traffic through one CU. Direct inversion of 88^2 in
 // leaves of 121 points (FP64, rank 8): 89.7 -> 22.2 ms, of 120^2 in leaves of
-// 225 points 415 -> 117 ms (290 ms with panels of 8 at four rows a lane, which
-// spill; 128 ms with 8 columns and 8 waves).
+// 225 points 415 -> 117 ms (290 ms with panels of 8 at four rows a lane, 128 ms
+// with 8 columns and 8 waves; in panels of 4 too the compiler keeps 144 bytes
+// per lane of the four rows' arrays in scratch).
 template <typename T, int RR>
 __global__ void __launch_bounds__(1024) dense_inverse_panel_kernel(T* work, T* __restrict__ dst, int m,
                                                                    int* __restrict__ singular)

@@ -305,9 +305,18 @@ __global__ void __launch_bounds__(64 * NW) mv_acc_kernel(Bases b, const MvAtom* 
     }
 }
 
-// Waves per atom: four fill the chip from 768 atoms on (1,024 atoms of the
-// 256^2 matrix, FP32: 80.0 us with four, 78.6 with eight); 448 atoms of the 3D
-// 27 x 33 x 30 one (six vectors): 192 us with eight, 159 with sixteen.
+// Waves per atom, by the number of atoms. Whole calls with 4, 8 and 16 waves,
+// mean over both directions, both precisions, one and six vectors, in us:
+//   2D, rank 16:   256 atoms (128^2) 68.4 63.1 62.6; 512 (150^2) 103.3 103.5
+//   104.4; 768 (200^2) 174.5 180.3 178.5; 1,024 (256^2) 237.9 238.0 248.2;
+//   2,048 (300^2, rank 8) 292 307 330;
+//   3D, rank 16:   440 (27 x 33 x 30) 346 306 277; 512 (32^3) 409 368 361; 664
+//   (34 x 36 x 33) 643 577 552; 768 (36^3) 806 758 730; 944 1141 1099 1088;
+//   1,024 (40^3) 1294 1246 1242.
+// From 768 on the 2D matrices gain from four; the 3D ones, whose atoms carry
+// several times the records, would still gain 4 to 10% from sixteen there.
+// (H^T with 7 and 8 vectors and sixteen waves keeps 6 to 29 of its registers in
+// scratch.)
 static int mv_waves(int atoms) { return atoms >= 768 ? 4 : 16; }
 
 template <typename T, int K, bool TR>

@@ -9,11 +9,12 @@ namespace dmhm {
 // G2 = U (same), both k x cap, and the kept rank. The rotations act on the
 // columns of R^T (the rows of the triangular R): Jacobi on the transposed
 // triangular factor of a QR converges in fewer sweeps (7-8 against 10-15 on
-// sketch factors of decaying spectra, 20 columns). With R^T W = A (columns
+// sketch factors of decaying spectra, 20 columns, counting a last one without
+// rotations). With R^T W = A (columns
 // of A orthogonal, norms s), R = W S (A/s)^T: G1 = A and G2 = W, and no
 // column is divided by its norm.
 // ---------------------------------------------------------------------------
-// KMAX bounds k (LDS sized for it); NT threads, TPP (a power of two <= 8)
+// KMAX bounds k (LDS sized for it); NT threads, TPP (a power of two <= 16)
 // per column pair.
 template <typename T, int KMAX, int NT, int TPP = 8>
 __global__ void __launch_bounds__(NT) svd_kernel(Bases b, const SvdTask* __restrict__ tasks,
@@ -187,12 +188,12 @@ void launch_svd_phase(const Phase& ph, const Bases& b, TruncPolicy pol, hipStrea
     // 24-column factors: 16 threads per column pair for phases of few factors
     // (one workgroup per CU, the time is one factor's latency), 8 threads
     // beyond (a 256^2 inversion's SVDs: 55.1 ms with the line at 256 factors,
-    // 54.6 at 1,024). A factor of k = 20 takes 3 to 5 sweeps of about 1,450
-    // cycles per round: the reads, the three sums over a pair's threads, the
-    // rotation's dependent chain, the writes and a barrier. 55 us per launch of
-    // few factors and 108 us for 850; 74 and 134 us with one thread sorting the
-    // columns (43,000 of 150,000 cycles), two Newton steps per estimate and a
-    // last sweep without rotations.
+    // 54.6 at 1,024). A factor of k = 20 takes 4 or 5 sweeps (32,000 of a 256^2
+    // product; 1 to 4 in a 64^2 inversion, k = 12) of about 1,450 cycles per
+    // round: the reads, the three sums over a pair's threads, the rotation's
+    // dependent chain, the writes and a barrier. 57 us per launch of few factors
+    // and 108 us for 850; 74 and 134 us with one thread sorting the columns
+    // (43,000 of 150,000 cycles) and a last sweep without rotations.
     if (ph.svdK <= 24 && n < kSvdLatencyTasks) svd_kernel<T, 24, 192, 16><<<n, 192, 0, s>>>(b, t, pol.tolMode, pol.relTol);
     else if (ph.svdK <= 24) svd_kernel<T, 24, 128, 8><<<n, 128, 0, s>>>(b, t, pol.tolMode, pol.relTol);
     else if (ph.svdK <= 40) svd_kernel<T, 40, 192><<<n, 192, 0, s>>>(b, t, pol.tolMode, pol.relTol);

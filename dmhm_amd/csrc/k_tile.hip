@@ -258,8 +258,9 @@ __global__ void __launch_bounds__(256) tile_seg_kernel(Bases b, const TileSeg* _
 // row block b of a pair takes the rows of parity b. Rows and columns outside
 // the tile are clamped to its last one (their results are never stored);
 // inner indices outside the contribution are read at its last one and zeroed.
-// Loads of the next chunk (possibly of the next contribution) are issued
-// before the MFMAs of the current one, into the other of two register sets.
+// Loads of the next chunk (possibly of the next contribution) are written
+// before the MFMAs of the current one, into the other of two register sets
+// (MfUnit::run says what the compiler keeps of that).
 //
 // Contribution records and run-time ranks are read 64 at a time, one per
 // lane, and handed out by lane reads: two memory latencies per 64
@@ -531,10 +532,12 @@ struct MfUnit {
         Frag f0, f1;
         if (!next()) return;
         fetch(f0);
-        // After the last chunk the fetch repeats it: loads on every path keep
-        // the wait before use(f) at "all but the newest chunk" (a fetch under
-        // a branch made it "all", 62 against 50 ms per 256^2 FP64 product),
-        // and one use per register set keeps one set of accumulators.
+        // After the last chunk the fetch repeats it, so that no fetch is under a
+        // branch (a fetch under one, 62 against 50 ms per 256^2 FP64 product),
+        // and one use per register set keeps one set of accumulators. The
+        // compiler overlaps one half of the loop only: the wait before use(f1)
+        // leaves f0's loads in flight, but f1's, which nothing needs once the
+        // loop ends, it moves behind use(f0) and the first exit.
         while (true) {
             const bool more1 = next();
             fetch(f1);

@@ -107,7 +107,7 @@ struct MvProjItem {
     int32_t ldv, rows;
     int32_t rankIdx, cap;
 };
-// Rows from which a projection takes a workgroup instead of a wave.
+// A projection of more rows takes a workgroup instead of a wave.
 constexpr int kMvBigRows = 512;
 struct MvAtom {
     int64_t yrow;
