@@ -2420,6 +2420,10 @@ int dmhm_hmat_matvec_bytes(dmhm_hmat h, int k, double* bytes, double* flops)
 namespace dmhm {
 void Plan::upload()
 {
+    if (!gtab.empty()) {
+        dGather = device_pool().outside(gtab.size() * sizeof(int64_t));
+        HIPCHECK(copy_sync(dGather, gtab.data(), gtab.size() * sizeof(int64_t), hipMemcpyHostToDevice));
+    }
     for (auto& ph : phases) {
         if (!ph.segSrc.empty()) {
             // Segment table of a merged tile phase: the members' source
@@ -2460,10 +2464,7 @@ void Plan::upload()
             HIPCHECK(copy_sync(ph.dContribs, ph.contribs.data(), ph.contribs.size() * sizeof(Contrib),
                                hipMemcpyHostToDevice));
         }
-        if (!ph.gtab.empty()) {
-            ph.dGather = device_pool().outside(ph.gtab.size() * sizeof(int64_t));
-            HIPCHECK(copy_sync(ph.dGather, ph.gtab.data(), ph.gtab.size() * sizeof(int64_t), hipMemcpyHostToDevice));
-        }
+        if (ph.gtab) ph.dGather = dGather;
         const void* src = nullptr; size_t bytes = 0;
         if (ph.kind == PH_QR && !ph.qr.empty()) {
             // Sort the (independent) tasks by panel class: register-resident
@@ -2526,11 +2527,9 @@ void Plan::upload()
         }
         // Host copies of the big arrays are no longer needed (unless merged
         // plans will be checked against them).
-        if (!keepHost) {
-            std::vector<Contrib>().swap(ph.contribs);
-            std::vector<int64_t>().swap(ph.gtab);
-        }
+        if (!keepHost) std::vector<Contrib>().swap(ph.contribs);
     }
+    if (!keepHost) std::vector<int64_t>().swap(gtab);
 }
 
 void Plan::release()
@@ -2541,8 +2540,10 @@ void Plan::release()
         if (ph.dTasks) (void)hipFree(ph.dTasks);
         if (ph.dAux) (void)hipFree(ph.dAux);
         if (ph.dSegs) (void)hipFree(ph.dSegs);
-        if (ph.dGather) (void)hipFree(ph.dGather);
-        ph.dTiles = ph.dContribs = ph.dTasks = ph.dAux = ph.dSegs = ph.dGather = nullptr;
+        ph.dTiles = ph.dContribs = ph.dTasks = ph.dAux = ph.dSegs = nullptr;
+        ph.dGather = nullptr;
     }
+    if (dGather) (void)hipFree(dGather);
+    dGather = nullptr;
 }
 } // namespace dmhm

@@ -54,8 +54,8 @@ __device__ __forceinline__ int contrib_q(const BV& b, const Contrib& C)
 }
 
 template <typename T, int MR, int NC, int QC, int LN, int RN, typename BV>
-__device__ __forceinline__ void tile_load(const BV& b, const Contrib& C, const int64_t* __restrict__ gt, int p0, int q,
-                                          int m, int k, T alpha, T beta, T (&lr)[LN], T (&rr)[RN], T& a)
+__device__ __forceinline__ void tile_load(const BV& b, const Tile& tl, const Contrib& C,
+                                          const int64_t* __restrict__ gtab, int p0, int q, int m, int k, T alpha, T beta, T (&lr)[LN], T (&rr)[RN], T& a)
 {
     const int tid = threadIdx.x;
     const int qc = min(QC, q - p0);
@@ -78,7 +78,7 @@ __device__ __forceinline__ void tile_load(const BV& b, const Contrib& C, const i
         int jj, pp;
         if (!tR) { pp = e % QC; jj = e / QC; } else { jj = e % NC; pp = e / NC; }
         const bool ok = e < QC * NC && jj < k && pp < qc;
-        rr[u] = ok ? (!tR ? R[(p0 + pp) + (gR ? gt[jj] : (int64_t)jj * C.ldr)] : R[jj + (int64_t)(p0 + pp) * C.ldr])
+        rr[u] = ok ? (!tR ? R[(p0 + pp) + (gR ? gather_column(tl, gtab, jj) : (int64_t)jj * C.ldr)] : R[jj + (int64_t)(p0 + pp) * C.ldr])
                    : T(0);
     }
 }
@@ -113,7 +113,6 @@ template <typename T, int MR, int NC, int TM, int TN, typename BV>
 __device__ __forceinline__ void tile_body(const BV& b, const Tile& tl, const Contrib* __restrict__ cs,
                                           const int64_t* __restrict__ gtab, T alpha, T beta)
 {
-    const int64_t* __restrict__ gt = gtab + tl.gather;      // read for gathered contributions only
     constexpr int QC = TileCfg<T, MR>::QC;
     constexpr int RT = MR / TM;
     static_assert(RT * (NC / TN) == 256, "the thread grid must cover 256 threads");
@@ -143,7 +142,7 @@ __device__ __forceinline__ void tile_body(const BV& b, const Tile& tl, const Con
     uint8_t flags = 0;
     if (c < tl.ce) {
         const Contrib C = cs[c];
-        tile_load<T, MR, NC, QC, LN, RN>(b, C, gt, p0, q, m, k, alpha, beta, lr, rr, a);
+        tile_load<T, MR, NC, QC, LN, RN>(b, tl, C, gtab, p0, q, m, k, alpha, beta, lr, rr, a);
         flags = C.flags;
     }
     int buf = 0;
@@ -161,7 +160,7 @@ __device__ __forceinline__ void tile_body(const BV& b, const Tile& tl, const Con
         }
         if (c < tl.ce) {
             const Contrib C = cs[c];
-            tile_load<T, MR, NC, QC, LN, RN>(b, C, gt, p0, q, m, k, alpha, beta, lr, rr, a);
+            tile_load<T, MR, NC, QC, LN, RN>(b, tl, C, gtab, p0, q, m, k, alpha, beta, lr, rr, a);
             flags = C.flags;
         }
         const T* __restrict__ Lb = Ls[buf];
@@ -426,7 +425,7 @@ struct MfFrag {
 typedef uint32_t mf_u2 __attribute__((ext_vector_type(2), aligned(8)));
 typedef uint32_t mf_u4 __attribute__((ext_vector_type(4), aligned(8)));
 static_assert(sizeof(Tile) == 56 && offsetof(Tile, k) == 16 && offsetof(Tile, koff) == 32 &&
-              offsetof(Tile, gather) == 48 && offsetof(Tile, slot) == 44, "tile record layout");
+              offsetof(Tile, gather) == 48 && offsetof(Tile, gcols) == 52 && offsetof(Tile, slot) == 44, "tile record layout");
 static_assert(sizeof(Contrib) == 40 && offsetof(Contrib, ldl) == 16 && offsetof(Contrib, lslot) == 32 &&
               offsetof(Contrib, flags) == 35, "contribution record layout");
 __device__ __forceinline__ int64_t mf_i64(uint32_t lo, uint32_t hi) { return (int64_t)((uint64_t)hi << 32 | lo); }
@@ -435,10 +434,11 @@ __device__ __forceinline__ Tile mf_tile(const Tile* __restrict__ p)
     const mf_u4* v = reinterpret_cast<const mf_u4*>(p);
     const mf_u4 a = v[0], b = v[1], c = v[2];
     Tile t;
-    t.gather = (int)reinterpret_cast<const mf_u2*>(p)[6][0];
+    const mf_u2 d = reinterpret_cast<const mf_u2*>(p)[6];
     t.off = mf_i64(a[0], a[1]); t.ld = (int)a[2]; t.m = (int)a[3];
     t.k = (int)b[0]; t.mrank = (int)b[1]; t.krank = (int)b[2]; t.moff = (int)b[3];
     t.koff = (int)c[0]; t.cb = (int)c[1]; t.ce = (int)c[2];
+    t.gather = (int)d[0]; t.gcols = (int)d[1];
     t.slot = (uint8_t)c[3]; t.mslot = (uint8_t)(c[3] >> 8); t.kslot = (uint8_t)(c[3] >> 16);
     t.flags = (uint8_t)(c[3] >> 24);
     return t;
@@ -659,7 +659,7 @@ __device__ __forceinline__ void mfma_body(const BV& b, const Tile& tl, const Con
     u.n = n;
 #pragma unroll
     for (int cb = 0; cb < CB; ++cb)
-        u.gcol[cb] = tl.gather >= 0 ? gtab[tl.gather + min(col0 + mf_row<CB>(cb, li), n - 1)] : 0;
+        u.gcol[cb] = tl.gather >= 0 ? gather_column(tl, gtab, min(col0 + mf_row<CB>(cb, li), n - 1)) : 0;
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb)
 #pragma unroll

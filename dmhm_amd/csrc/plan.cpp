@@ -45,30 +45,37 @@ void order_tiles(Phase& ph)
     ph.nLong = 0;
     const int rb = ph.maxMTile <= 16 ? 16 : 32, cb = ph.maxKTile <= 16 ? 16 : 32;
     const double units = (double)((ph.maxMTile + rb - 1) / rb) * ((ph.maxKTile + cb - 1) / cb);
-    auto chunks = [&](const Tile& t) {
+    std::vector<int64_t> chunks;
+    chunks.reserve(ph.tiles.size());
+    double total = 0;
+    for (const Tile& t : ph.tiles) {
         int64_t n = 0;
         for (int c = t.cb; c < t.ce; ++c) n += (ph.contribs[c].q + 15) >> 4;
-        return n;
-    };
-    double total = 0;
-    for (const Tile& t : ph.tiles) total += (double)chunks(t) * units;
+        chunks.push_back(n);
+        total += (double)n * units;
+    }
     const int64_t lim = std::max<int64_t>(8, (int64_t)(total / kTileWaves / 2));
     // Class 0: long; then by powers of four of the chunk count.
-    std::vector<std::vector<Tile>> cls(1);
-    for (const Tile& t : ph.tiles) {
-        const int64_t n = chunks(t);
+    auto cls = [&](int64_t n) {
         size_t c = 0;
         if (n <= lim)
             for (c = 1; (n << (2 * c)) <= lim && n > 0; ++c) {}
-        if (cls.size() <= c) cls.resize(c + 1);
-        cls[c].push_back(t);
+        return c;
+    };
+    std::vector<size_t> first;                  // of each class
+    for (int64_t n : chunks) {
+        const size_t c = cls(n) + 1;
+        if (first.size() <= c) first.resize(c + 1);
+        ++first[c];
     }
-    ph.nLong = (int)cls[0].size();
+    ph.nLong = first.size() > 1 ? (int)first[1] : 0;
+    for (size_t c = 1; c < first.size(); ++c) first[c] += first[c - 1];
     int64_t by32 = 0, by64 = 0;                 // 16-column blocks in units of 32 and of 64 columns
     for (const Tile& t : ph.tiles) { by32 += (t.k + 31) / 32 * 2; by64 += (t.k + 63) / 64 * 4; }
     ph.wide = 8 * by64 <= 9 * by32;
-    ph.tiles.clear();
-    for (auto& v : cls) ph.tiles.insert(ph.tiles.end(), v.begin(), v.end());
+    std::vector<Tile> sorted(ph.tiles.size());
+    for (size_t i = 0; i < ph.tiles.size(); ++i) sorted[first[cls(chunks[i])]++] = ph.tiles[i];
+    ph.tiles.swap(sorted);
 }
 
 static Contrib mkc(uint8_t lslot, int64_t loff, int ldl, uint8_t rslot, int64_t roff, int ldr,
@@ -138,7 +145,7 @@ void Planner::subh(PhaseBuilder& proj, PhaseBuilder& acc, uint8_t mslot, const L
                     else
                         acc.add(tile, mkc(mslot, D + (int64_t)ra * m, m, in.slot, roff, in.ld, m, -1, 0,
                                           cflags | CF_TRANS_L | gflag, alpha));
-                    if (gathered) acc.setGather(tile, in.gather + 64 * c);
+                    if (gathered) acc.setGather(tile, in.gather, in.gcols);
                 }
                 if (flops) *flops += 2.0 * g_.atomSize[a] * (trans ? m : n) * k;
             }
@@ -161,7 +168,7 @@ void Planner::subh(PhaseBuilder& proj, PhaseBuilder& acc, uint8_t mslot, const L
                     t.m = std::min(64, cap - 64 * rc); t.mrank = li2; t.moff = 64 * rc; t.mslot = mslot;
                     t.k = std::min(64, k - 64 * c); t.krank = krank; t.koff = 64 * c; t.kslot = kslot;
                     t.slot = SLOT_WS; t.flags = 0;
-                    if (gathered) t.gather = in.gather + 64 * c;
+                    if (gathered) { t.gather = in.gather; t.gcols = in.gcols; }
                     const int tile = proj.addTile(t);
                     for (int a = colB.atomBegin; a < colB.atomEnd; ++a) {
                         const int ra = g_.atomStart[a] - colB.off;
@@ -745,7 +752,7 @@ Plan* Planner::hhProduct(const Layout& LA, const Layout& LB, const Layout& LC, i
         // are stacked: one sub-H product of width cap * n, whose input panel is
         // their stored factors side by side, computes all their exact factors
         // at once (wider tiles, fewer contributions). The panel is not formed:
-        // the products read its columns through a table of their offsets.
+        // the products read its columns through a table of the factors' offsets.
         // (Copying the factors into it first cost 5.7 of 62 ms per 256^2
         // rank-16 FP64 product and 1.3 of 13 ms per FP32 3D update, and the
         // copies, 15 GB against 1.5 GB of stored factors, were then read from
@@ -755,7 +762,7 @@ Plan* Planner::hhProduct(const Layout& LA, const Layout& LB, const Layout& LC, i
             p1.role = 1;
             Phase& a1 = newPhase(PH_TILE);
             PhaseBuilder proj(p1), acc(a1);
-            std::vector<int64_t> gtab;
+            std::vector<int64_t>& gtab = plan->gtab;
             std::map<std::pair<int, int>, std::vector<int>> stacks;
             std::vector<std::pair<int, int>> order;
             for (size_t i = 0; i < wPending.size(); ++i) {
@@ -791,23 +798,23 @@ Plan* Planner::hhProduct(const Layout& LA, const Layout& LB, const Layout& LC, i
                 const Box& outB = g.boxes[wf0.level][outBoxId];
                 const int64_t OUT = wsAlloc((int64_t)outB.size * cap * n);
                 const int tab = (int)gtab.size();
+                gtab.push_back(inB.size);
                 for (int i = 0; i < n; ++i) {
                     const Pending& wp = wPending[idx[i]];
                     const Block& lr = g.blocks[left ? wp.bA : wp.bB];
                     const int li = lr.lrIndex;
                     const int64_t src = left ? LA.vOff[li] : LB.uOff[li];
-                    for (int c = 0; c < cap; ++c) gtab.push_back(src + (int64_t)c * inB.size);
+                    gtab.push_back(src);
                     WFactor& w = W[wp.wIndex];
                     if (left) w.PV.off = OUT + (int64_t)i * cap * outB.size;
                     else w.PU.off = OUT + (int64_t)i * cap * outB.size;
                 }
                 PanelTiles pt = addPanelTiles(acc, {SLOT_WS, OUT, outB.size}, wf0.level, outBoxId, cap * n, -1, 0, 0);
                 subh(proj, acc, left ? SLOT_B : SLOT_A, left ? LB : LA, left ? w0.bB : w0.bA, left,
-                     {left ? SLOT_A : SLOT_B, 0, inB.size, tab}, inLevel, inBoxId, pt, cap * n, -1, 0, 1.0f, 0,
+                     {left ? SLOT_A : SLOT_B, 0, inB.size, tab, cap}, inLevel, inBoxId, pt, cap * n, -1, 0, 1.0f, 0,
                      &plan->flops);
             }
-            p1.gtab = gtab;
-            a1.gtab = std::move(gtab);
+            p1.gtab = a1.gtab = &gtab;
             proj.finalize();
             acc.finalize();
         }
@@ -1013,12 +1020,15 @@ Plan* merge_plans(const std::vector<PlanPart>& parts, bool segmentTiles)
     std::unique_ptr<Plan> out(new Plan());
     const size_t np = parts.size();
     std::vector<int64_t> wsBase(np);
+    std::vector<int> gatherBase(np);
     int64_t ws = 0;
     for (size_t i = 0; i < np; ++i) {
         wsBase[i] = ws;
         ws += (parts[i].plan->wsElems + 63) & ~int64_t(63);
         out->flops += parts[i].plan->flops;
         out->batches = std::max(out->batches, parts[i].plan->batches);
+        gatherBase[i] = (int)out->gtab.size();
+        if (!segmentTiles) out->gtab.insert(out->gtab.end(), parts[i].plan->gtab.begin(), parts[i].plan->gtab.end());
     }
     out->wsElems = ws;
     // Shifts of part i: the workspace slot goes to the part's region.
@@ -1061,8 +1071,8 @@ Plan* merge_plans(const std::vector<PlanPart>& parts, bool segmentTiles)
                     m.maxMTile = std::max(m.maxMTile, ph.maxMTile);
                     break;
                 }
-                const int cbase = (int)m.contribs.size(), gbase = (int)m.gtab.size();
-                m.gtab.insert(m.gtab.end(), ph.gtab.begin(), ph.gtab.end());
+                const int cbase = (int)m.contribs.size(), gbase = gatherBase[i];
+                if (ph.gtab) m.gtab = &out->gtab;
                 for (Tile t : ph.tiles) {
                     t.off += vsh(i, t.slot);
                     t.mrank = rsh(i, t.mslot, t.mrank);
@@ -1148,6 +1158,26 @@ Plan* merge_plans(const std::vector<PlanPart>& parts, bool segmentTiles)
     return out.release();
 }
 
+// The table holds the factors that a tile's columns belong to.
+static bool gatherOk(const Phase& ph, const Tile& t)
+{
+    return t.gather >= 0 && t.gcols > 0 && ph.gtab &&
+           t.gather + 1 + (int64_t)(t.koff + t.k - 1) / t.gcols < (int64_t)ph.gtab->size() && (*ph.gtab)[t.gather] > 0;
+}
+
+// Lowest and highest start of a tile's gathered columns (those of one factor
+// ascend).
+static std::pair<int64_t, int64_t> gatherRange(const Phase& ph, const Tile& t)
+{
+    std::pair<int64_t, int64_t> r(INT64_MAX, INT64_MIN);
+    for (int j = 0, end; j < t.k; j = end) {
+        end = std::min(t.k, j + t.gcols - (t.koff + j) % t.gcols);
+        r.first = std::min(r.first, gather_column(t, ph.gtab->data(), j));
+        r.second = std::max(r.second, gather_column(t, ph.gtab->data(), end - 1));
+    }
+    return r;
+}
+
 std::string check_plan(const Plan& p, const int64_t* slotElems, const int64_t* rankElems)
 {
     auto size = [&](int slot) { return slot == SLOT_WS ? p.wsElems : slotElems[slot]; };
@@ -1169,6 +1199,8 @@ std::string check_plan(const Plan& p, const int64_t* slotElems, const int64_t* r
             if (!inside(t.slot, t.off + vs[t.slot], t.ld, t.m, t.k)) return where(i, "tile output out of bounds");
             if (!rk(t.mslot, t.mrank) || !rk(t.kslot, t.krank)) return where(i, "tile rank index");
             if (t.cb < 0 || t.ce > (int)ph.contribs.size() || t.cb > t.ce) return where(i, "tile contribution range");
+            const bool gathered = gatherOk(ph, t);
+            const std::pair<int64_t, int64_t> cols = gathered ? gatherRange(ph, t) : std::pair<int64_t, int64_t>();
             for (int q = t.cb; q < t.ce; ++q) {
                 const Contrib& c = ph.contribs[q];
                 const bool tl = c.flags & CF_TRANS_L, tr = c.flags & CF_TRANS_R;
@@ -1176,8 +1208,8 @@ std::string check_plan(const Plan& p, const int64_t* slotElems, const int64_t* r
                 const bool okL = tl ? inside(c.lslot, lo, c.ldl, c.q, t.m) : inside(c.lslot, lo, c.ldl, t.m, c.q);
                 bool okR = true;
                 if (c.flags & CF_GATHER_R) {
-                    okR = !tr && t.gather >= 0 && t.gather + (int64_t)t.k <= (int64_t)ph.gtab.size();
-                    for (int j = 0; j < t.k && okR; ++j) okR = inside(c.rslot, ro + ph.gtab[t.gather + j], c.q, c.q, 1);
+                    okR = !tr && gathered && inside(c.rslot, ro + cols.first, c.q, c.q, 1) &&
+                          inside(c.rslot, ro + cols.second, c.q, c.q, 1);
                 } else okR = tr ? inside(c.rslot, ro, c.ldr, t.k, c.q) : inside(c.rslot, ro, c.ldr, c.q, t.k);
                 if (!okL) return where(i, "left operand out of bounds");
                 if (!okR) return where(i, "right operand out of bounds");
@@ -1213,14 +1245,16 @@ std::string check_plan(const Plan& p, const int64_t* slotElems, const int64_t* r
             rank(t.mslot, t.mrank);
             rank(t.kslot, t.krank);
             if (t.cb < 0 || t.ce > (int)ph.contribs.size() || t.cb > t.ce) { f.bad = true; continue; }
+            const bool gathered = gatherOk(ph, t);
+            const std::pair<int64_t, int64_t> cols = gathered ? gatherRange(ph, t) : std::pair<int64_t, int64_t>();
             for (int q = t.cb; q < t.ce; ++q) {
                 const Contrib& x = ph.contribs[q];
                 const bool tl = x.flags & CF_TRANS_L, tr = x.flags & CF_TRANS_R;
                 if (tl) region(x.lslot, x.loff, x.ldl, x.q, t.m); else region(x.lslot, x.loff, x.ldl, t.m, x.q);
                 if (x.flags & CF_GATHER_R) {
-                    if (tr || t.gather < 0 || t.gather + (int64_t)t.k > (int64_t)ph.gtab.size()) f.bad = true;
-                    else
-                        for (int j = 0; j < t.k; ++j) region(x.rslot, x.roff + ph.gtab[t.gather + j], x.q, x.q, 1);
+                    if (tr || !gathered) { f.bad = true; continue; }
+                    region(x.rslot, x.roff + cols.first, x.q, x.q, 1);
+                    region(x.rslot, x.roff + cols.second, x.q, x.q, 1);
                 } else if (tr) region(x.rslot, x.roff, x.ldr, t.k, x.q);
                 else region(x.rslot, x.roff, x.ldr, x.q, t.k);
                 rank(x.qslot, x.qrank);

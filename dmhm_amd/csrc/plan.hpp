@@ -23,6 +23,7 @@
 #include <string>
 #include <vector>
 #include "geometry.hpp"
+#include "hostdev.hpp"
 
 namespace dmhm {
 
@@ -32,9 +33,9 @@ namespace dmhm {
 enum Slot : uint8_t { SLOT_A = 0, SLOT_B = 1, SLOT_C = 2, SLOT_WS = 3, SLOT_X = 4, SLOT_Y = 5,
                       SLOT_WIDTH = 6, SLOT_FLAG = 7, NUM_SLOTS = 8 };
 
-// CF_GATHER_R: the right operand is a panel of scattered columns; column j of
-// the tile starts at element gtab[Tile::gather + j] + roff of the slot
-// (Phase::gtab; ldr unused, not transposed).
+// CF_GATHER_R: the right operand is a stack of factors side by side, read where
+// they are stored (not transposed, ldr unused); gather_column gives the element
+// of the slot, less roff, where a column of the tile starts.
 enum ContribFlags : uint8_t { CF_TRANS_L = 1, CF_TRANS_R = 2, CF_RUNTIME_ALPHA = 4, CF_RUNTIME_BETA = 8,
                               CF_GATHER_R = 16 };
 enum TileFlags : uint8_t { TF_ACCUMULATE = 1, TF_RUNTIME_BETA = 2 };
@@ -57,8 +58,19 @@ struct Tile {
     int32_t moff, koff;
     int32_t cb, ce;         // contribution range
     uint8_t slot, mslot, kslot, flags;
-    int32_t gather = -1;    // first entry of the tile's columns in Phase::gtab, or -1
+    int32_t gather = -1;    // its stack's entry in Plan::gtab, or -1 ...
+    int32_t gcols = 0;      // ... and the columns of each of the stack's factors
 };
+// Start of column j of a tile whose right operands are a stack: the tile's
+// columns begin at column koff of the stack, and entry `gather` of the table
+// holds the factors' leading dimension, the next ones the factors' offsets.
+// (One entry per column made the tables of a 3D 32^3 rank-32 product 2.8 GB,
+// more than all its other tables, and its planning 7.9 s instead of 5.2.)
+DMHM_HD int64_t gather_column(const Tile& t, const int64_t* gtab, int j)
+{
+    const uint32_t col = (uint32_t)(t.koff + j), f = col / (uint32_t)t.gcols;
+    return gtab[t.gather + 1 + f] + (int64_t)(col - f * t.gcols) * gtab[t.gather];
+}
 
 struct QrTask {              // Householder QR of an m x k panel, Q in place
     int64_t off;            // panel offset (slot)
@@ -152,7 +164,7 @@ struct Phase {
     std::vector<MvProjItem> mvProj;
     std::vector<MvAtom> mvAtoms;
     std::vector<MvContrib> mvContribs;
-    std::vector<int64_t> gtab;            // PH_TILE: column offsets of gathered right operands
+    const std::vector<int64_t>* gtab = nullptr;   // PH_TILE that reads stacks: the plan's table
     // PH_TILE of a merged plan built without copying: per member, the source
     // phase (host, uploaded with its plan) and the member's shifts; the
     // device table of TileSeg is built at upload.
@@ -172,7 +184,8 @@ struct Phase {
     int qrRegK = 0;         // widest task of classes 0..3
     int svdK = 0;           // largest SVD factor of the phase (set by upload)
     // device copies (filled by upload)
-    void* dTiles = nullptr; void* dContribs = nullptr; void* dTasks = nullptr; void* dGather = nullptr;
+    void* dTiles = nullptr; void* dContribs = nullptr; void* dTasks = nullptr;
+    const void* dGather = nullptr;      // the plan's
     int maxKTile = 0;       // widest tile (selects the kernel variant)
     int maxMTile = 0;       // tallest tile
     int role = 0;           // 0 accumulation, 1 projection (profiling identity)
@@ -189,6 +202,8 @@ struct Phase {
 
 struct Plan {
     std::vector<Phase> phases;
+    std::vector<int64_t> gtab;      // stacks of right operands (gather_column)
+    void* dGather = nullptr;        // on the device (filled by upload)
     int64_t wsElems = 0;    // workspace elements (of the run-time precision)
     double flops = 0;       // algorithmic flops (GEMM shapes)
     int64_t contribCount = 0, tileCount = 0;
@@ -218,7 +233,7 @@ public:
     explicit PhaseBuilder(Phase& ph) : ph_(ph) {}
     int addTile(const Tile& t) { ph_.tiles.push_back(t); return (int)ph_.tiles.size() - 1; }
     void add(int tile, const Contrib& c) { pending_.push_back({tile, c}); }
-    void setGather(int tile, int at) { ph_.tiles[tile].gather = at; }
+    void setGather(int tile, int at, int cols) { ph_.tiles[tile].gather = at; ph_.tiles[tile].gcols = cols; }
     void finalize();
 private:
     Phase& ph_;
@@ -229,7 +244,8 @@ struct Operand {            // a panel or matrix block region
     uint8_t slot;
     int64_t off;
     int32_t ld;
-    int32_t gather = -1;    // scattered columns: first entry in the phase's gtab (off: row offset)
+    int32_t gather = -1;    // a stack of factors: its entry in the plan's gtab (off: row offset)
+    int32_t gcols = 0;      // and the columns of each
 };
 
 // Terms of C = A B for three H-matrices of one geometry, from the reference's
