@@ -195,15 +195,23 @@ struct MvAcc {
 #pragma unroll
         for (int u = 0; u < 16; ++u) f.l[u] = L[(TAIL ? min(u, q - 1) : u) * ld];
     }
+    // A record's products are summed by themselves: a wave's sum over all its
+    // records is hundreds of terms long, and as one chain it was off by 4.0e-7
+    // (256^2, FP32, one vector, relative to the result).
     template <bool TAIL>
     __device__ __forceinline__ void use(const Frag& f)
     {
+        T sum[K];
 #pragma unroll
-        for (int u = 0; u < 16; ++u) {
+        for (int kk = 0; kk < K; ++kk) sum[kk] = f.l[0] * bcast(f.r[kk >> 2], 16 * (kk & 3));
+#pragma unroll
+        for (int u = 1; u < 16; ++u) {
             if (TAIL && u >= f.q) continue;     // uniform
 #pragma unroll
-            for (int kk = 0; kk < K; ++kk) acc[kk] += f.l[u] * bcast(f.r[kk >> 2], 16 * (kk & 3) + u);
+            for (int kk = 0; kk < K; ++kk) sum[kk] += f.l[u] * bcast(f.r[kk >> 2], 16 * (kk & 3) + u);
         }
+#pragma unroll
+        for (int kk = 0; kk < K; ++kk) acc[kk] += sum[kk];
     }
     template <bool TAIL>
     __device__ __forceinline__ void run(uint64_t left)
